@@ -192,8 +192,7 @@ struct mhmhip_ctx {
   int32_t *d_node_gauge = nullptr;  // [n_cells] first gauge at the node, -1: none
   uint8_t *d_lag = nullptr;         // [n_cells] ring lag of each node (its tile slot's lag)
   int32_t *d_slot_out = nullptr;    // [n_slots] LDS output rows of the tiled kernel
-  // L1 output sums (mhmhip_output_accumulate): rows in the reference's
-  // output order, (kind, horizon) each
+  // L1 output sums (mhmhip_output_accumulate)
   double *d_out = nullptr;
   int64_t out_rows_cap = 0;
   OutAcc out_cfg{};
@@ -228,6 +227,7 @@ struct mhmhip_ctx {
   struct GraphKey {
     int32_t nsteps = -1, mode = -1, S = -1, block = -1, wg = -1, prof = -1, B = -1, out_n = -1,
             rep = -1;
+    uint64_t out_mask = 0;
     const void *ring = nullptr, *gauge = nullptr, *steps = nullptr, *inflow = nullptr,
                *qacc = nullptr, *out = nullptr, *cring = nullptr;
     int64_t ring_len = 0;
@@ -235,7 +235,7 @@ struct mhmhip_ctx {
       return nsteps == o.nsteps && mode == o.mode && S == o.S && block == o.block && wg == o.wg &&
              prof == o.prof && B == o.B && ring == o.ring && gauge == o.gauge && steps == o.steps &&
              inflow == o.inflow && qacc == o.qacc && ring_len == o.ring_len && out == o.out &&
-             out_n == o.out_n && rep == o.rep && cring == o.cring;
+             out_n == o.out_n && out_mask == o.out_mask && rep == o.rep && cring == o.cring;
     }
   };
   GraphKey gkey;
@@ -1163,7 +1163,7 @@ int make_step(mhmhip_ctx *x, const mhmhip_step &s, StepDev &d) {
   d.revap = 1.0 / d.evap;
   d.init_sm = (s.tt == 1) && !s.read_states;  // mo_mhm.f90:448
   d.doy = s.doy;
-  d.meteo_same = 0;
+  d.change = SC_METEO | SC_DAY | SC_MONTH | (d.init_sm ? SC_INIT : 0);
   d.wrow = m * 24 + s.hour;
   return MHMHIP_OK;
 }
@@ -2198,21 +2198,12 @@ extern "C" int mhmhip_output_accumulate(mhmhip_ctx *x, const int32_t *flags) {
   if (flags[17])
     return x->fail(MHMHIP_EINVAL, "output_accumulate: outputFlxState(18) (neutrons) is not on "
                                   "this path");
-  // the reference's output order (mHM_updateDataset, mo_write_fluxes_states.f90:318-436)
-  static const int order[] = {1, 2, 3, 4, 5, 6, 7, 8, 18, 9, 10, 11, 12, 13, 14, 15, 16, 17,
-                              19, 20, 21};
   OutAcc o{};
-  int n = 0;
-  for (int k : order) {
-    if (!flags[k - 1]) continue;
-    const int nh = out_per_horizon(k) ? x->nh : 1;
-    for (int h = 0; h < nh; ++h) {
-      if (n >= kOutRowsMax) return x->fail(MHMHIP_EINVAL, "output_accumulate: too many rows");
-      o.kind[n] = (int8_t)k;
-      o.hor[n] = (int8_t)h;
-      ++n;
-    }
-  }
+  for (int k = 1; k <= 21; ++k)
+    if (flags[k - 1])
+      for (int h = 0; h < (out_per_horizon(k) ? x->nh : 1); ++h)
+        o.mask |= (uint64_t)1 << out_bit(k, h, x->nh);
+  const int n = o.n = __builtin_popcountll(o.mask);
   if (n == 0) {
     x->out_on = false;
     return MHMHIP_OK;
@@ -2228,7 +2219,6 @@ extern "C" int mhmhip_output_accumulate(mhmhip_ctx *x, const int32_t *flags) {
               "output_accumulate");
   }
   o.sum = x->d_out;
-  o.n = n;
   x->out_cfg = o;
   x->out_on = true;
   x->out_count = 0;
@@ -2241,9 +2231,10 @@ extern "C" int mhmhip_get_output_sum(mhmhip_ctx *x, int32_t k, int32_t horizon, 
   if (!x->out_cfg.sum) return x->fail(MHMHIP_ESTATE, "get_output_sum: accumulation never started");
   if (set < 0 || set >= x->n_sets) return x->fail(MHMHIP_EINVAL, "get_output_sum: bad set");
   const int h = out_per_horizon(k) ? horizon - 1 : 0;
+  const int bit = h >= 0 && h < x->nh ? out_bit(k, h, x->nh) : -1;
   int row = -1;
-  for (int r = 0; r < x->out_cfg.n; ++r)
-    if (x->out_cfg.kind[r] == k && x->out_cfg.hor[r] == h) row = r;
+  if (bit >= 0 && (x->out_cfg.mask >> bit & 1))
+    row = __builtin_popcountll(x->out_cfg.mask & (((uint64_t)1 << bit) - 1));
   if (row < 0 || (out_per_horizon(k) && (horizon < 1 || horizon > x->nh)))
     return x->fail(MHMHIP_EINVAL, "get_output_sum: output " + std::to_string(k) +
                                       " (horizon " + std::to_string(horizon) +
@@ -2532,15 +2523,18 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
   if (route && !steps[0].read_states) CHECK_RC(refresh_reg_rout(x));
   std::vector<StepDev> hs(nsteps);
   for (int32_t k = 0; k < nsteps; ++k) CHECK_RC(make_step(x, steps[k], hs[k]));
-  // a step whose forcing column, day and day/night factors (and, with meteo
-  // weights, month and hour) equal the step before's has the same
-  // disaggregated meteo values (the fused kernel keeps them; its first step
-  // of a launch computes them regardless)
+  // what each step changes: a step whose forcing column, day and day/night
+  // factors (and, with meteo weights, month and hour) equal the step before's
+  // has the same disaggregated meteo values (the fused kernel keeps them; its
+  // first step of a launch looks everything up regardless)
   for (int32_t k = 1; k < nsteps; ++k) {
-    const StepDev &p = hs[k - 1], &c = hs[k];
-    hs[k].meteo_same = p.day == c.day && p.doy == c.doy && p.month0 == c.month0 &&
-                       p.f_pet == c.f_pet && p.f_prec == c.f_prec && p.f_temp == c.f_temp &&
-                       (!x->W || p.wrow == c.wrow);
+    const StepDev &p = hs[k - 1];
+    StepDev &c = hs[k];
+    const bool day = p.day != c.day || p.doy != c.doy, month = p.month0 != c.month0;
+    const bool meteo = day || month || p.f_pet != c.f_pet || p.f_prec != c.f_prec ||
+                       p.f_temp != c.f_temp || (x->W && p.wrow != c.wrow);
+    c.change = (meteo ? SC_METEO : 0) | (day ? SC_DAY : 0) | (month ? SC_MONTH : 0) |
+               (c.init_sm ? SC_INIT : 0);
   }
   CHECK_RC(forcing_wait(x, hs.data(), nsteps));
   x->s_dirty = x->x_dirty = true;
@@ -2734,6 +2728,7 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
     key.qacc = r.qacc;
     key.out = a.out.sum;
     key.out_n = a.out.sum ? a.out.n : 0;
+    key.out_mask = a.out.sum ? a.out.mask : 0;
     key.rep = rep;
     key.cring = route && x->coarse ? x->d_cring : nullptr;
     if (!x->graph_exec || !(key == x->gkey)) {

@@ -79,23 +79,24 @@ struct DV {
 // -(ln2_hi + ln2_lo), so just above x = 1 (e = 1, F = 1/2) the two terms
 // cancel with no rounding and log x is log1p(u) of u = 2m - 1 = x - 1.
 // Within 1.25 ulp.  Every operation is an IEEE +, -, *, fma, rint or an exact
-// frexp, and the table holds the same numbers on host and device (LDS,
-// filled by mathtab_fill), so the two builds agree bit for bit.  Each step
+// frexp, and the table holds the same numbers on host and device, so the two
+// builds agree bit for bit.  Each step
 // runs over all N values before the next one, which gives the scheduler N
 // independent dependency chains to interleave.  Rows are 4 doubles (32 B):
 // a row's address is one shift of j.
 #if defined(__HIP_DEVICE_COMPILE__)
-__shared__ __attribute__((aligned(16))) double s_mathtab[kLogTabN * 4 + kExpTabN * 2];
+__shared__ __attribute__((aligned(16))) double s_mathtab[kPowLogN * 2 + kExpTabN * 2];
 #endif
 
-// Every workgroup of a kernel that evaluates a log or an exp calls this
+// Every workgroup of a kernel that evaluates a power or an exp calls this
 // before the first one (all threads, before any of them returns).  The
-// tables are copied in 16-byte pieces, a thread's first three loads issued
-// before its stores, so that the copy waits for memory once.
+// tables (base-2 logarithm rows and 2^(j/256), 6 KB) are copied in 16-byte
+// pieces, a thread's first three loads issued before its stores, so that the
+// copy waits for memory once.
 __device__ inline void mathtab_fill() {
 #if defined(__HIP_DEVICE_COMPILE__)
-  constexpr int n = (kLogTabN * 4 + kExpTabN * 2) / 2;
-  const double2 *src = reinterpret_cast<const double2 *>(kMathTab);
+  constexpr int n = (kPowLogN * 2 + kExpTabN * 2) / 2;
+  const double2 *src = reinterpret_cast<const double2 *>(kPowTab);
   double2 *dst = reinterpret_cast<double2 *>(s_mathtab);
   const int i0 = threadIdx.x, bs = blockDim.x;
   // pieces past the table copy its last piece again (no branch between the
@@ -110,21 +111,19 @@ __device__ inline void mathtab_fill() {
 #endif
 }
 
-__host__ __device__ inline const double *logtab() {
+// The natural logarithm's rows stay in memory on the device too: only the
+// daily PET of Priestley-Taylor and Penman-Monteith takes one.
+__host__ __device__ inline const double *logtab() { return kMathTab; }
+
+__host__ __device__ inline const double *powtab() {
 #if defined(__HIP_DEVICE_COMPILE__)
   return s_mathtab;
 #else
-  return kMathTab;
+  return kPowTab;
 #endif
 }
 
-__host__ __device__ inline const double *exptab() {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return s_mathtab + kExpTabOff;
-#else
-  return kMathTab + kExpTabOff;
-#endif
-}
+__host__ __device__ inline const double *exptab() { return powtab() + kPowExpOff; }
 
 template <int N>
 __host__ __device__ inline DV<N> log_pos_v(const DV<N> &x) {
@@ -196,16 +195,80 @@ __host__ __device__ inline DV<N> exp_fin_v(const DV<N> &zin) {
   return out;
 }
 
-// x**y for x > 0 as exp(y log x), N pairs at once: within (2 + 3 |y log x|)
-// ulp of the exact power (log's error and the rounding of y log x, amplified
-// by exp); for the chain's arguments |y log x| stays of order 10, a few
-// 1e-15 relative at most.
+// x**y for x > 0 as 2^(y log2 x), N pairs at once, table-driven (Tang's
+// method for both halves, in base 2): x = m 2^e (frexp), the row of m's
+// interval gives R and L = -log2 R (one double: R is chosen for it),
+// u = m R - 1 (one fma; |u| <= 1/128) and
+//   log2 x = e + L + u (c0 + ... + c5 u^5);
+// with y256 = 256 y, z = 256 y log2 x as y256 e + (y256 L + y256 (u ...)), two
+// fma, n = RN(z), r = z - n (exact, |r| <= 1/2):
+//   x**y = 2^(n >> 8) 2^((n & 255)/256) (1 + r (d0 + ... + d3 r^3)),
+// the table's 2^(j/256) as hi + lo.  Working in units of 1/256 of a binary
+// logarithm leaves no multiplication by ln 2 or 256/ln 2 and makes the
+// reduction exact: 28 vector instructions and two 16-byte table reads per
+// power on gfx950, where exp(y log x) took 37 and three.  The rows on either
+// side of x = 1 hold R = 2 and R = 1 with exact logarithms, so 1**y is 1.
+// Within (2 + 3 |y log x|) ulp of the exact power (the rounding of z,
+// amplified by the exponential); over the chain's arguments 1.3 to 1.5 ulp
+// rms against mpmath, where exp(y log x) with two such roundings had 1.7 to 1.9.
+// Phases run over all N values, the loads of a phase's table rows together,
+// so that N independent chains interleave and each phase waits for LDS once.
+template <int N>
+__host__ __device__ __forceinline__ DV<N> pow_v(const DV<N> &y256, const DV<N> &x) {
+  DV<N> u, hi, lo, z, p, out;
+  int e[N];
+  const char *tab = reinterpret_cast<const char *>(powtab());
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    u.v[i] = frexp(x.v[i], &e[i]);  // m in [1/2, 1)
+    uint64_t bits;
+    __builtin_memcpy(&bits, &u.v[i], 8);
+    const double *t =
+        reinterpret_cast<const double *>(tab + (((uint32_t)(bits >> 32) >> 9) & 0x7F0u));
+    lo.v[i] = t[0];
+    hi.v[i] = t[1];
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) u.v[i] = fma(u.v[i], lo.v[i], -1.0);
+#pragma unroll
+  for (int i = 0; i < N; ++i) p.v[i] = kPowC[5];
+#pragma unroll
+  for (int k = 4; k >= 0; --k)
+#pragma unroll
+    for (int i = 0; i < N; ++i) p.v[i] = fma_k(p.v[i], u.v[i], kPowC[k]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const double y = y256.v[i];
+    z.v[i] = fma(y, (double)e[i], fma(y, hi.v[i], y * (p.v[i] * u.v[i])));
+  }
+  const char *etab = reinterpret_cast<const char *>(exptab());
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const double n = rint(z.v[i]);
+    u.v[i] = z.v[i] - n;  // r
+    const int ni = (int)n;
+    e[i] = ni >> 8;  // floor(n / 256)
+    const double *t = reinterpret_cast<const double *>(etab + (((uint32_t)ni << 4) & 0xFF0u));
+    hi.v[i] = t[0];
+    lo.v[i] = t[1];
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) p.v[i] = kPowD[3];
+#pragma unroll
+  for (int k = 2; k >= 0; --k)
+#pragma unroll
+    for (int i = 0; i < N; ++i) p.v[i] = fma_k(p.v[i], u.v[i], kPowD[k]);
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    out.v[i] = ldexp(hi.v[i] + fma(hi.v[i] * u.v[i], p.v[i], lo.v[i]), e[i]);
+  return out;
+}
+
 template <int N>
 __host__ __device__ MHMHIP_OUTLINE DV<N> exp_ylogx_v(DV<N> y, DV<N> x) {
-  DV<N> l = log_pos_v<N>(x);
 #pragma unroll
-  for (int i = 0; i < N; ++i) l.v[i] = y.v[i] * l.v[i];
-  return exp_fin_v<N>(l);
+  for (int i = 0; i < N; ++i) y.v[i] = y.v[i] * 256.0;  // exact
+  return pow_v<N>(y, x);
 }
 
 __host__ __device__ inline double log_pos(double x) { return log_pos_v<1>(DV<1>{{x}}).v[0]; }
@@ -304,11 +367,16 @@ __device__ __forceinline__ double vmax(double a, double b) {
   asm("v_max_f64 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
   return d;
 }
-// max(a, 0) with the zero an inline constant, and max(a, k) for a constant k
-// passed in a scalar register pair
+// max(a, 0) and min(a, 1) with the bound an inline constant, and max(a, k) for
+// a constant k passed in a scalar register pair
 __device__ __forceinline__ double vmax0(double a) {
   double d;
   asm("v_max_f64 %0, %1, 0" : "=v"(d) : "v"(a));
+  return d;
+}
+__device__ __forceinline__ double vmin1(double a) {
+  double d;
+  asm("v_min_f64 %0, %1, 1.0" : "=v"(d) : "v"(a));
   return d;
 }
 __device__ __forceinline__ double vmax_k(double a, double k) {
@@ -510,6 +578,180 @@ __device__ __forceinline__ void runoff_sat_zone(double k2, double &sat, double &
 __device__ __forceinline__ double total_runoff(double fS, double fast, double slow, double base,
                                                double direct) {
   return ((base + slow + fast) * (1.0 - fS)) + (direct * fS);
+}
+
+// ---------------------------------------------------------------------------
+// The same step for an ordinary cell, without branches and selects.  The
+// cell kernels are bound by the number of vector instructions they issue
+// (every type at one wave instruction per four cycles), and about half of the
+// functions above is compares, 64-bit selects (two instructions each) and
+// copies at the ends of divergent branches.  For parameters and states in
+// their physical ranges (ordinary_params, ordinary_states: non-negative
+// rates, field capacity above wilting point, a store within its bounds, ...)
+// every branch is a minimum, a maximum or has a known outcome.  A cell outside
+// these ranges takes the functions above; which of the two a cell takes
+// depends on that cell alone.  The values are those of the functions above:
+// equal bits, except that where two branches meet (a store filled or emptied
+// exactly, the degree-day factor reaching its maximum, field capacity) the
+// result may be the other branch's, one rounding away.
+
+constexpr double kBig = 1e15;   // parameters beyond this are not ordinary
+constexpr double kTiny = 1e-15;
+
+// x**(2/3) of a canopy ratio (pow23 without its exponent handling): the seed
+// in single precision straight from x, in range for x >= 2^-32, where its
+// error stays below 2^-18 and the Halley step's below 2^-56.  Smaller
+// ratios go through pow23; 0, negative and NaN ratios give NaN (the caller's
+// maximum with 0 then gives 0, as for the reference's power of them).
+__device__ __forceinline__ double pow23_ratio(double x) {
+  const float f = (float)x;
+  const double y =
+      (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf(f) * (-1.0f / 3.0f));
+  const double r = fma(-x, (y * y) * y, 1.0);
+  double v = x * fma(y * r, fma(r, 2.0 / 9.0, 1.0 / 3.0), y);
+  // the high words of 2^-1042 .. 2^-32
+  if ((uint32_t)__double2hiint(x) - 1u < 0x3DF00000u - 1u) v = pow23(x);
+  return v;
+}
+
+// Canopy (canopy_fill, canopy_evap).  rmax: 0 when interc_max <= eps, which
+// makes the ratio 0 and the evaporation 0, else RN(1/interc_max).
+__device__ __forceinline__ void canopy_ordinary(double pet, double interc_max, double rmax,
+                                                double precip, double &interc,
+                                                double &throughfall, double &evap_canopy) {
+  const double aux = interc + precip;
+  throughfall = vmax0(aux - interc_max);
+  const double full = vmin(aux, interc_max);
+  const double ratio = div_rcp(full, interc_max, rmax);
+  evap_canopy = vmin(vmax0(pet * pow23_ratio(ratio)), full);
+  interc = full - evap_canopy;
+}
+
+// snow_accum_melt, first what the meteo values alone give: the degree-day
+// factor (its rise ends where it meets its maximum), the melt a large enough
+// pack would give (a cold step's product is negative and melts nothing) and
+// whether precipitation is snow (1) or rain (0).
+struct SnowMeteo {
+  double ddf, melt, cold;
+};
+__device__ __forceinline__ SnowMeteo snow_meteo(double incr, double dmax, double dnp, double tth,
+                                                double prec, double temp) {
+  SnowMeteo m;
+  m.ddf = vmin(dnp + incr * prec, dmax);
+  m.melt = vmax0(m.ddf * (temp - tth));
+  m.cold = temp > tth ? 0.0 : 1.0;
+  return m;
+}
+
+__device__ __forceinline__ void snow_ordinary(double melt_meteo, double cold, double thr,
+                                              double &pack, double &melt, double &prec_effect,
+                                              double &rain, double &snow) {
+  snow = thr * cold;
+  rain = thr - snow;
+  melt = vmin(melt_meteo, pack);
+  pack = (pack + snow) - melt;
+  prec_effect = melt + rain;
+}
+
+// The sealed storage of soil_moisture (pe: pet / evap); sealed: fS > 0.
+// Without sealed area the storage stays and the fluxes are of no weight (the
+// caller reports them as 0).
+__device__ __forceinline__ void sealed_ordinary(bool sealed, double thrS, double rthrS, double pe,
+                                                double ecan, double peff, double &runoff_sealed,
+                                                double &storage_sealed, double &aet_sealed) {
+  const double tmp = storage_sealed + peff;
+  runoff_sealed = vmax0(tmp - thrS);
+  const double st = vmin(tmp, thrS);
+  aet_sealed = vmin(vmax0((pe - ecan) * div_rcp(st, thrS, rthrS)), st);
+  storage_sealed = sealed ? st - aet_sealed : storage_sealed;
+}
+
+// soil_moisture's infiltration into one horizon: the horizon takes pin
+// (1 - frac), at most what fills it, and passes on the rest.
+__device__ __forceinline__ double infiltrate_ordinary(double pin, double frac, double sat,
+                                                      double &sm) {
+  const double tmp = pin * (1.0 - frac);
+  const double infil = pin - vmin(tmp, sat - sm);
+  sm = vmin(sm + tmp, sat);
+  return infil;
+}
+
+// Feddes: (sm - wp) slope between wilting point and field capacity, slope =
+// RN(fr / (fc - wp)): two roundings, as fr (sm - wp) / (fc - wp) has.
+// Jarvis: fr min(theta / c1, 1), theta = (sm - wp) / (sat - wp) within 0 .. 1
+// (slope: RN(1 / (sat - wp)), fw = sat - wp, rc1 = RN(1 / c1)).
+template <bool JV>
+__device__ __forceinline__ double stress_ordinary(double sm, double wp, double fr, double slope,
+                                                  double fw, double c1, double rc1) {
+  if constexpr (JV) {
+    const double th = vmin1(vmax0(div_rcp(sm - wp, fw, slope)));
+    return fr * vmin1(div_rcp(th, c1, rc1));
+  } else {
+    return vmin(vmax0((sm - wp) * slope), fr);
+  }
+}
+
+// soil_moisture's evapotranspiration of one horizon: demand a = pet - ecan -
+// what the horizons above gave; the store keeps at least eps.
+__device__ __forceinline__ double evaporate_ordinary(double demand, double f, double &sm) {
+  const double a = vmax0(demand * f);
+  const double aet = vmin(a, sm - kEps);
+  sm = vmax_k(sm - a, kEps);
+  return aet;
+}
+
+// runoff_fast and runoff_slow_perc (alpha1 = 1 + alpha in the caller's power)
+__device__ __forceinline__ void runoff_fast_ordinary(double k0, double pin, double thr,
+                                                     double &unsat, double &fast) {
+  unsat = unsat + pin;
+  fast = vmax0(vmin(unsat - kEps, k0 * (unsat - thr)));
+  unsat = unsat - fast;
+}
+
+__device__ __forceinline__ void runoff_slow_perc_ordinary(double k1, double kp, double karst,
+                                                          double pw, double &sat, double &unsat,
+                                                          double &slow, double &perc) {
+  slow = vmax0(vmin(unsat - kEps, k1 * pw));
+  unsat = unsat - slow;
+  perc = kp * unsat;
+  const double p = vmin(perc, unsat);
+  sat = sat + p * karst;
+  unsat = unsat - p;
+}
+
+// Whether a cell's parameters are in the ranges the functions above assume
+// (a NaN is not).
+template <int NH, bool JV>
+__device__ __forceinline__ bool ordinary_params(double fS, double thrS, double incr, double dmax,
+                                                double dnp, double k0, double k1, double k2,
+                                                double kp, double karst, double alpha, double thrU,
+                                                const double *sat, const double *fr,
+                                                const double *fc, const double *wp,
+                                                const double *bexp, double c1) {
+  // no short circuits: one straight line of compares
+  bool ok = (fS >= 0.0) & (!(fS > 0.0) | (thrS > kTiny)) & (thrS < kBig) & (incr >= 0.0) &
+            (incr < kBig) & (dnp >= 0.0) & (dnp < kBig) & (dmax >= 0.0) & (dmax < kBig) &
+            (k0 >= 0.0) & (k0 < kBig) & (k1 >= 0.0) & (k1 < kBig) & (k2 >= 0.0) & (k2 <= 1.0) &
+            (kp >= 0.0) & (kp < kBig) & (karst >= 0.0) & (karst < kBig) & (alpha > -1.0) &
+            (alpha < 64.0) & (thrU > kTiny) & (thrU < kBig);
+#pragma unroll
+  for (int h = 0; h < NH; ++h) {
+    ok = ok & (sat[h] >= 1.0) & (sat[h] < kBig) & (bexp[h] >= 1.0) & (bexp[h] < 64.0) &
+         (fr[h] >= 0.0) & (fr[h] < kBig) & (fabs(wp[h]) < kBig) & (fc[h] - wp[h] > kTiny) &
+         (fc[h] > 4.0 * kTiny) & (fc[h] <= sat[h]);
+    if constexpr (JV) ok = ok & (sat[h] - wp[h] > kTiny);
+  }
+  if constexpr (JV) ok = ok & (c1 > kTiny) & (c1 < kBig);
+  return ok;
+}
+
+template <int NH>
+__device__ __forceinline__ bool ordinary_states(double pack, double unsat, double satS,
+                                                const double *sm, const double *sat) {
+  bool ok = (pack >= 0.0) & (unsat >= 0.0) & (unsat < kBig) & (satS >= 0.0);
+#pragma unroll
+  for (int h = 0; h < NH; ++h) ok = ok & (sm[h] >= kEps) & (sm[h] <= sat[h]);
+  return ok;
 }
 
 // src/mHM/mo_pet.f90:73-116 with extraterr_rad_approx (314-355).  The

@@ -12,6 +12,19 @@ ln 2 that log_pos_v multiplies by the exponent, so that for x just above 1
 Exponential, 2^(j/256) for j = 0..255 as hi = RN(2^(j/256)) and
 lo = RN(2^(j/256) - hi).
 
+Power (pow_v in chain.h): base-2 logarithm rows {R, L} for j = 0..127, one per
+interval [(128 + j)/256, (129 + j)/256) of the frexp mantissa m: R near the
+reciprocal of the interval's middle, u = m R - 1 and log2(m) = L +
+log2(1 + u).  R is searched next to that reciprocal so that L = -log2(R) lies
+within 2^-10 of half a unit of a double's last place (the accurate tables of
+Gal, in "Computing elementary functions: a new approach for achieving high
+accuracy and good performance", LNCS 235 (1986) 1-16): one double holds it.
+The first row has R = 2 and the last R = 1, both with exact logarithms, so
+that log2 x is 0 at x = 1.  Then 2^(j/256) as above, and the coefficients of
+log2(1 + u) = u (c0 + ... + c5 u^5) on [-1/256, 1/128] and of
+2^(r/256) = 1 + r (d0 + ... + d3 r^3) on [-1/2, 1/2], interpolated at Chebyshev
+nodes (relative errors below 2^-52 and 2^-58).
+
 Values from mpmath at 256 bits.
 Run: python mhm_amd/csrc/gen_mathtab.py > mhm_amd/csrc/mathtab.h
 """
@@ -42,6 +55,33 @@ def exp_row(j):
     return hi, float(T - mp.mpf(hi))
 
 
+def pow_row(j):
+    if j == 0:
+        return 2.0, -1.0
+    if j == 127:
+        return 1.0, 0.0
+    R = float(mp.mpf(512) / (2 * (128 + j) + 1))
+    while True:
+        L = -mp.log(mp.mpf(R), 2)
+        if abs(L - mp.mpf(float(L))) < math.ulp(float(L)) * mp.mpf(2) ** -11:
+            return R, float(L)
+        R = math.nextafter(R, 2.0)
+
+
+def chebyshev_fit(f, a, b, n):
+    """Coefficients (constant first) of the degree n - 1 polynomial through f
+    at the n Chebyshev nodes of [a, b]."""
+    a, b = mp.mpf(a), mp.mpf(b)
+    x = [(a + b) / 2 + (b - a) / 2 * mp.cos(mp.pi * (2 * k + 1) / (2 * n)) for k in range(n)]
+    A = mp.matrix(n, n)
+    y = mp.matrix(n, 1)
+    for i in range(n):
+        y[i] = f(x[i])
+        for k in range(n):
+            A[i, k] = x[i] ** k
+    return [float(c) for c in mp.lu_solve(A, y)]
+
+
 def main():
     assert LN2_HI + LN2_LO == float(mp.log(2))
     print("// mathtab.h -- generated by gen_mathtab.py; do not edit.")
@@ -62,6 +102,22 @@ def main():
         hi, lo = exp_row(j)
         print("    %s, %s," % (hi.hex(), lo.hex()))
     print("};")
+    print("constexpr int kPowLogN = 128;")
+    print("constexpr int kPowExpOff = kPowLogN * 2;  // the 2^(j/256) rows' first element")
+    print("alignas(16) constexpr double kPowTab[kPowLogN * 2 + kExpTabN * 2] = {")
+    print("    // {R, L}: log2(m) = L + log2(m R), by interval of m")
+    for j in range(128):
+        print("    %s, %s," % tuple(v.hex() for v in pow_row(j)))
+    print("    // {hi, lo} of 2^(j/%d), j = 0..%d" % (EXP_N, EXP_N - 1))
+    for j in range(EXP_N):
+        hi, lo = exp_row(j)
+        print("    %s, %s," % (hi.hex(), lo.hex()))
+    print("};")
+    c = chebyshev_fit(lambda u: mp.log(1 + u, 2) / u, mp.mpf(-1) / 256, mp.mpf(1) / 128, 6)
+    d = chebyshev_fit(lambda r: (mp.power(2, r / 256) - 1) / r, mp.mpf(-1) / 2, mp.mpf(1) / 2, 4)
+    print("// log2(1 + u) / u and (2^(r/256) - 1) / r, constant term first")
+    print("constexpr double kPowC[6] = {%s};" % ", ".join(v.hex() for v in c))
+    print("constexpr double kPowD[4] = {%s};" % ", ".join(v.hex() for v in d))
     print("}  // namespace mhmhip")
 
 

@@ -58,6 +58,15 @@ __host__ __device__ constexpr int xr_infil(int nh) { return XR_NSCALAR; }
 __host__ __device__ constexpr int xr_aet(int nh) { return XR_NSCALAR + nh; }
 __host__ __device__ constexpr int xr_count(int nh) { return XR_NSCALAR + 2 * nh; }
 
+// What a step of a run changes against the step before (StepDev::change): the
+// time loop looks its per-lane values up again only then.
+enum StepChange {
+  SC_METEO = 1,  // forcing column, day or disaggregation factors
+  SC_DAY = 2,    // forcing column or day of year (the daily PET)
+  SC_MONTH = 4,  // month (interception capacity, pan coefficient)
+  SC_INIT = 8,   // the step resets the soil moisture (init_sm)
+};
+
 // Per-step scalars on the device (host-evaluated from the step clock).
 struct StepDev {
   double dr, tand, sind, cosd;  // extraterr_rad_approx day-of-year terms
@@ -70,7 +79,7 @@ struct StepDev {
   int32_t isday;                // 6 < hour <= 18
   int32_t init_sm;              // tt == 1 .and. .not. read_states
   int32_t doy;
-  int32_t meteo_same;           // same forcing column, day and factors as the step before
+  int32_t change;               // StepChange bits: what differs from the step before
   int32_t wrow;                 // month0 * 24 + hour: the row of the meteo weights
 };
 
@@ -82,16 +91,26 @@ struct MonthTables {
 };
 
 // Output aggregation of L1 states and fluxes (mHM_updateDataset,
-// src/mHM/mo_write_fluxes_states.f90:283-438): row r of the sums holds output
-// kind[r] (outputFlxState index 1..21) of horizon hor[r]; every step adds
-// each row's value to its sum (updateVariable, mo_nc_output.f90:140-148).
-constexpr int kOutRowsMax = 64;
+// src/mHM/mo_write_fluxes_states.f90:283-438): one sum per selected output
+// (outputFlxState index 1..21) and horizon; every step adds the output's value
+// to its sum (updateVariable, mo_nc_output.f90:140-148).  An output has a bit
+// (out_bit), in the order a step makes them: canopy and snow, soil and fast
+// interflow, the rest; the sums' rows are the selected bits in order.
 struct OutAcc {
   double *sum;               // [n][ld], null: off
-  int32_t n;
-  int8_t kind[kOutRowsMax];
-  int8_t hor[kOutRowsMax];
+  uint64_t mask;             // selected bits
+  int32_t n;                 // their number
 };
+__host__ __device__ constexpr int out_bits(int nh) { return 16 + 4 * nh; }
+// The bit of output k (horizon h, 0-based, for those per horizon); -1: none.
+__host__ __device__ constexpr int out_bit(int k, int h, int nh) {
+  return k == 1 ? 0 : k == 2 ? 1 : k == 9 ? 2 : k == 20 ? 3 : k == 21 ? 4
+       : k == 3 ? 5 + h : k == 4 ? 5 + nh + h : k == 5 ? 5 + 2 * nh : k == 6 ? 6 + 2 * nh
+       : k == 10 ? 7 + 2 * nh : k == 12 ? 8 + 2 * nh : k == 13 ? 9 + 2 * nh
+       : k == 17 ? 10 + 2 * nh + h : k == 19 ? 10 + 3 * nh + h
+       : k == 7 ? 10 + 4 * nh : k == 8 ? 11 + 4 * nh : k == 11 ? 12 + 4 * nh
+       : k == 14 ? 13 + 4 * nh : k == 15 ? 14 + 4 * nh : k == 16 ? 15 + 4 * nh : -1;
+}
 
 struct CellArgs {
   const double *P;

@@ -59,15 +59,63 @@ __device__ __forceinline__ void stn(double *row, uint32_t boff, double x) {
 #endif
 }
 
+// The kernel's arguments read through the constant address space: CellArgs is
+// the first argument of every cell kernel, so its copy is at the start of the
+// argument segment.  Members that are indexed at run time (OutAcc's) and
+// out-of-line functions read it there with scalar loads; a by-value copy of
+// them would live in scratch memory.
+typedef const __attribute__((address_space(4))) CellArgs ConstArgs;
+__device__ __forceinline__ ConstArgs *kernel_args() {
+  return (ConstArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+}
+// A pointer that is the same in every lane, as one the compiler knows to be
+__device__ __forceinline__ ConstArgs *uniform(ConstArgs *p) {
+  const uint64_t v = (uint64_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return (ConstArgs *)(((uint64_t)hi << 32) | lo);
+}
+// For a block that a time loop runs now and then: the arguments read there
+// instead of being held in scalar registers across the loop.
+__device__ __forceinline__ ConstArgs *rare(ConstArgs *p) {
+  asm volatile("" : "+s"(p));
+  return p;
+}
+// every argument but the output sums
+__device__ __forceinline__ CellArgs read_args(ConstArgs *p) {
+  CellArgs a;
+  a.P = p->P, a.S = p->S, a.X = p->X, a.F = p->F, a.ring = p->ring, a.area = p->area;
+  a.lag = p->lag, a.tst = p->tst, a.rtst = p->rtst, a.steps = p->steps;
+  a.n_cells = p->n_cells, a.sstride = p->sstride, a.ld = p->ld;
+  a.forcing_days = p->forcing_days, a.ring_len = p->ring_len, a.pet_case = p->pet_case;
+  a.jarvis = p->jarvis, a.hourly = p->hourly, a.ring_rep = p->ring_rep;
+  a.raw_total = p->raw_total, a.nT = p->nT, a.rnT = p->rnT, a.W = p->W;
+  return a;
+}
+
 template <int NH>
 struct CellRegs {
-  double fS, thrS, c1, k0s, k1s, k2s, kps, alpha, karst, thrU, dmaxs, dnps, incr, tth, ddthr;
+  double fS, thrS, c1, k0s, k1s, k2s, kps, alpha, karst, thrU, dmaxs, dnps, incr, tth;
   double sat[NH], fr[NH], fc[NH], wp[NH], bexp[NH];
   // correctly rounded reciprocals of the per-cell divisors (div_rcp)
-  double rthrS, rsat[NH], rfw[NH];
+  double rthrS, rsat[NH];
   double inter, pack, seal, unsat, satS;
   double sm[NH];
 };
+
+// Waits for every load of a cell's parameters and states.
+template <int NH>
+__device__ __forceinline__ void settle_all(CellRegs<NH> &c) {
+  settle(c.fS), settle(c.thrS), settle(c.c1), settle(c.k0s), settle(c.k1s), settle(c.k2s);
+  settle(c.kps), settle(c.alpha), settle(c.karst), settle(c.thrU), settle(c.dmaxs);
+  settle(c.dnps), settle(c.incr), settle(c.tth), settle(c.inter), settle(c.pack);
+  settle(c.seal), settle(c.unsat), settle(c.satS);
+#pragma unroll
+  for (int h = 0; h < NH; ++h) {
+    settle(c.sat[h]), settle(c.bexp[h]), settle(c.sm[h]);
+    settle(c.fr[h]), settle(c.fc[h]), settle(c.wp[h]);
+  }
+}
 
 template <int NH>
 struct FluxRegs {
@@ -101,14 +149,9 @@ __device__ __forceinline__ void load_params(const CellArgs &a, uint32_t bv, Cell
     c.wp[h] = P(pr_wp(NH) + h);
     c.bexp[h] = P(pr_exp(NH) + h);
   }
-  // snow_accum_melt's branch threshold (mo_snow_accum_melt.f90:127)
-  c.ddthr = (c.dmaxs - c.dnps) / c.incr;
   c.rthrS = 1.0 / c.thrS;
 #pragma unroll
-  for (int h = 0; h < NH; ++h) {
-    c.rsat[h] = 1.0 / c.sat[h];
-    c.rfw[h] = 1.0 / (c.fc[h] - c.wp[h]);
-  }
+  for (int h = 0; h < NH; ++h) c.rsat[h] = 1.0 / c.sat[h];
 }
 
 template <int NH>
@@ -137,9 +180,10 @@ __device__ __forceinline__ void store_states(const CellArgs &a, uint32_t bv0,
   for (int h = 0; h < NH; ++h) S(SR_NSCALAR + h, c.sm[h]);
 }
 
+// the step's meteo values and the fluxes of the canopy and the snow
 template <int NH>
-__device__ __forceinline__ void store_fluxes_pre(const CellArgs &a, uint32_t bv0,
-                                                 const FluxRegs<NH> &x) {
+__device__ __forceinline__ void store_fluxes_canopy(const CellArgs &a, uint32_t bv0,
+                                                    const FluxRegs<NH> &x) {
   const uint32_t bv = opaque(bv0);
   auto X = [&](int r, double y) { stn(a.X + (int64_t)r * a.ld, bv, y); };
   X(XR_PET, x.pet);
@@ -152,6 +196,14 @@ __device__ __forceinline__ void store_fluxes_pre(const CellArgs &a, uint32_t bv0
   X(XR_PEFF, x.peff);
   X(XR_RAIN, x.rain);
   X(XR_SNOW, x.snow);
+}
+
+// those of the sealed area, the soil and the fast interflow
+template <int NH>
+__device__ __forceinline__ void store_fluxes_soil(const CellArgs &a, uint32_t bv0,
+                                                  const FluxRegs<NH> &x) {
+  const uint32_t bv = opaque(bv0);
+  auto X = [&](int r, double y) { stn(a.X + (int64_t)r * a.ld, bv, y); };
   X(XR_RUNOFFSEAL, x.rseal);
   X(XR_AETSEAL, x.aseal);
   X(XR_FAST, x.fast);
@@ -162,7 +214,7 @@ __device__ __forceinline__ void store_fluxes_pre(const CellArgs &a, uint32_t bv0
   }
 }
 
-// the fluxes chain_post sets
+// those of the slow interflow and the groundwater
 template <int NH>
 __device__ __forceinline__ void store_fluxes_post(const CellArgs &a, uint32_t bv0,
                                                   const FluxRegs<NH> &x) {
@@ -176,7 +228,8 @@ __device__ __forceinline__ void store_fluxes_post(const CellArgs &a, uint32_t bv
 
 template <int NH>
 __device__ __forceinline__ void store_fluxes(const CellArgs &a, uint32_t bv, const FluxRegs<NH> &x) {
-  store_fluxes_pre<NH>(a, bv, x);
+  store_fluxes_canopy<NH>(a, bv, x);
+  store_fluxes_soil<NH>(a, bv, x);
   store_fluxes_post<NH>(a, bv, x);
 }
 
@@ -185,63 +238,70 @@ __device__ __forceinline__ void store_fluxes(const CellArgs &a, uint32_t bv, con
 // output's value of the step -- states after it, its fluxes -- in the
 // reference's expression and operation order, added to its sum.  Horizon
 // sums run from 0 over the horizons in order (sum(..., dim = 2)); the
-// unsealed fraction is 1 - fSealed (mo_mhm_interface_run.f90:239).
-template <int NH>
-__device__ __forceinline__ double pick_h(const double *v, int h) {
-  double y = v[0];
-#pragma unroll
-  for (int k = 1; k < NH; ++k)
-    if (h == k) y = v[k];
-  return y;
+// unsealed fraction is 1 - fSealed (mo_mhm_interface_run.f90:239).  In three
+// parts, each as soon as its values are known; put(bit, value) is called
+// for the outputs in the order of their bits.
+template <int NH, typename Put>
+__device__ __forceinline__ void outputs_canopy(const CellRegs<NH> &c, const FluxRegs<NH> &x,
+                                               Put put) {
+  put(out_bit(1, 0, NH), [&] { return c.inter; });
+  put(out_bit(2, 0, NH), [&] { return c.pack; });
+  put(out_bit(9, 0, NH), [&] { return x.pet; });
+  put(out_bit(20, 0, NH), [&] { return x.peff; });
+  put(out_bit(21, 0, NH), [&] { return x.melt; });
 }
 
-template <int NH>
-__device__ __forceinline__ void add_outputs(const CellArgs &a, uint32_t bv, const CellRegs<NH> &c,
-                                         const FluxRegs<NH> &x) {
+template <int NH, typename Put>
+__device__ __forceinline__ void outputs_soil(const CellRegs<NH> &c, const FluxRegs<NH> &x,
+                                             double ecan, Put put) {
   const double fs = c.fS, fns = 1.0 - c.fS;
-  for (int r = 0; r < a.out.n; ++r) {
-    const int h = a.out.hor[r];
-    double v = 0.0;
-    switch (a.out.kind[r]) {
-      case 1: v = c.inter; break;
-      case 2: v = c.pack; break;
-      case 3: v = pick_h<NH>(c.sm, h); break;
-      case 4: v = pick_h<NH>(c.sm, h) / pick_h<NH>(c.sat, h); break;
-      case 5: {
-        double s1 = 0.0, s2 = 0.0;
+  auto hsum = [](const double (&v)[NH]) {
+    double s = 0.0;
 #pragma unroll
-        for (int k = 0; k < NH; ++k) s1 = s1 + c.sm[k];
+    for (int h = 0; h < NH; ++h) s = s + v[h];
+    return s;
+  };
 #pragma unroll
-        for (int k = 0; k < NH; ++k) s2 = s2 + c.sat[k];
-        v = s1 / s2;
-        break;
-      }
-      case 6: v = c.seal; break;
-      case 7: v = c.unsat; break;
-      case 8: v = c.satS; break;
-      case 9: v = x.pet; break;
-      case 10: {
-        double s1 = 0.0;
+  for (int h = 0; h < NH; ++h) put(out_bit(3, h, NH), [&] { return c.sm[h]; });
 #pragma unroll
-        for (int k = 0; k < NH; ++k) s1 = s1 + x.aet[k];
-        v = s1 * fns + x.ecan + x.aseal * fs;
-        break;
-      }
-      case 11: v = x.total; break;
-      case 12: v = x.rseal * fs; break;
-      case 13: v = x.fast * fns; break;
-      case 14: v = x.slow * fns; break;
-      case 15: v = x.bflow * fns; break;
-      case 16: v = x.perc * fns; break;
-      case 17: v = pick_h<NH>(x.infil, h) * fns; break;
-      case 19: v = pick_h<NH>(x.aet, h) * fns; break;
-      case 20: v = x.peff; break;
-      case 21: v = x.melt; break;
-      default: break;
-    }
-    double *row = a.out.sum + (int64_t)r * a.ld;
-    str(row, bv, ldr(row, bv) + v);
-  }
+  for (int h = 0; h < NH; ++h) put(out_bit(4, h, NH), [&] { return c.sm[h] / c.sat[h]; });
+  put(out_bit(5, 0, NH), [&] { return hsum(c.sm) / hsum(c.sat); });
+  put(out_bit(6, 0, NH), [&] { return c.seal; });
+  put(out_bit(10, 0, NH), [&] { return hsum(x.aet) * fns + ecan + x.aseal * fs; });
+  put(out_bit(12, 0, NH), [&] { return x.rseal * fs; });
+  put(out_bit(13, 0, NH), [&] { return x.fast * fns; });
+#pragma unroll
+  for (int h = 0; h < NH; ++h) put(out_bit(17, h, NH), [&] { return x.infil[h] * fns; });
+#pragma unroll
+  for (int h = 0; h < NH; ++h) put(out_bit(19, h, NH), [&] { return x.aet[h] * fns; });
+}
+
+template <int NH, typename Put>
+__device__ __forceinline__ void outputs_post(const CellRegs<NH> &c, const FluxRegs<NH> &x,
+                                             Put put) {
+  const double fns = 1.0 - c.fS;
+  put(out_bit(7, 0, NH), [&] { return c.unsat; });
+  put(out_bit(8, 0, NH), [&] { return c.satS; });
+  put(out_bit(11, 0, NH), [&] { return x.total; });
+  put(out_bit(14, 0, NH), [&] { return x.slow * fns; });
+  put(out_bit(15, 0, NH), [&] { return x.bflow * fns; });
+  put(out_bit(16, 0, NH), [&] { return x.perc * fns; });
+}
+
+// The plain kernel's: straight to the sums.
+template <int NH>
+__device__ __forceinline__ void add_outputs(ConstArgs *k, int64_t ld, uint32_t bv,
+                                            const CellRegs<NH> &c, const FluxRegs<NH> &x) {
+  const uint64_t mask = k->out.mask;
+  double *row = k->out.sum;
+  auto put = [&](int bit, auto value) {
+    if (!(mask >> bit & 1)) return;
+    str(row, bv, ldr(row, bv) + value());
+    row += ld;
+  };
+  outputs_canopy<NH>(c, x, put);
+  outputs_soil<NH>(c, x, x.ecan, put);
+  outputs_post<NH>(c, x, put);
 }
 
 // Daily PET before disaggregation (get_corrected_pet, mo_meteo_handler.f90:1050-1097).
@@ -321,16 +381,17 @@ __device__ __forceinline__ StepDev read_step(const ConstStep *p) {
   st.isday = p->isday;
   st.init_sm = p->init_sm;
   st.doy = p->doy;
-  st.meteo_same = p->meteo_same;
+  st.change = p->change;
   st.wrow = p->wrow;
   return st;
 }
 
 // L11_runoff_acc for L1 = L11 with map_flag (mo_mrm_pre_routing.f90:110-126):
-// qAcc = 0; qAcc = qAcc + q * area; qAcc = qAcc * 1000 / TST   [m3 s-1]
-// (rtst = RN(1/TST): the division as div_rcp, same bits)
-__device__ __forceinline__ double runoff_acc(double q, double area, double tst, double rtst) {
-  return div_rcp((0.0 + q * area) * 1000.0, tst, rtst);
+// qAcc = 0; qAcc = qAcc + q * area; qAcc = qAcc * 1000 / TST   [m3 s-1], as q
+// times the cell's area * 1000 / TST (one product a step instead of two and a
+// division; as many roundings).  raw_total: the total itself.
+__device__ __forceinline__ double runoff_scale(const CellArgs &a, uint32_t bc) {
+  return a.raw_total ? 1.0 : ldr(a.area, bc) * 1000.0 / a.tst;
 }
 
 // Every horizon's (sm / sat)**beta depends only on the soil moisture at the
@@ -362,25 +423,39 @@ __device__ __forceinline__ DV<NH> horizon_pows(const CellRegs<NH> &c) {
 // unsat**(1 + alpha), percolation, baseflow, total runoff).  The canopy's
 // (interc / interc_max)**(2/3) is pow23.
 // JV: Jarvis soil-moisture stress (processCase(3) = 2, 3) instead of Feddes
-// The soil-moisture stress parameters of a cell (root fractions, field
-// capacity, wilting point, RN(1 / (fc - wp))), passed on their own: the
-// fused kernel keeps them in LDS between steps.
+// The soil-moisture stress parameters of a cell, passed on their own: the
+// fused kernel keeps them in LDS between steps.  For the general functions
+// fw is the field capacity and slope RN(1 / (fc - wp)); for the ordinary ones
+// see stress_ordinary (Feddes does not read fw).
 template <int NH>
 struct Stress {
-  double fr[NH], fc[NH], wp[NH], rfw[NH];
+  double fr[NH], wp[NH], slope[NH], fw[NH];
 };
 
-template <int NH>
-__device__ __forceinline__ Stress<NH> stress_of(const CellRegs<NH> &c) {
+template <int NH, bool JV>
+__device__ __forceinline__ Stress<NH> stress_of(const CellRegs<NH> &c, bool ordinary) {
   Stress<NH> t;
 #pragma unroll
   for (int h = 0; h < NH; ++h) {
+    const double range = (JV && ordinary ? c.sat[h] : c.fc[h]) - c.wp[h];
     t.fr[h] = c.fr[h];
-    t.fc[h] = c.fc[h];
     t.wp[h] = c.wp[h];
-    t.rfw[h] = c.rfw[h];
+    t.slope[h] = (!JV && ordinary ? c.fr[h] : 1.0) / range;
+    t.fw[h] = ordinary ? range : c.fc[h];
   }
   return t;
+}
+
+template <int NH, bool JV>
+__device__ __forceinline__ bool ordinary_cell(const CellRegs<NH> &c, bool init_sm) {
+  bool ok = ordinary_params<NH, JV>(c.fS, c.thrS, c.incr, c.dmaxs, c.dnps, c.k0s, c.k1s, c.k2s,
+                                    c.kps, c.karst, c.alpha, c.thrU, c.sat, c.fr, c.fc, c.wp,
+                                    c.bexp, c.c1);
+  // a step that resets the soil moisture starts from half the field capacity
+  double sm[NH];
+#pragma unroll
+  for (int h = 0; h < NH; ++h) sm[h] = init_sm ? 0.5 * c.fc[h] : c.sm[h];
+  return ok && ordinary_states<NH>(c.pack, c.unsat, c.satS, sm, c.sat);
 }
 
 template <int NH, bool JV>
@@ -389,9 +464,11 @@ __device__ __forceinline__ void chain_pre(CellRegs<NH> &c, FluxRegs<NH> &x, doub
                                           const double *pwh, const Stress<NH> &t) {
   const double ratio = canopy_fill(maxinter, rmaxinter, x.prec, c.inter, x.thr);
   canopy_evap(x.pet, maxinter, ratio, ratio > 0.0 ? pow23(ratio) : 0.0, c.inter, x.ecan);
-  snow_accum_melt(c.incr, c.dmaxs, c.dnps, c.ddthr, x.prec, x.temp, c.tth, x.thr, c.pack, x.ddf,
+  // snow_accum_melt's branch threshold (mo_snow_accum_melt.f90:127)
+  const double ddthr = (c.dmaxs - c.dnps) / c.incr;
+  snow_accum_melt(c.incr, c.dmaxs, c.dnps, ddthr, x.prec, x.temp, c.tth, x.thr, c.pack, x.ddf,
                   x.melt, x.peff, x.rain, x.snow);
-  soil_moisture<NH, JV>(c.fS, c.thrS, c.rthrS, x.pet, evap, revap, c.sat, t.fr, t.fc, t.wp, t.rfw,
+  soil_moisture<NH, JV>(c.fS, c.thrS, c.rthrS, x.pet, evap, revap, c.sat, t.fr, t.fw, t.wp, t.slope,
                         c.c1, x.ecan, x.peff, pwh, x.rseal, c.seal, x.infil, c.sm, x.aet, x.aseal);
   runoff_fast(c.k0s, x.infil[NH - 1], c.thrU, c.unsat, x.fast);
 }
@@ -404,20 +481,166 @@ __device__ __forceinline__ void chain_post(CellRegs<NH> &c, FluxRegs<NH> &x, dou
 }
 
 template <int NH, bool JV>
-__device__ __forceinline__ void chain_step(const CellArgs &a, CellRegs<NH> &c, FluxRegs<NH> &x,
-                                           double maxinter, double rmaxinter, double evap,
-                                           double revap) {
+__device__ __forceinline__ void chain_step(CellRegs<NH> &c, FluxRegs<NH> &x, double maxinter,
+                                           double rmaxinter, double evap, double revap,
+                                           const Stress<NH> &t) {
   const DV<NH> pwh = horizon_pows<NH>(c);
-  chain_pre<NH, JV>(c, x, maxinter, rmaxinter, evap, revap, pwh.v, stress_of<NH>(c));
+  chain_pre<NH, JV>(c, x, maxinter, rmaxinter, evap, revap, pwh.v, t);
   chain_post<NH>(c, x, c.unsat > 0.0 ? exp_ylogx(1.0 + c.alpha, c.unsat) : 0.0);
+}
+
+// The same step for an ordinary cell, in the parts the fused kernel
+// interleaves: canopy and snow; the soil with the horizon powers of the
+// step's starting soil moisture (wet: some lane of the wave has water to
+// infiltrate; a dry wave's powers are not needed) and the fast interflow; the
+// slow interflow (pw_slow: its power), groundwater and total runoff.
+template <int NH>
+__device__ __forceinline__ void ordinary_canopy(CellRegs<NH> &c, FluxRegs<NH> &x, double melt_meteo,
+                                                double cold, double maxinter, double rmaxinter) {
+  canopy_ordinary(x.pet, maxinter, rmaxinter, x.prec, c.inter, x.thr, x.ecan);
+  snow_ordinary(melt_meteo, cold, x.thr, c.pack, x.melt, x.peff, x.rain, x.snow);
+}
+
+template <int NH, bool JV>
+__device__ __forceinline__ void ordinary_soil(CellRegs<NH> &c, FluxRegs<NH> &x, double demand,
+                                              double pe, double ecan, double peff, bool wet,
+                                              const double *pwh, double rc1,
+                                              const Stress<NH> &t) {
+  sealed_ordinary(c.fS > 0.0, c.thrS, c.rthrS, pe, ecan, peff, x.rseal, c.seal, x.aseal);
+#pragma unroll
+  for (int h = 0; h < NH; ++h) x.infil[h] = 0.0;
+  if (wet) {
+#pragma unroll
+    for (int h = 0; h < NH; ++h)
+      x.infil[h] = infiltrate_ordinary(h ? x.infil[h ? h - 1 : 0] : peff, pwh[h], c.sat[h], c.sm[h]);
+  }
+  double used = 0.0;
+#pragma unroll
+  for (int h = 0; h < NH; ++h) {
+    const double f = stress_ordinary<JV>(c.sm[h], t.wp[h], t.fr[h], t.slope[h], t.fw[h], c.c1, rc1);
+    x.aet[h] = evaporate_ordinary(h ? demand - used : demand, f, c.sm[h]);
+    used = h ? used + x.aet[h] : x.aet[h];
+  }
+  runoff_fast_ordinary(c.k0s, x.infil[NH - 1], c.thrU, c.unsat, x.fast);
+}
+
+// what a cell without sealed area reports for it
+template <int NH>
+__device__ __forceinline__ void report_sealed(const CellRegs<NH> &c, FluxRegs<NH> &x) {
+  x.rseal = c.fS > 0.0 ? x.rseal : 0.0;
+  x.aseal = c.fS > 0.0 ? x.aseal : 0.0;
+}
+
+template <int NH>
+__device__ __forceinline__ void ordinary_post(CellRegs<NH> &c, FluxRegs<NH> &x, double pw_slow,
+                                              double rseal) {
+  runoff_slow_perc_ordinary(c.k1s, c.kps, c.karst, pw_slow, c.satS, c.unsat, x.slow, x.perc);
+  x.bflow = c.k2s * c.satS;
+  c.satS = c.satS - x.bflow;
+  x.total = total_runoff(c.fS, x.fast, x.slow, x.bflow, rseal);
+}
+
+// base of the slow interflow's power (an empty store: a power next to 0)
+__device__ __forceinline__ double slow_base(double unsat) { return vmax_k(unsat, DBL_MIN); }
+
+// The plain kernel's: each flux leaves as soon as it is known, so that the
+// registers do not hold them across the powers.
+template <int NH, bool JV>
+__device__ __forceinline__ void ordinary_step(const CellArgs &a, uint32_t bv, CellRegs<NH> &c,
+                                              FluxRegs<NH> &x, double maxinter, double rmaxinter,
+                                              double pe, const Stress<NH> &t) {
+  const SnowMeteo m = snow_meteo(c.incr, c.dmaxs, c.dnps, c.tth, x.prec, x.temp);
+  x.ddf = m.ddf;
+  ordinary_canopy<NH>(c, x, m.melt, m.cold, maxinter, rmaxinter);
+  store_fluxes_canopy<NH>(a, bv, x);
+  const bool wet = __any(x.peff != 0.0);
+  DV<NH> py, px;
+  if (wet) {
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+      py.v[h] = 256.0 * c.bexp[h];
+      px.v[h] = div_rcp(c.sm[h], c.sat[h], c.rsat[h]);
+    }
+    px = pow_v<NH>(py, px);
+  }
+  ordinary_soil<NH, JV>(c, x, x.pet - x.ecan, pe, x.ecan, x.peff, wet, px.v, JV ? 1.0 / c.c1 : 0.0,
+                        t);
+  const double rseal = x.rseal;  // finite, of weight 0 without sealed area
+  report_sealed<NH>(c, x);
+  store_fluxes_soil<NH>(a, bv, x);
+  const DV<1> pw = pow_v<1>(DV<1>{{256.0 * (1.0 + c.alpha)}}, DV<1>{{slow_base(c.unsat)}});
+  ordinary_post<NH>(c, x, pw.v[0], rseal);
+  store_fluxes_post<NH>(a, bv, x);
 }
 
 // ---------------------------------------------------------------------------
 // Plain path: one launch per model step; every state and flux is written.
 // The cell's loads are issued before the log / exp tables are filled, so the
 // fill's reads and barrier wait behind them rather than in front.
+//
+// A cell outside the ordinary ranges reloads everything and takes
+// general_step: out of line, so that the registers of the kernel are those of
+// the ordinary step (four waves per SIMD).
+struct StepArgs {
+  StepDev st;
+  int64_t t;
+};
+
 template <int NH, bool JV, bool OUT>
-__global__ __launch_bounds__(256) void cell_step_kernel(CellArgs a, StepDev st, int64_t t) {
+__device__ __forceinline__ void step_end(ConstArgs *k, const CellArgs &a, uint32_t c, uint32_t bv,
+                                         int64_t t, double scale, int32_t g,
+                                         const CellRegs<NH> &r, const FluxRegs<NH> &x) {
+  store_states<NH>(a, bv, r);
+  if (OUT) add_outputs<NH>(k, a.ld, bv, r, x);
+  if (a.ring) {
+    const double q = x.total * scale;
+    for (int32_t i = 0; i < a.ring_rep; ++i)
+      a.ring[ring_row(t * a.ring_rep + i, g, a.ring_len) * a.ld + bv / 8u] = q;
+  }
+}
+
+template <int NH>
+__device__ __forceinline__ void step_start(const CellArgs &a, const StepDev &st, uint32_t bc,
+                                           uint32_t bv, double pre, double tavg, double tmax,
+                                           double tmin, CellRegs<NH> &r, FluxRegs<NH> &x) {
+  const double pd = pet_day<NH>(a, st, bv, bc, tavg, tmax, tmin);
+  disagg_step<NH>(a, st, bc, pd, tavg, pre, x.pet, x.temp, x.prec);
+  if (st.init_sm) {
+#pragma unroll
+    for (int h = 0; h < NH; ++h) r.sm[h] = 0.5 * r.fc[h];
+  }
+}
+
+template <int NH, bool JV, bool OUT>
+__device__ __attribute__((noinline)) void general_step(ConstArgs *args, uint32_t c, uint32_t bv) {
+  ConstArgs *k = uniform(args);
+  const CellArgs a = read_args(k);
+  const __attribute__((address_space(4))) StepArgs *sa =
+      (const __attribute__((address_space(4))) StepArgs *)(k + 1);
+  const StepDev st = read_step(&sa->st);
+  const uint32_t bc = c * 8u;
+  CellRegs<NH> r;
+  FluxRegs<NH> x;
+  load_params<NH, JV>(a, bv, r);
+  load_states<NH>(a, bv, r);
+  const double pre = ldr(frow_ptr(a, MHMHIP_F_PRE, st.day), bc);
+  const double tavg = ldr(frow_ptr(a, MHMHIP_F_TAVG, st.day), bc);
+  const double tmax = a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMAX, st.day), bc) : 0.0;
+  const double tmin = a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMIN, st.day), bc) : 0.0;
+  step_start<NH>(a, st, bc, bv, pre, tavg, tmax, tmin, r, x);
+  const double maxinter = ldr(a.P + (int64_t)(pr_maxinter(NH) + st.month0) * a.ld, bv);
+  chain_step<NH, JV>(r, x, maxinter, 1.0 / maxinter, st.evap, st.revap,
+                     stress_of<NH, JV>(r, false));
+  store_fluxes<NH>(a, bv, x);
+  step_end<NH, JV, OUT>(k, a, c, bv, sa->t, a.ring ? runoff_scale(a, bc) : 0.0,
+                        a.ring && a.lag ? a.lag[c] : 0, r, x);
+}
+
+template <int NH, bool JV, bool OUT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NH > 3 ? 2 : OUT ? 3 : 4)))
+void cell_step_kernel(CellArgs a, StepArgs sa) {
+  static_assert(sizeof(CellArgs) % alignof(StepArgs) == 0, "StepArgs follows CellArgs");
+  const StepDev &st = sa.st;
   const uint32_t c0 = blockIdx.x * blockDim.x + threadIdx.x;
   const bool act = c0 < a.n_cells;
   const uint32_t c = act ? c0 : 0u;  // an idle lane loads cell 0 and leaves after the fill
@@ -431,38 +654,347 @@ __global__ __launch_bounds__(256) void cell_step_kernel(CellArgs a, StepDev st, 
   const double tavg = ldr(frow_ptr(a, MHMHIP_F_TAVG, st.day), bc);
   const double tmax = a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMAX, st.day), bc) : 0.0;
   const double tmin = a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMIN, st.day), bc) : 0.0;
-  mathtab_fill();  // the chain's log and exp read it (every thread, before any returns)
+  mathtab_fill();  // the chain's powers read it (every thread, before any returns)
   if (!act) return;
-  const double pd = pet_day<NH>(a, st, bv, bc, tavg, tmax, tmin);
-  disagg_step<NH>(a, st, bc, pd, tavg, pre, x.pet, x.temp, x.prec);
-  if (st.init_sm) {
-#pragma unroll
-    for (int h = 0; h < NH; ++h) r.sm[h] = 0.5 * r.fc[h];
+  const bool ordinary = ordinary_cell<NH, JV>(r, st.init_sm != 0);
+  if (ordinary) {
+    double scale = a.ring ? runoff_scale(a, bc) : 0.0;
+    int32_t g = a.ring && a.lag ? a.lag[c] : 0;
+    step_start<NH>(a, st, bc, bv, pre, tavg, tmax, tmin, r, x);
+    double maxinter = ldr(a.P + (int64_t)(pr_maxinter(NH) + st.month0) * a.ld, bv);
+    // no load is waited for once the stores start: they share a counter
+    settle(maxinter);
+    settle(scale);
+    asm volatile("" : "+v"(g));
+    settle_all<NH>(r);
+    ordinary_step<NH, JV>(a, bv, r, x, maxinter, maxinter > kEps ? 1.0 / maxinter : 0.0,
+                          div_rcp(x.pet, st.evap, st.revap), stress_of<NH, JV>(r, true));
+    step_end<NH, JV, OUT>(kernel_args(), a, c, bv, sa.t, scale, g, r, x);
   }
-  const double maxinter = ldr(a.P + (int64_t)(pr_maxinter(NH) + st.month0) * a.ld, bv);
-  chain_step<NH, JV>(a, r, x, maxinter, 1.0 / maxinter, st.evap, st.revap);
-  store_states<NH>(a, bv, r);
-  store_fluxes<NH>(a, bv, x);
-  if (OUT) add_outputs<NH>(a, bv, r, x);
-  if (a.ring) {
-    const double q = a.raw_total ? x.total : runoff_acc(x.total, ldr(a.area, bc), a.tst, a.rtst);
-    const int32_t g = a.lag ? a.lag[c] : 0;
-    for (int32_t i = 0; i < a.ring_rep; ++i)
-      a.ring[ring_row(t * a.ring_rep + i, g, a.ring_len) * a.ld + bv / 8u] = q;
-  }
+  // last, where the call finds no other value in use
+  if (!ordinary) general_step<NH, JV, OUT>(kernel_args(), opaque(c), opaque(bv));
 }
 
 // Per-lane LDS slots of the fused kernel (dynamic shared memory,
-// lane_slots(NH) doubles per thread, laid out lane after lane; an odd count
+// lane_slots doubles per thread, laid out lane after lane; an odd count
 // puts the 64-bit accesses of a wave's lanes on distinct bank pairs): the
-// values that change once per forcing day, month or day/night switch, and
-// the soil-moisture stress parameters read once per step -- in LDS rather
-// than in registers across the whole time loop.
+// values that change once per forcing day, month or day/night switch, the
+// soil-moisture stress parameters read once per step and the launch's output
+// sums -- in LDS rather than in registers across the whole time loop.  The
+// sums take the steps' values in step order as they would in memory, and cost
+// a launch one read and one write of a row instead of one per step.
 enum LaneSlot {
-  LS_PRE = 0, LS_TAVG, LS_PD, LS_MAXI, LS_RMAXI, LS_XPET, LS_XTEMP, LS_XPREC, LS_STRESS
+  LS_PD = 0, LS_MAXI, LS_RMAXI, LS_XPET, LS_XPE, LS_XPREC, LS_XMELT, LS_XCOLD, LS_STRESS
 };
-__host__ __device__ constexpr int lane_slots(int nh) { return (LS_STRESS + 4 * nh) | 1; }
+// Jarvis and the general functions read a fourth stress parameter; a general
+// lane of the Feddes kernel takes it from memory
+__host__ __device__ constexpr int stress_slots(int nh, bool jv) { return (jv ? 4 : 3) * nh; }
+__host__ __device__ constexpr int lane_slots(int nh, bool jv, int n_out) {
+  return (LS_STRESS + stress_slots(nh, jv) + n_out) | 1;
+}
 extern __shared__ double s_lane[];
+
+// The lane's place in a fused launch.
+struct FusedLane {
+  uint32_t bc, bv;     // byte offsets of the cell in a forcing row, of (cell, set) in a row
+  uint32_t slot;       // first LDS slot
+  double scale;        // runoff_scale
+  double *ring;        // ring row 0 of the node (its lag folded in), null: no routing
+  int64_t roff;        // element offset of the step's first ring row
+};
+
+// The step's qOUT to its rep ring rows.
+__device__ __forceinline__ void put_ring(const CellArgs &a, FusedLane &u, int64_t wrap, int rep,
+                                         double total) {
+  if (!a.ring) return;
+  const double q = total * u.scale;
+  int i = rep;
+  do {
+    u.ring[u.roff] = q;
+    u.roff += a.ld;
+    if (u.roff == wrap) u.roff = 0;
+  } while (--i > 0);
+}
+
+// disagg_step with the forcing day's values read here
+template <int NH>
+__device__ __forceinline__ void disagg_at(const CellArgs &a, const StepDev &st, uint32_t bc,
+                                          double pd, double &pet, double &temp, double &prec) {
+  const double pre = ldr(frow_ptr(a, MHMHIP_F_PRE, st.day), bc);
+  const double tavg = ldr(frow_ptr(a, MHMHIP_F_TAVG, st.day), bc);
+  disagg_step<NH>(a, st, bc, pd, tavg, pre, pet, temp, prec);
+}
+
+// The daily PET into its slot, out of line and from its own loads: the time
+// loop around it holds no register for it.
+template <int NH>
+__device__ __attribute__((noinline)) void day_pet(ConstArgs *args, uint32_t bc, uint32_t bv,
+                                                  uint32_t slot, const ConstStep *step) {
+  const CellArgs a = read_args(uniform(args));
+  const StepDev st = read_step((const ConstStep *)uniform((ConstArgs *)step));
+  const double tavg = ldr(frow_ptr(a, MHMHIP_F_TAVG, st.day), bc);
+  const double tmax = a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMAX, st.day), bc) : 0.0;
+  const double tmin = a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMIN, st.day), bc) : 0.0;
+  s_lane[slot + LS_PD] = pet_day<NH>(a, st, bv, bc, tavg, tmax, tmin);
+}
+
+// The daily PET, the month's interception capacity and the step's
+// disaggregated meteo values, with what follows from them alone, into the
+// lane's slots, as far as the step changes them.
+template <int NH>
+__device__ __forceinline__ void look_up(ConstArgs *k, const FusedLane &u, const ConstStep *p,
+                                        int change, bool ordinary) {
+  if (change & SC_DAY) day_pet<NH>(k, u.bc, u.bv, u.slot, p);
+  const CellArgs a = read_args(rare(k));
+  const StepDev st = read_step(p);
+  // offsets opaque here: no per-lane address of these rows is held across
+  // the time loop
+  const uint32_t li = opaque(u.slot), oc = opaque(u.bc), ov = opaque(u.bv);
+  auto P = [&](int r) { return ldr(a.P + (int64_t)r * a.ld, ov); };
+  if (change & SC_MONTH) {
+    const double maxinter = P(pr_maxinter(NH) + st.month0);
+    s_lane[li + LS_MAXI] = maxinter;
+    s_lane[li + LS_RMAXI] = maxinter > kEps || !ordinary ? 1.0 / maxinter : 0.0;
+  }
+  double pet, temp, prec;
+  disagg_at<NH>(a, st, oc, s_lane[li + LS_PD], pet, temp, prec);
+  s_lane[li + LS_XPET] = pet;
+  s_lane[li + LS_XPREC] = prec;
+  if (ordinary) {
+    const SnowMeteo m = snow_meteo(P(PR_INCR), P(PR_DMAXS), P(PR_DNPS), P(PR_TTH), prec, temp);
+    s_lane[li + LS_XPE] = div_rcp(pet, st.evap, st.revap);
+    s_lane[li + LS_XMELT] = m.melt;
+    s_lane[li + LS_XCOLD] = m.cold;
+  } else {
+    s_lane[li + LS_XMELT] = temp;  // a general lane keeps the temperature there
+  }
+}
+
+// The temperature and the degree-day factor of a launch's last step, for its
+// fluxes: looked up again (the loop keeps what follows from them).
+template <int NH>
+__device__ __forceinline__ void last_meteo(ConstArgs *k, const FusedLane &u, const ConstStep *p,
+                                           FluxRegs<NH> &x) {
+  const CellArgs a = read_args(rare(k));
+  const StepDev st = read_step(p);
+  const uint32_t ov = opaque(u.bv);
+  auto P = [&](int r) { return ldr(a.P + (int64_t)r * a.ld, ov); };
+  double pet, prec;
+  disagg_at<NH>(a, st, opaque(u.bc), 0.0, pet, x.temp, prec);
+  x.ddf = snow_meteo(P(PR_INCR), P(PR_DMAXS), P(PR_DNPS), P(PR_TTH), prec, x.temp).ddf;
+}
+
+// Adds an output's value to the lane's sum slots, which follow one another in
+// the order of the selected bits (o: the next one's slot).
+__device__ __forceinline__ auto out_slots(uint64_t mask, uint32_t &o) {
+  return [mask, &o](int bit, auto value) {
+    if (!(mask >> bit & 1)) return;
+    s_lane[o] = s_lane[o] + value();
+    ++o;
+  };
+}
+__device__ __forceinline__ void load_sums(ConstArgs *k, int64_t ld, uint32_t bv, uint32_t o) {
+  for (int r = 0; r < k->out.n; ++r) s_lane[o + r] = ldr(k->out.sum + r * ld, bv);
+}
+__device__ __forceinline__ void store_sums(ConstArgs *k, int64_t ld, uint32_t bv, uint32_t o) {
+  for (int r = 0; r < k->out.n; ++r) str(k->out.sum + r * ld, bv, s_lane[o + r]);
+}
+
+template <int NH, bool JV>
+__device__ __forceinline__ Stress<NH> read_stress(uint32_t li) {
+  Stress<NH> t;
+#pragma unroll
+  for (int h = 0; h < NH; ++h) {
+    t.fr[h] = s_lane[li + LS_STRESS + h];
+    t.wp[h] = s_lane[li + LS_STRESS + NH + h];
+    t.slope[h] = s_lane[li + LS_STRESS + 2 * NH + h];
+    t.fw[h] = JV ? s_lane[li + LS_STRESS + (JV ? 3 : 0) * NH + h] : 0.0;
+  }
+  return t;
+}
+
+// The lane's slots and its place in the ring: the lane's row offset (its lag)
+// is fixed, the step's row uniform.
+template <int NH, bool JV>
+__device__ __forceinline__ void fused_lane(const CellArgs &a, uint32_t c, uint32_t bv,
+                                           uint32_t slot, int64_t t0, const Stress<NH> &t,
+                                           FusedLane &u) {
+  u.bc = c * 8u;
+  u.bv = bv;
+  u.slot = slot;
+#pragma unroll
+  for (int h = 0; h < NH; ++h) {
+    s_lane[slot + LS_STRESS + h] = t.fr[h];
+    s_lane[slot + LS_STRESS + NH + h] = t.wp[h];
+    s_lane[slot + LS_STRESS + 2 * NH + h] = t.slope[h];
+    if (JV) s_lane[slot + LS_STRESS + (JV ? 3 : 0) * NH + h] = t.fw[h];
+  }
+  u.scale = 0.0;
+  u.ring = nullptr;
+  u.roff = 0;
+  if (a.ring) {
+    u.scale = runoff_scale(a, u.bc);
+    u.ring = a.ring + (int64_t)(a.lag ? a.lag[c] : 0) * a.ld + bv / 8u;
+    u.roff = t0 * a.ring_rep % a.ring_len * a.ld;
+  }
+}
+
+// what the first step of a launch looks up
+constexpr int kAllChanged = SC_METEO | SC_DAY | SC_MONTH;
+
+// The time loop of an ordinary cell.  Turn s of the loop finishes step s and
+// starts step s + 1: the canopy and snow of step s + 1 need nothing of the
+// soil and its horizon powers nothing but the soil moisture step s leaves, so
+// these powers and step s's slow-interflow power run as one batch of
+// independent chains, and a wave in which no lane has water to infiltrate at
+// step s + 1 leaves the horizon powers out.  The first turn only starts.
+template <int NH, bool JV, bool OUT>
+__device__ __forceinline__ void fused_ordinary(const CellArgs &a, FusedLane &u, CellRegs<NH> &r,
+                                               const ConstStep *steps, int32_t nsteps) {
+  ConstArgs *k = kernel_args();
+  const uint64_t mask = OUT ? k->out.mask : 0;
+  const int n_canopy = __builtin_popcountll(mask & 0x1F);  // outputs_canopy's bits
+  if (OUT) load_sums(k, a.ld, u.bv, u.slot + LS_STRESS + stress_slots(NH, JV));
+  const int rep = a.ring_rep;
+  const int64_t wrap = a.ring_len * a.ld;
+  // exponents in units of 1/256 (pow_v)
+  const double alpha256 = 256.0 * (1.0 + r.alpha), rc1 = JV ? 1.0 / r.c1 : 0.0;
+#pragma unroll
+  for (int h = 0; h < NH; ++h) r.bexp[h] = 256.0 * r.bexp[h];
+  FluxRegs<NH> x;
+  // step s + 1's canopy evaporation, demand left (pet - ecan), effective
+  // precipitation and horizon powers, carried into the next turn
+  double ecan = 0.0, demand = 0.0, peff = 0.0;
+  DV<NH> pwh;
+#pragma unroll
+  for (int h = 0; h < NH; ++h) pwh.v[h] = 0.0;
+  bool wet = false;
+#pragma nounroll
+  for (int32_t s = -1; s < nsteps; ++s) {
+    const bool last = s == nsteps - 1;
+    uint32_t o = opaque(u.slot) + LS_STRESS + stress_slots(NH, JV);  // output sum slots
+    if (s >= 0) {
+      const uint32_t li = opaque(u.slot);
+      ordinary_soil<NH, JV>(r, x, demand, s_lane[li + LS_XPE], ecan, peff, wet, pwh.v, rc1,
+                            read_stress<NH, JV>(li));
+      if (last || OUT) {
+        FluxRegs<NH> y = x;
+        report_sealed<NH>(r, y);
+        if (last) store_fluxes_soil<NH>(read_args(rare(k)), u.bv, y);
+        if (OUT) {
+          o = opaque(u.slot) + LS_STRESS + stress_slots(NH, JV) + n_canopy;
+          outputs_soil<NH>(r, y, ecan, out_slots(mask, o));
+        }
+      }
+    }
+    if (!last) {
+      const ConstStep *next = steps + (s + 1);
+      const int change = next->change | (s < 0 ? kAllChanged : 0);
+      if (change) {
+        if (change & kAllChanged) look_up<NH>(k, u, next, change, true);
+        if (change & SC_INIT) {
+          ConstArgs *q = rare(k);
+          const uint32_t ov = opaque(u.bv);
+#pragma unroll
+          for (int h = 0; h < NH; ++h) {
+            r.sm[h] = 0.5 * ldr(q->P + (int64_t)(pr_fc(NH) + h) * q->ld, ov);
+            settle(r.sm[h]);
+          }
+        }
+      }
+      const uint32_t li = opaque(u.slot);
+      x.pet = s_lane[li + LS_XPET];
+      x.prec = s_lane[li + LS_XPREC];
+      ordinary_canopy<NH>(r, x, s_lane[li + LS_XMELT], s_lane[li + LS_XCOLD],
+                          s_lane[li + LS_MAXI], s_lane[li + LS_RMAXI]);
+      if (s + 2 == nsteps) {
+        last_meteo<NH>(k, u, next, x);
+        store_fluxes_canopy<NH>(read_args(rare(k)), u.bv, x);
+      }
+      if (OUT) {
+        uint32_t oc = opaque(u.slot) + LS_STRESS + stress_slots(NH, JV);
+        outputs_canopy<NH>(r, x, out_slots(mask, oc));
+      }
+      ecan = x.ecan;
+      demand = x.pet - x.ecan;
+      peff = x.peff;
+      wet = __any(peff != 0.0);
+    }
+    double pw_slow;
+    if (wet && !last) {
+      DV<NH + 1> py, px;
+      py.v[0] = alpha256;
+      px.v[0] = slow_base(r.unsat);
+#pragma unroll
+      for (int h = 0; h < NH; ++h) {
+        py.v[h + 1] = r.bexp[h];
+        px.v[h + 1] = div_rcp(r.sm[h], r.sat[h], r.rsat[h]);
+      }
+      px = pow_v<NH + 1>(py, px);
+      pw_slow = px.v[0];
+#pragma unroll
+      for (int h = 0; h < NH; ++h) pwh.v[h] = px.v[h + 1];
+    } else {
+      pw_slow = pow_v<1>(DV<1>{{alpha256}}, DV<1>{{slow_base(r.unsat)}}).v[0];
+    }
+    if (s >= 0) {
+      ordinary_post<NH>(r, x, pw_slow, x.rseal);
+      put_ring(a, u, wrap, rep, x.total);
+      if (last) store_fluxes_post<NH>(read_args(rare(k)), u.bv, x);
+      if (OUT) outputs_post<NH>(r, x, out_slots(mask, o));
+    }
+  }
+  if (OUT) store_sums(k, a.ld, u.bv, u.slot + LS_STRESS + stress_slots(NH, JV));
+}
+
+// The time loop of any other cell, out of line and from its own loads (see
+// general_step): the registers of the kernel are those of the ordinary loop.
+struct FusedArgs {
+  int64_t t0;
+  int32_t nsteps, step0;
+};
+
+template <int NH, bool JV, bool OUT>
+__device__ __attribute__((noinline)) void fused_general(ConstArgs *args, uint32_t c, uint32_t bv,
+                                                        uint32_t slot) {
+  ConstArgs *k = uniform(args);
+  const CellArgs a = read_args(k);
+  const __attribute__((address_space(4))) FusedArgs *fa =
+      (const __attribute__((address_space(4))) FusedArgs *)(k + 1);
+  const int32_t nsteps = fa->nsteps;
+  const ConstStep *steps = (const ConstStep *)(a.steps + fa->step0);
+  CellRegs<NH> r;
+  load_params<NH, JV>(a, bv, r);
+  load_states<NH>(a, bv, r);
+  FusedLane u;
+  fused_lane<NH, JV>(a, c, bv, slot, fa->t0, stress_of<NH, JV>(r, false), u);
+  const int rep = a.ring_rep;
+  const int64_t wrap = a.ring_len * a.ld;
+#pragma nounroll
+  for (int32_t s = 0; s < nsteps; ++s) {
+    const ConstStep *p = steps + s;
+    const int change = p->change | (s == 0 ? kAllChanged : 0);
+    if (change & kAllChanged) look_up<NH>(k, u, p, change, false);
+    const uint32_t li = opaque(u.slot);
+    Stress<NH> t = read_stress<NH, JV>(li);
+#pragma unroll
+    for (int h = 0; h < NH; ++h)
+      t.fw[h] = ldr(a.P + (int64_t)(pr_fc(NH) + h) * a.ld, opaque(bv));
+    if (change & SC_INIT) {
+#pragma unroll
+      for (int h = 0; h < NH; ++h) r.sm[h] = 0.5 * t.fw[h];
+    }
+    FluxRegs<NH> x;
+    x.pet = s_lane[li + LS_XPET];
+    x.temp = s_lane[li + LS_XMELT];
+    x.prec = s_lane[li + LS_XPREC];
+    chain_step<NH, JV>(r, x, s_lane[li + LS_MAXI], s_lane[li + LS_RMAXI], p->evap, p->revap, t);
+    put_ring(a, u, wrap, rep, x.total);
+    if (s == nsteps - 1) store_fluxes<NH>(a, u.bv, x);
+    if (OUT) add_outputs<NH>(k, a.ld, u.bv, r, x);
+  }
+  store_states<NH>(a, bv, r);
+}
 
 // ---------------------------------------------------------------------------
 // Fused path: nsteps model steps per launch with parameters and states held
@@ -470,132 +1002,33 @@ extern __shared__ double s_lane[];
 // (the reference recomputes the same value every hour), maximum interception
 // once per month.  Only the routing input leaves the lane each step; states
 // are written at the end and the last step's fluxes as soon as each is known.
-// Per-step fluxes are scoped to the loop body so they do not stay live across
-// steps.
+// A cell takes the ordinary or the general loop by its own parameters and
+// states, whatever the wave's other lanes take.
 template <int NH, bool JV, bool OUT>
-#ifndef MHMHIP_FUSED_WAVES
-#define MHMHIP_FUSED_WAVES 2
-#endif
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MHMHIP_FUSED_WAVES)))
-void cell_fused_kernel(CellArgs a, int64_t t0, int32_t nsteps,
-                                                         int32_t step0) {
-  mathtab_fill();  // the chain's log and exp read it (before any thread returns)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NH > 3 ? 2 : JV || OUT ? 3 : 4)))
+void cell_fused_kernel(CellArgs a, FusedArgs fa) {
+  static_assert(sizeof(CellArgs) % alignof(FusedArgs) == 0, "FusedArgs follows CellArgs");
+  mathtab_fill();  // the chain's powers read it (before any thread returns)
   const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= a.n_cells) return;
-  const uint32_t bc = c * 8u;
   const uint32_t bv = (uint32_t)(blockIdx.y * a.sstride + c) * 8u;
+  // this lane's LDS slots (lane_slots doubles, laid out lane by lane)
+  const uint32_t slot = threadIdx.x * (uint32_t)lane_slots(NH, JV, OUT ? a.out.n : 0);
+  const ConstStep *steps = (const ConstStep *)(a.steps + fa.step0);
   CellRegs<NH> r;
   load_params<NH, JV>(a, bv, r);
   load_states<NH>(a, bv, r);
-  // this lane's LDS slots (lane_slots(NH) doubles, laid out lane by lane)
-  const uint32_t lane0 = threadIdx.x * (uint32_t)lane_slots(NH);
-#pragma unroll
-  for (int h = 0; h < NH; ++h) {
-    s_lane[lane0 + LS_STRESS + h] = r.fr[h];
-    s_lane[lane0 + LS_STRESS + NH + h] = r.fc[h];
-    s_lane[lane0 + LS_STRESS + 2 * NH + h] = r.wp[h];
-    s_lane[lane0 + LS_STRESS + 3 * NH + h] = r.rfw[h];
+  const bool ordinary = ordinary_cell<NH, JV>(r, steps->init_sm != 0);
+  if (ordinary) {
+    FusedLane u;
+    fused_lane<NH, JV>(a, c, bv, slot, fa.t0, stress_of<NH, JV>(r, true), u);
+    settle(u.scale);
+    settle_all<NH>(r);
+    fused_ordinary<NH, JV, OUT>(a, u, r, steps, fa.nsteps);
+    store_states<NH>(a, bv, r);
   }
-  const double area = a.ring ? ldr(a.area, bc) : 0.0;
-  int cached_day = -1, cached_doy = -1, cached_month = -1;
-  const ConstStep *steps = (const ConstStep *)(a.steps + step0);
-  // ring: the lane's row offset (its lag) is fixed, the step's row uniform
-  double *rlane = nullptr;
-  int64_t roff = 0;
-  if (a.ring) {
-    rlane = a.ring + (int64_t)(a.lag ? a.lag[c] : 0) * a.ld + bv / 8u;
-    roff = t0 * a.ring_rep % a.ring_len * a.ld;
-  }
-  // The horizon powers of a step depend only on its starting soil moisture,
-  // known when the step before reaches its slow interflow: one call
-  // evaluates that step's unsat**(1 + alpha) and the next step's NH horizon
-  // powers side by side (independent chains for the scheduler); the first
-  // step's come from here, a step that resets the soil moisture recomputes.
-  DV<NH> pwh = horizon_pows<NH>(r);
-#pragma nounroll
-  for (int32_t s = 0; s < nsteps; ++s) {
-    const StepDev st = read_step(steps + s);
-    // the slot index opaque each step: the slots are read where they are
-    // used, not held in registers across the loop
-    const uint32_t li = opaque(lane0);
-    if (st.day != cached_day || st.doy != cached_doy) {
-      // offsets opaque here: no per-lane address of these rows is held
-      // across the time loop
-      const uint32_t oc = opaque(bc), ov = opaque(bv);
-      const double pre = ldr(frow_ptr(a, MHMHIP_F_PRE, st.day), oc);
-      const double tavg = ldr(frow_ptr(a, MHMHIP_F_TAVG, st.day), oc);
-      const double tmax =
-          a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMAX, st.day), oc) : 0.0;
-      const double tmin =
-          a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMIN, st.day), oc) : 0.0;
-      s_lane[li + LS_PRE] = pre;
-      s_lane[li + LS_TAVG] = tavg;
-      s_lane[li + LS_PD] = pet_day<NH>(a, st, ov, oc, tavg, tmax, tmin);
-      cached_day = st.day;
-      cached_doy = st.doy;
-    }
-    if (st.month0 != cached_month) {
-      const double maxinter = ldr(a.P + (int64_t)(pr_maxinter(NH) + st.month0) * a.ld,
-                                  opaque(bv));
-      s_lane[li + LS_MAXI] = maxinter;
-      s_lane[li + LS_RMAXI] = 1.0 / maxinter;
-      cached_month = st.month0;
-    }
-    FluxRegs<NH> x;
-    if (s == 0 || !st.meteo_same) {
-      // day or night factors changed (or a new day): disaggregate again
-      const double pd = s_lane[li + LS_PD], tavg = s_lane[li + LS_TAVG];
-      const double pre = s_lane[li + LS_PRE];
-      disagg_step<NH>(a, st, opaque(bc), pd, tavg, pre, x.pet, x.temp, x.prec);
-      s_lane[li + LS_XPET] = x.pet;
-      s_lane[li + LS_XTEMP] = x.temp;
-      s_lane[li + LS_XPREC] = x.prec;
-    } else {
-      x.pet = s_lane[li + LS_XPET];
-      x.temp = s_lane[li + LS_XTEMP];
-      x.prec = s_lane[li + LS_XPREC];
-    }
-    Stress<NH> t;
-#pragma unroll
-    for (int h = 0; h < NH; ++h) {
-      t.fr[h] = s_lane[li + LS_STRESS + h];
-      t.fc[h] = s_lane[li + LS_STRESS + NH + h];
-      t.wp[h] = s_lane[li + LS_STRESS + 2 * NH + h];
-      t.rfw[h] = s_lane[li + LS_STRESS + 3 * NH + h];
-    }
-    if (st.init_sm) {
-#pragma unroll
-      for (int h = 0; h < NH; ++h) r.sm[h] = 0.5 * t.fc[h];
-      pwh = horizon_pows<NH>(r);
-    }
-    chain_pre<NH, JV>(r, x, s_lane[li + LS_MAXI], s_lane[li + LS_RMAXI], st.evap, st.revap,
-                      pwh.v, t);
-    // the last step's fluxes leave as soon as they are known, so that they
-    // are not held across the powers
-    const bool last = s == nsteps - 1;
-    if (last && !OUT) store_fluxes_pre<NH>(a, bv, x);
-    DV<NH + 1> py, px;
-    py.v[0] = 1.0 + r.alpha;
-    px.v[0] = r.unsat > 0.0 ? r.unsat : 1.0;
-    horizon_pow_args<NH, NH + 1>(r, py, px, 1);
-    const DV<NH + 1> pw = exp_ylogx_v<NH + 1>(py, px);
-    chain_post<NH>(r, x, r.unsat > 0.0 ? pw.v[0] : 0.0);
-#pragma unroll
-    for (int h = 0; h < NH; ++h) pwh.v[h] = pw.v[h + 1];
-    if (a.ring) {
-      // the step's qOUT for each of its routing sub-steps (rows in routing steps)
-      const double q = a.raw_total ? x.total : runoff_acc(x.total, area, a.tst, a.rtst);
-      for (int32_t i = 0; i < a.ring_rep; ++i) {
-        rlane[roff] = q;
-        roff += a.ld;
-        if (roff == a.ring_len * a.ld) roff = 0;
-      }
-    }
-    if (last && OUT) store_fluxes_pre<NH>(a, bv, x);
-    if (last) store_fluxes_post<NH>(a, bv, x);
-    if (OUT) add_outputs<NH>(a, bv, r, x);
-  }
-  store_states<NH>(a, bv, r);
+  // last, where the call finds no other value in use
+  if (!ordinary) fused_general<NH, JV, OUT>(kernel_args(), c, bv, slot);
 }
 
 // ---------------------------------------------------------------------------
@@ -1121,36 +1554,37 @@ static hipError_t step_nh(const CellArgs &a, const StepDev &st, int64_t t, int b
   dim3 grid((unsigned)((a.n_cells + block - 1) / block), (unsigned)n_sets);
   const bool out = a.out.sum != nullptr;
   if (a.jarvis && out)
-    hipLaunchKernelGGL((cell_step_kernel<NH, true, true>), grid, dim3(block), 0, s, a, st, t);
+    hipLaunchKernelGGL((cell_step_kernel<NH, true, true>), grid, dim3(block), 0, s, a, StepArgs{st, t});
   else if (a.jarvis)
-    hipLaunchKernelGGL((cell_step_kernel<NH, true, false>), grid, dim3(block), 0, s, a, st, t);
+    hipLaunchKernelGGL((cell_step_kernel<NH, true, false>), grid, dim3(block), 0, s, a, StepArgs{st, t});
   else if (out)
-    hipLaunchKernelGGL((cell_step_kernel<NH, false, true>), grid, dim3(block), 0, s, a, st, t);
+    hipLaunchKernelGGL((cell_step_kernel<NH, false, true>), grid, dim3(block), 0, s, a, StepArgs{st, t});
   else
-    hipLaunchKernelGGL((cell_step_kernel<NH, false, false>), grid, dim3(block), 0, s, a, st, t);
+    hipLaunchKernelGGL((cell_step_kernel<NH, false, false>), grid, dim3(block), 0, s, a, StepArgs{st, t});
   return hipGetLastError();
 }
 
 template <int NH>
 static hipError_t fused_nh(const CellArgs &a, int64_t t0, int nsteps, int step0, int block,
                            int n_sets, hipStream_t s) {
-  // the lanes' LDS slots of a workgroup stay within 64 KB
-  while ((size_t)block * lane_slots(NH) * sizeof(double) > 65536) block /= 2;
-  const size_t shm = (size_t)block * lane_slots(NH) * sizeof(double);
-  dim3 grid((unsigned)((a.n_cells + block - 1) / block), (unsigned)n_sets);
   const bool out = a.out.sum != nullptr;
+  const size_t lane = lane_slots(NH, a.jarvis != 0, out ? a.out.n : 0) * sizeof(double);
+  // the lanes' LDS slots of a workgroup stay within 64 KB
+  while (block * lane > 65536) block /= 2;
+  const size_t shm = block * lane;
+  dim3 grid((unsigned)((a.n_cells + block - 1) / block), (unsigned)n_sets);
   if (a.jarvis && out)
-    hipLaunchKernelGGL((cell_fused_kernel<NH, true, true>), grid, dim3(block), shm, s, a, t0,
-                       nsteps, step0);
+    hipLaunchKernelGGL((cell_fused_kernel<NH, true, true>), grid, dim3(block), shm, s, a,
+                       FusedArgs{t0, nsteps, step0});
   else if (a.jarvis)
-    hipLaunchKernelGGL((cell_fused_kernel<NH, true, false>), grid, dim3(block), shm, s, a, t0,
-                       nsteps, step0);
+    hipLaunchKernelGGL((cell_fused_kernel<NH, true, false>), grid, dim3(block), shm, s, a,
+                       FusedArgs{t0, nsteps, step0});
   else if (out)
-    hipLaunchKernelGGL((cell_fused_kernel<NH, false, true>), grid, dim3(block), shm, s, a, t0,
-                       nsteps, step0);
+    hipLaunchKernelGGL((cell_fused_kernel<NH, false, true>), grid, dim3(block), shm, s, a,
+                       FusedArgs{t0, nsteps, step0});
   else
-    hipLaunchKernelGGL((cell_fused_kernel<NH, false, false>), grid, dim3(block), shm, s, a, t0,
-                       nsteps, step0);
+    hipLaunchKernelGGL((cell_fused_kernel<NH, false, false>), grid, dim3(block), shm, s, a,
+                       FusedArgs{t0, nsteps, step0});
   return hipGetLastError();
 }
 
