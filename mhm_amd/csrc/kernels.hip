@@ -1131,21 +1131,36 @@ __device__ __forceinline__ void lds_barrier() {
 // The host keeps a window's ring rows contiguous (ring length and window
 // starts are multiples of B).
 // Same per-node arithmetic as route_node (mo_mrm_routing.f90:425-472).
-constexpr int kTileAhead = 8;
+//
+// What bounds it: where a launch has many bins due, the ring's reads (1,800
+// bins x 64 steps: 236 MB in 56 us, the rate of a large copy); at the ends of
+// a run's tile pipeline and on small basins a diagonal's latency: LDS write,
+// barrier and read (146 cycles), eight dependent FP64 operations and whatever
+// else a wave issues (a lone wave issues an FP64 instruction every 8 cycles,
+// others every 4).  So a wave runs a loop with only what its slots need
+// (ROOTS, RARE below), masked instead of selected, between the first and the
+// last diagonal that one of its slots handles (slots are laid out by lag), and
+// outside those keeps the barriers only: some 32 instructions per diagonal for
+// most waves.  Against one loop for all slots, with selects and an index per
+// fetch: the average launch of 1024x1024 nodes over 1440 steps 44.4 -> 38.8 us,
+// 1,800 bins 63 -> 56 us, eleven bins (latency alone, 0.2 us a diagonal) 21.0 ->
+// 19.4 us; 8 fetches ahead instead of 4 gave the same.  Four steps per diagonal
+// (one LDS round trip for four steps) were slower where many bins are due (68
+// us: a window fills and drains over four times the steps), 17.7 us for eleven.
+constexpr int kTileAhead = 4;
 
 struct TileLane {
-  const double *p;      // series element of diagonal 0 (real) or window step 0 (proxy)
-  uint32_t stride;      // bytes between consecutive elements of the series (0: idle)
+  const double *p;      // series element of window step 0
+  uint64_t stride;      // bytes between consecutive elements of the series (0: idle)
   double *bout;         // tile root: boundary series of this window, else null
   int64_t t0;           // global step of window step 0
-  int32_t lag, nb, nc, c0;
+  int32_t lag, nb, nc, c0;  // nb: steps of this window, 0: idle
   uint32_t bv;          // byte offset of (set, node) in a row
-  int32_t a, pos, set;
+  int32_t a, set;
   int32_t gauge;        // first gauge at the node, -1: none
   int32_t orow_t, orow_g;  // LDS output rows of the tile-root series / gauge sums, -1: none
-  bool act, real, proxy;
+  bool real, proxy;
   double qtin1, qtr1, c1, c2;
-  double qlast;         // qOUT of the run's last step (when it falls in this window)
   double qacc;          // Qmod summed over the steps (ACC)
 };
 
@@ -1156,129 +1171,113 @@ struct TileOutRow {
   int32_t nb;      // steps to write
 };
 
-// One sweep over the bin's nd diagonals; NCW bounds the upstream slots summed
-// (the wave's largest upstream count rounded up to 1, 3, 5 or 8 -- a node's
-// slots past its own count read a +0.0 slot, which leaves the running sum's
-// value unchanged).  LDS: qTR parity buffers [2][W], +0.0 at 2W and 3W, so
-// that buffer 1's offsets are buffer 0's plus W for upstream and zero slots
-// alike.  STAGE: the tile-root series and gauge sums go to LDS rows (out,
-// B values each) and leave after the sweep, so that the loop holds no global
-// store: stores count in the same counter as the loads in flight, and each
-// one would shorten the wait for a fetched value.
-template <int NCW, bool STAGE, bool ACC>
-__device__ __forceinline__ void tile_sweep(const RouteArgs &r, TileLane &u, double *qtr, int nd,
-                                           double *out, int B, int out_cap) {
-  constexpr int W = kTileSlots;
+// LDS parity buffers, in doubles: a value per slot and for the zero slot W,
+// whose +0.0 stands for a node's missing upstream slots (adding it leaves the
+// running sum's value unchanged).
+constexpr int kTileBuf = kTileSlots + 1;
+
+// The diagonals [lo, hi) of the bin's nd (a multiple of kTileAhead) that a
+// wave's slots handle, lo a multiple of kTileAhead.
+struct TileSpan {
+  int lo, hi, nd;
+};
+
+// One sweep over the bin's diagonals; NCW bounds the upstream slots read
+// together.  ROOTS: a slot of the wave hands a series on (a tile root's, a
+// gauge's); RARE: a slot has more than NCW upstream slots, does not add its
+// own qOUT or is cut by an inflow gauge.  STAGE: the tile-root series and
+// gauge sums go to LDS rows (out, B + 1 values apart: the lanes of a wave
+// write different banks) and leave after the sweep, so that the loop holds no
+// global store: stores count in the same counter as the loads in flight, and
+// each one would shorten the wait for a fetched value.  Every lane then writes,
+// without a branch: a lane without a row its scratch entry after them.
+template <int NCW, bool ROOTS, bool RARE, bool STAGE, bool ACC>
+__device__ __forceinline__ void tile_sweep(const RouteArgs &r, TileLane &u, double *qtr,
+                                           TileSpan w, double *out, int out_rows, int B) {
+  constexpr int W = kTileSlots, A = kTileAhead;
   const int s = threadIdx.x;
-  uint32_t up[NCW];  // byte offsets in buffer 0
-  const uint32_t zoff = (uint32_t)(2 * W) * 8u;
+  const double *up[NCW];  // the upstream slots in buffer 0
 #pragma unroll
-  for (int c = 0; c < NCW; ++c) up[c] = c < u.nc ? (uint32_t)(u.c0 + c) * 8u : zoff;
-  const bool link = (u.a & NF_LINK) != 0, qflag = (u.a & NF_QOUT) != 0, cut = (u.a & NF_CUT) != 0;
-  const bool rare = u.bout != nullptr || u.gauge >= 0;
-  const char *qtr_b = reinterpret_cast<const char *>(qtr);
-  // Value for diagonal df: a real slot's qOUT sits in ring row df of the
-  // window (the ring is written lag rows late), the same row for every real
-  // slot of the bin; a proxy's boundary element is its window step df - lag,
-  // clamped into the window.  The address is formed from the index each time:
-  // written as a conditional advance, the compiler reuses the previous
-  // element where the clamp holds it, and each fetch then waits for the one
-  // before.
-  // (a real slot's index is df itself: no shift, no clamp below nd)
-  const int32_t fshift = u.real ? 0 : u.lag;
-  const int32_t fmax = u.real ? 0x7FFFFFFF : (u.nb > 0 ? u.nb - 1 : 0);
-  auto fetch = [&](int df) -> double {
-    const uint32_t jc = (uint32_t)min(max(df - fshift, 0), fmax);
-    return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(u.p) +
-                                             (uint64_t)jc * u.stride);
+  for (int c = 0; c < NCW; ++c) up[c] = qtr + (c < u.nc ? u.c0 + c : W);
+  const bool noq = u.real && !(u.a & NF_QOUT), cut = u.real && (u.a & NF_CUT);
+  const int scratch = out_rows * (B + 1) + s;
+  double *ot = out + (u.orow_t >= 0 ? u.orow_t * (B + 1) : scratch);
+  double *og = out + (u.orow_g >= 0 ? u.orow_g * (B + 1) : scratch);
+  const int tstep = u.orow_t >= 0 ? 1 : 0, gstep = u.orow_g >= 0 ? 1 : 0;
+  const bool gauges = ROOTS && __any(u.gauge >= 0);
+  // value for diagonal d: the slot's step d - lag, its first or last one
+  // outside its diagonals
+  const char *p = reinterpret_cast<const char *>(u.p);
+  const uint32_t moves = u.nb > 0 ? u.nb - 1 : 0;
+  double qq[A];
+  auto fetch = [&](int d, double &q) {
+    if ((uint32_t)(d - u.lag - 1) < moves) p += u.stride;
+    q = *reinterpret_cast<const double *>(p);
   };
-  // steps this slot updates (real and due), and the run's last step in the window
-  const uint32_t nupd = u.act && u.real ? (uint32_t)u.nb : 0u;
-  const int32_t jlast = (int32_t)min<int64_t>(r.t_hi - 1 - u.t0, 0x7FFFFFFF);
-  double qq[kTileAhead];
-#pragma unroll
-  for (int i = 0; i < kTileAhead; ++i) qq[i] = 0.0;
-  double musk = u.qtr1 + u.c1 * (u.qtin1 - u.qtr1);
-  // STAGE: a diagonal's outputs are written to LDS on the next diagonal, after
-  // its upstream reads are issued, not before the barrier that ends it.
-  // Every lane writes both, without a branch: a lane with nothing to keep
-  // writes its own scratch entries (after the rows).  Rows are B + 1 apart:
-  // the lanes of a wave write different banks.
-  double pq = 0.0, ps = 0.0;
-  const int scratch_t = out_cap * (B + 1) + s;
-  const int scratch_g = scratch_t + W;
-  int it = scratch_t, ig = scratch_g;
-  auto put_rows = [&]() {
-    out[it] = pq;
-    out[ig] = ps;
-  };
+  double musk = u.qtr1 + u.c1 * (u.qtin1 - u.qtr1);  // qTR(IT1) + C1 (qTIN(IT1) - qTR(IT1))
   // Diagonal d reads parity buffer (d + 1) & 1, written on diagonal d - 1 by
   // the upstream slots (one level deeper, one diagonal earlier, same step),
-  // and writes buffer d & 1.  A slot writes every diagonal: an inactive
-  // slot's value is read only by a parent that is inactive for the same step.
+  // and writes buffer d & 1 (wb).
   auto diagonal = [&](int d, int wb, double qo) {
     const int j = d - u.lag;
-    const char *rb_b = qtr_b + (wb ^ 1) * W * 8;  // the buffer written on diagonal d - 1
+    if ((uint32_t)j >= (uint32_t)u.nb) return;
     double v[NCW];
 #pragma unroll
-    for (int c = 0; c < NCW; ++c) v[c] = *reinterpret_cast<const double *>(rb_b + up[c]);
-    if (STAGE) put_rows();
-    // upstream qTR in routing rank
-    double sum = 0.0;
+    for (int c = 0; c < NCW; ++c) v[c] = up[c][(wb ^ 1) * kTileBuf];
+    // upstream qTR in routing rank, then the node's own qOUT
+    double sum = v[0];
 #pragma unroll
-    for (int c = 0; c < NCW; ++c) sum = sum + v[c];
-    if (NCW == 8 && u.nc > 8) {
-      const double *rb = qtr + (wb ^ 1) * W;
-      for (int c = 8; c < u.nc; ++c) sum = sum + rb[u.c0 + c];
+    for (int c = 1; c < NCW; ++c) sum = sum + v[c];
+    if (RARE) {
+#pragma nounroll
+      for (int c = NCW; c < u.nc; ++c) sum = sum + qtr[(wb ^ 1) * kTileBuf + u.c0 + c];
     }
-    if (qflag) sum = sum + qo;
+    sum = sum + (RARE && noq ? 0.0 : qo);
     // musk = qTR(IT1) + C1 (qTIN(IT1) - qTR(IT1)), formed on the diagonal before
     double q = musk + u.c2 * (sum - u.qtin1);
-    if (cut) q = 0.0;
-    qtr[wb * W + s] = u.proxy ? qo : q;
-    const bool upd = (uint32_t)j < nupd;
-    if (upd && link) u.qtr1 = q;
-    if (upd) u.qtin1 = sum;
+    if (RARE && cut) q = 0.0;
+    qtr[wb * kTileBuf + s] = u.proxy ? qo : q;
+    u.qtr1 = q;
+    u.qtin1 = sum;
+    musk = q + u.c1 * (sum - q);
     // Qmod of step j, added in step order
-    if (ACC && upd && u.t0 + j >= r.acc_from) u.qacc = u.qacc + sum;
-    musk = u.qtr1 + u.c1 * (u.qtin1 - u.qtr1);
-    if (upd && j == jlast) u.qlast = qo;
-    if (STAGE) {
-      it = upd && u.orow_t >= 0 ? u.orow_t * (B + 1) + j : scratch_t;
-      ig = upd && u.orow_g >= 0 ? u.orow_g * (B + 1) + j : scratch_g;
-      pq = q;
-      ps = sum;
-    } else if (upd && rare) {
-      // at most two stores, none in a loop
+    if (ACC && u.t0 + j >= r.acc_from) u.qacc = u.qacc + sum;
+    if (STAGE && ROOTS) {
+      *ot = q;
+      ot += tstep;
+      if (gauges) {
+        *og = sum;
+        og += gstep;
+      }
+    } else if (ROOTS) {
       if (u.bout) u.bout[j] = q;
       if (u.gauge >= 0)
         r.gauge_out[((u.t0 + j - r.t_base) * r.n_sets + u.set) * r.n_gauges + u.gauge] = sum;
     }
   };
-  // The first pass only fetches.  Fetches stay in diagonal order, one per
-  // diagonal, in every pass, so that a value is waited for kTileAhead - 1
-  // fetches after its own (a prologue whose loads the compiler reorders would
-  // make the loop wait for all of them).
-  for (int d0 = -kTileAhead; d0 < nd; d0 += kTileAhead) {
 #pragma unroll
-    for (int i = 0; i < kTileAhead; ++i) {
-      const int d = d0 + i;
-      if (d >= 0 && d < nd) {
-        diagonal(d, i & 1, qq[i]);
-        lds_barrier();
-      }
-      qq[i] = fetch(min(d + kTileAhead, nd - 1));
+  for (int i = 0; i < A; ++i) fetch(w.lo + i, qq[i]);
+#pragma nounroll
+  for (int d = 0; d < w.lo; ++d) lds_barrier();
+  int d0 = w.lo;
+#pragma nounroll
+  for (; d0 < w.hi; d0 += A) {
+#pragma unroll
+    for (int i = 0; i < A; ++i) {
+      // every lane waits for this diagonal's value here, whether it uses it
+      // or not: the register is free for the next fetch
+      settle(qq[i]);
+      diagonal(d0 + i, i & 1, qq[i]);
+      lds_barrier();
+      fetch(d0 + i + A, qq[i]);
     }
   }
-  if (STAGE) {
-    put_rows();
-    lds_barrier();
-  }
+#pragma nounroll
+  for (; d0 < w.nd; ++d0) lds_barrier();
 }
 
-// LDS: qTR parity buffers [2][W], +0.0 at 2W and 3W, then (STAGE) the bin's
-// output rows: g.out_rows TileOutRow, then g.out_rows x (B + 1) values and
-// 2 W scratch values.
+// LDS: the parity buffers, then (STAGE) the bin's output rows: g.out_rows
+// TileOutRow, then g.out_rows x (B + 1) values and a scratch value per slot.
 // ACC: Qmod summed per node (r.qacc).
 template <bool STAGE, bool ACC>
 __global__ __launch_bounds__(kTileSlots) void route_tile_kernel(RouteArgs r, TileArgs g,
@@ -1293,48 +1292,45 @@ __global__ __launch_bounds__(kTileSlots) void route_tile_kernel(RouteArgs r, Til
   TileLane u;
   const int32_t k = L - (g.tau_max - (m.b >> 16));
   u.a = m.a;
-  u.pos = m.pos;
   u.set = set;
   u.real = (m.a & SF_REAL) != 0;
   u.proxy = (m.a & SF_PROXY) != 0;
-  u.act = (u.real || u.proxy) && k >= 0 && k < g.nwin;
+  const bool act = (u.real || u.proxy) && k >= 0 && k < g.nwin;
   u.t0 = r.t_lo + (int64_t)k * g.B;
-  u.nb = u.act ? (int)min((int64_t)g.B, r.t_hi - u.t0) : 0;
+  u.nb = act ? (int)min((int64_t)g.B, r.t_hi - u.t0) : 0;
   u.lag = m.a & 0xFFF;
   u.nc = (m.a >> 12) & 0xF;
   u.c0 = m.b & 0xFFFF;
   const int64_t ld = (int64_t)r.n_sets * r.sstride;
   u.bv = u.real ? (uint32_t)(set * r.sstride + m.pos) * 8u : 0u;
   u.qtin1 = u.qtr1 = u.c1 = u.c2 = 0.0;
-  // series of the slot: ring rows t0 mod R + d, d < nd (t0 and R are
-  // multiples of B, and the ring has kTileHeight rows past R) or the
-  // boundary series of the proxy's tile root; idle slots re-read one valid
-  // element
+  // series of the slot: ring rows t0 mod R + lag + j (t0 and R are multiples
+  // of B, and the ring has the tiles' height in rows past R) or the boundary
+  // series of the proxy's tile root; idle slots re-read one valid element
   const int64_t bseries = ((int64_t)(k & 1) * r.n_sets + set) * g.n_bnd;
-  if (u.act && u.real) {
-    u.p = r.ring + ring_row(u.t0, 0, r.ring_len) * ld + (int64_t)set * r.sstride + m.pos;
-    u.stride = (uint32_t)(ld * 8);
+  if (act && u.real) {
+    u.p = r.ring + ring_row(u.t0, u.lag, r.ring_len) * ld + (int64_t)set * r.sstride + m.pos;
+    u.stride = (uint64_t)ld * 8u;
     u.qtin1 = ldr(r.qTIN, u.bv);
     if (m.a & NF_LINK) {
       u.qtr1 = ldr(r.pub + ((u.t0 - 1) & 1) * ld, u.bv);
       u.c1 = ldr(r.C1, u.bv);
       u.c2 = ldr(r.C2, u.bv);
     }
-  } else if (u.act) {
+  } else if (act) {
     u.p = g.bnd + (bseries + m.bnd) * g.bstride;
     u.stride = 8;
   } else {
     u.p = g.bnd;
     u.stride = 0;
   }
-  u.bout = (u.act && (m.a & SF_TROOT)) ? g.bnd + (bseries + m.bnd) * g.bstride : nullptr;
+  u.bout = (act && (m.a & SF_TROOT)) ? g.bnd + (bseries + m.bnd) * g.bstride : nullptr;
   // gauges: the node's first gauge only (the host copies it to the others)
-  u.gauge = (u.act && u.real && (m.a & NF_GAUGE)) ? g.node_gauge[m.pos] : -1;
+  u.gauge = (act && u.real && (m.a & NF_GAUGE)) ? g.node_gauge[m.pos] : -1;
   u.orow_t = u.orow_g = -1;
-  u.qlast = 0.0;
-  u.qacc = ACC && u.act && u.real ? ldr(r.qacc, u.bv) : 0.0;
+  u.qacc = ACC && act && u.real ? ldr(r.qacc, u.bv) : 0.0;
   double *qtr = lds;
-  TileOutRow *rows = reinterpret_cast<TileOutRow *>(lds + 3 * W + 1);
+  TileOutRow *rows = reinterpret_cast<TileOutRow *>(lds + 2 * kTileBuf);
   double *out = reinterpret_cast<double *>(rows + g.out_rows);
   if (STAGE) {
     // the slot's output rows (host-numbered inside the bin); an idle owner
@@ -1352,25 +1348,40 @@ __global__ __launch_bounds__(kTileSlots) void route_tile_kernel(RouteArgs r, Til
                             u.gauge >= 0 ? u.nb : 0};
     }
   }
-  if (s == 0) qtr[2 * W] = qtr[3 * W] = 0.0;
+  if (s < 2) qtr[s * kTileBuf + W] = 0.0;
   lds_barrier();
-  const int nd = bi.height + g.B - 1;
-  if (__any(u.nc > 5)) tile_sweep<8, STAGE, ACC>(r, u, qtr, nd, out, g.B, g.out_rows);
-  else if (__any(u.nc > 3)) tile_sweep<5, STAGE, ACC>(r, u, qtr, nd, out, g.B, g.out_rows);
-  else if (__any(u.nc > 1)) tile_sweep<3, STAGE, ACC>(r, u, qtr, nd, out, g.B, g.out_rows);
-  else tile_sweep<1, STAGE, ACC>(r, u, qtr, nd, out, g.B, g.out_rows);
+  TileSpan w;
+  w.nd = (bi.height + g.B - 1 + kTileAhead - 1) / kTileAhead * kTileAhead;
+  int lo = u.nb > 0 ? u.lag : 0x7FFFFFFF, hi = u.nb > 0 ? u.lag + u.nb : 0;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = min(lo, __shfl_xor(lo, o));
+    hi = max(hi, __shfl_xor(hi, o));
+  }
+  w.hi = __builtin_amdgcn_readfirstlane(hi);
+  w.lo = min(__builtin_amdgcn_readfirstlane(lo), w.hi) & ~(kTileAhead - 1);
+  const bool rare = u.nc > 5 || (u.real && (!(u.a & NF_QOUT) || (u.a & NF_CUT)));
+  if (__any(rare))
+    tile_sweep<5, true, true, STAGE, ACC>(r, u, qtr, w, out, g.out_rows, g.B);
+  else if (__any(u.bout != nullptr || u.gauge >= 0))
+    tile_sweep<5, true, false, STAGE, ACC>(r, u, qtr, w, out, g.out_rows, g.B);
+  else if (__any(u.nc > 3))
+    tile_sweep<5, false, false, STAGE, ACC>(r, u, qtr, w, out, g.out_rows, g.B);
+  else
+    tile_sweep<3, false, false, STAGE, ACC>(r, u, qtr, w, out, g.out_rows, g.B);
   if (STAGE) {
-    // the sweep ended with a barrier after the last rows: they are complete
+    // the sweep's last barrier follows its last rows
     for (int idx = s; idx < bi.out_rows * g.B; idx += W) {
       const int rr = idx / g.B, j = idx - rr * g.B;
       const TileOutRow o = rows[rr];
       if (j < o.nb) o.base[(int64_t)j * o.stride] = out[rr * (g.B + 1) + j];
     }
   }
-  if (u.act && u.real) {
+  if (act && u.real) {
     str(r.qTIN, u.bv, u.qtin1);
     if (m.a & NF_LINK) str(r.pub + ((u.t0 + u.nb - 1) & 1) * ld, u.bv, u.qtr1);
-    if (r.qOUT && r.t_hi - 1 - u.t0 < u.nb) str(r.qOUT, u.bv, u.qlast);
+    // qOUT of the run's last step, from its ring row
+    if (r.qOUT && r.t_hi - 1 - u.t0 < u.nb) str(r.qOUT, u.bv, u.p[(r.t_hi - 1 - u.t0) * ld]);
     if (ACC) str(r.qacc, u.bv, u.qacc);
   }
 }
@@ -1633,9 +1644,9 @@ hipError_t launch_route_tile(const RouteArgs &r, const TileArgs &g, int64_t bin_
       (uint64_t)r.n_sets * (uint64_t)r.sstride * 8u > 0xFFFFFFFFull)
     return hipErrorInvalidValue;
   dim3 grid((unsigned)(bin_hi - bin_lo), (unsigned)r.n_sets);
-  const size_t base = sizeof(double) * (3 * (size_t)kTileSlots + 1);
+  const size_t base = sizeof(double) * 2 * (size_t)kTileBuf;
   const size_t stage = (size_t)g.out_rows * (sizeof(TileOutRow) + sizeof(double) * (g.B + 1)) +
-                       sizeof(double) * 2 * kTileSlots;
+                       sizeof(double) * kTileSlots;
   const bool st = base + stage <= kTileStageLds;
   const size_t shm = st ? base + stage : base;
   if (st && r.qacc)
