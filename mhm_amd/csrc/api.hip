@@ -241,18 +241,10 @@ struct mhmhip_ctx {
   GraphKey gkey;
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
-  // one routed step of mhmhip_mrm_step (the coarser grid's aggregation, the
-  // inflow patch and the 1 + tile-depth tile launches) captured once and
-  // replayed every step; rebuilt when a buffer it reads or writes changes
-  struct StepKey {
-    const void *ring = nullptr, *gauge = nullptr, *inflow = nullptr, *qacc = nullptr;
-    bool operator==(const StepKey &o) const {
-      return ring == o.ring && gauge == o.gauge && inflow == o.inflow && qacc == o.qacc;
-    }
-  };
-  StepKey skey;
-  hipGraph_t step_graph = nullptr;
-  hipGraphExec_t step_exec = nullptr;
+  // one-launch routing of mhmhip_mrm_step (launch_route_step): its counters
+  // and words lie in d_bnd, which the windowed routing overwrites
+  bool flow_ready = false;        // cleared since
+  uint32_t *flow_fail = nullptr;  // pinned host word past the staging: a wait gave up
 
   // kernel timing (mhmhip_set_profiling)
   struct Pending {
@@ -450,13 +442,15 @@ extern "C" int mhmhip_create(const mhmhip_config *cfg, mhmhip_ctx **out) {
     mhmhip_destroy(x);
     return rc;
   }
-  if (hipHostMalloc((void **)&x->stage, sizeof(double) * x->sstride * mhmhip_ctx::kStageSlots,
+  if (hipHostMalloc((void **)&x->stage,
+                    sizeof(double) * (x->sstride * mhmhip_ctx::kStageSlots + 1),
                     hipHostMallocDefault) != hipSuccess) {
     g_create_error = "create: pinned staging allocation failed";
     mhmhip_destroy(x);
     return MHMHIP_ENOMEM;
   }
-  std::fill(x->stage, x->stage + x->sstride * mhmhip_ctx::kStageSlots, 0.0);
+  std::fill(x->stage, x->stage + x->sstride * mhmhip_ctx::kStageSlots + 1, 0.0);
+  x->flow_fail = reinterpret_cast<uint32_t *>(x->stage + x->sstride * mhmhip_ctx::kStageSlots);
   for (int i = 0; i < mhmhip_ctx::kStageSlots; ++i)
     if (hipEventCreateWithFlags(&x->stage_ev[i], hipEventDisableTiming) != hipSuccess) {
       g_create_error = "create: staging event creation failed";
@@ -1444,6 +1438,24 @@ int route_tiles(mhmhip_ctx *x, const RouteArgs &r, const TileArgs &g, int32_t L_
   return MHMHIP_OK;
 }
 
+// One step (t_lo = 0, a ring of one step) in one launch; qTR in its current
+// parity slot, updated there.
+int route_one_step(mhmhip_ctx *x, RouteArgs r, const TileArgs &g) {
+  r.pub = x->d_pub + x->qtr_slot * x->ld;
+  const int64_t astride = 2 * g.n_bnd * kTileWindowMax;  // a set's share of d_bnd
+  if (!x->flow_ready) {
+    CHECK_HIP(x, hipMemsetAsync(x->d_bnd, 0, sizeof(double) * x->n_bnd_dev, x->stream), "route_step");
+    x->flow_ready = true;
+  }
+  CHECK_HIP(x, timed(x, MHMHIP_K_ROUTE_TILE, 0.0, [&] {
+              return launch_route_step(r, g, (int64_t)x->lay.bins.size(),
+                                       reinterpret_cast<uint64_t *>(x->d_bnd), astride,
+                                       x->flow_fail, x->stream);
+            }),
+            "route_step");
+  return MHMHIP_OK;
+}
+
 // Under capture: an edge from what stream `from` has enqueued so far to
 // what `to` enqueues next (the event is kept until the graph is dropped).
 int capture_edge(mhmhip_ctx *x, hipStream_t from, hipStream_t to, hipEvent_t *out = nullptr) {
@@ -1481,11 +1493,6 @@ int normalize_qtr(mhmhip_ctx *x) {
 }
 
 void drop_graph(mhmhip_ctx *x) {
-  if (x->step_exec) (void)hipGraphExecDestroy(x->step_exec);
-  if (x->step_graph) (void)hipGraphDestroy(x->step_graph);
-  x->step_exec = nullptr;
-  x->step_graph = nullptr;
-  x->skey = mhmhip_ctx::StepKey();
   if (x->graph_exec) (void)hipGraphExecDestroy(x->graph_exec);
   if (x->graph) (void)hipGraphDestroy(x->graph);
   for (auto &p : x->graph_events) {
@@ -1851,6 +1858,7 @@ extern "C" int mhmhip_bind_network(mhmhip_ctx *x, const mhmhip_network *net) {
   x->gam_set.assign((size_t)x->n_sets * x->n_domains, 0);
   x->coef_restart.assign((size_t)x->n_sets * x->n_domains, 0);
   x->qsub_loops = 0;
+  x->flow_ready = false;
   x->net_bound = true;
   x->qtr_slot = 1;
   drop_graph(x);
@@ -2351,6 +2359,10 @@ extern "C" int mhmhip_mrm_step(mhmhip_ctx *x, const mhmhip_step *st, double *gau
     if (!x->d_qsub) CHECK_RC(x->dalloc(&x->d_qsub, x->ld, "alloc Qmod sub-step sums"));
     CHECK_HIP(x, hipMemsetAsync(x->d_qsub, 0, sizeof(double) * x->ld, x->stream), "mrm_step");
   }
+  // One launch, whose workgroups hand tiles on and take a ticket each (12 ns
+  // per bin and set, sets side by side), instead of one launch per tile depth
+  // (6.5 to 9 us): where there are fewer than 512 bins per launch saved.
+  const bool flow = (int64_t)x->lay.bins.size() <= 512 * ((int64_t)g.tau_max + 1);
   // this step is step 0 of a one-step ring: mhm_step wrote its qOUT to ring
   // row lag (the tiles' layout), or, on a coarser routing grid, its
   // L1_total_runoff, which L11_runoff_acc aggregates into that row here
@@ -2367,50 +2379,18 @@ extern "C" int mhmhip_mrm_step(mhmhip_ctx *x, const mhmhip_step *st, double *gau
                 "runoff_agg");
     if (x->n_inflow > 0 && it == 0)
       CHECK_HIP(x, launch_inflow_patch(r, x->d_ring, x->d_lag, 0, 1, x->stream), "inflow_patch");
-    return route_tiles(x, r, g, 0, g.nwin + g.tau_max);
-  };
-  // the ordinary step (one routing, the model step's own runoff) replays a
-  // captured graph: one launch of 1 + tile-depth tile kernels instead of as
-  // many stream launches
-  const bool replay = loops == 1 && factor <= 1.0 && !x->prof;
-  if (replay) {
+    if (flow) return route_one_step(x, r, g);
     CHECK_RC(normalize_qtr(x));
-    mhmhip_ctx::StepKey key;
-    key.ring = x->d_ring;
-    key.gauge = x->d_gauge_buf;
-    key.inflow = inflow_row;
-    key.qacc = x->qacc_on ? x->d_qacc : nullptr;
-    if (!x->step_exec || !(key == x->skey)) {
-      if (x->step_exec) (void)hipGraphExecDestroy(x->step_exec);
-      if (x->step_graph) (void)hipGraphDestroy(x->step_graph);
-      x->step_exec = nullptr;
-      x->step_graph = nullptr;
-      CHECK_HIP(x, hipStreamBeginCapture(x->stream, hipStreamCaptureModeThreadLocal), "capture");
-      x->capturing = true;
-      const int rc = enqueue(0);
-      x->capturing = false;
-      hipGraph_t gr = nullptr;
-      const hipError_t e = hipStreamEndCapture(x->stream, &gr);
-      if (rc != MHMHIP_OK) {
-        if (gr) (void)hipGraphDestroy(gr);
-        return rc;
-      }
-      CHECK_HIP(x, e, "capture");
-      x->step_graph = gr;
-      CHECK_HIP(x, hipGraphInstantiate(&x->step_exec, gr, nullptr, nullptr, 0), "instantiate");
-      x->skey = key;
-    }
-    CHECK_HIP(x, hipGraphLaunch(x->step_exec, x->stream), "graph launch");
-    credit_route(x, kind, 1);
+    x->flow_ready = false;
+    CHECK_RC(route_tiles(x, r, g, 0, g.nwin + g.tau_max));
     x->qtr_slot = 0;
-  }
+    return MHMHIP_OK;
+  };
   // loops routings of this step's qOUT (mRM_routing, mo_mrm_routing.f90:224-284):
   // the states advance each time, Qmod is their average
-  for (int32_t it = 0; it < (replay ? 0 : loops); ++it) {
-    CHECK_RC(normalize_qtr(x));
+  for (int32_t it = 0; it < loops; ++it) {
     CHECK_RC(enqueue(it));
     credit_route(x, kind, 1);
-    x->qtr_slot = 0;
     if (loops > 1 && gauge_out && ng > 0) {
       CHECK_HIP(x, sync_copy(x, gone.data(), x->d_gauge_buf, sizeof(double) * ng,
                              hipMemcpyDeviceToHost), "download gauges");
@@ -2430,6 +2410,11 @@ extern "C" int mhmhip_mrm_step(mhmhip_ctx *x, const mhmhip_step *st, double *gau
     }
   }
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "mrm_step");
+  if (*x->flow_fail) {
+    *x->flow_fail = 0;
+    x->flow_ready = false;
+    return x->fail(MHMHIP_EHIP, "mrm_step: the wait for an upstream tile gave up");
+  }
   if (gauge_out) copy_dup_gauges(x, gauge_out, 1);
   return prof_collect(x);
 }
@@ -2754,6 +2739,7 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
   }
   if (route) {
     credit_route(x, kind, nr);
+    x->flow_ready = false;
     x->qtr_slot = (int)((nr - 1) & 1);
     if (x->qacc_on) x->qacc_count += nsteps;
     x->qsub_loops = rep;

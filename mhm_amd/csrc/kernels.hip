@@ -1386,6 +1386,205 @@ __global__ __launch_bounds__(kTileSlots) void route_tile_kernel(RouteArgs r, Til
   }
 }
 
+// ---------------------------------------------------------------------------
+// One routed step in one launch (mhmhip_mrm_step): every workgroup routes one
+// bin of one set as soon as the tiles upstream of it are done, instead of one
+// launch per tile depth.
+//
+// What bounds it: the chain of levels from the deepest node to the outlet.
+// With a launch per tile depth that was 8.9 us per 32 levels (launch, loads of
+// the slots' states, 33 barriers).  Here the loads come before the wait for
+// the upstream tiles, a tile root's outflow reaches the waiting workgroup in
+// 0.6 us (measured over a chain of 512), and inside a tile a wave walks its
+// own levels without barriers (slots are laid out by lag: waves in turn, the
+// last, which holds the lowest lags, first) at 85 ns a level: an LDS write and
+// read and six to eight dependent FP64 operations.  A step of 1024x1024 nodes
+// in tiles of 32 levels, 53 deep: 473 -> 183 us; of 24x30 nodes: 27 -> 11 us.
+// Levels with only their own slots unmasked took 220 us.
+//
+// Order: a workgroup's bin is its ticket, not its block index, and tickets
+// count bins from the last (deepest) to the first.  A tile's upstream tiles
+// are in a bin of a lower ticket or in its own bin at a larger depth, which
+// the workgroup handles before: a workgroup only waits for workgroups that
+// are already running, so the waits end whatever else is on the device.  A
+// ticket costs 12 ns (one counter per set).
+//
+// Hand-over: a tile root's value as two 64-bit words, each a 32-bit half and
+// the launch's 32-bit tag, so that each word says by itself whether it is
+// this launch's; relaxed device-scope accesses suffice.  The counter holds
+// the launch number and the tickets taken; who takes the last ticket sets it
+// for the next launch.
+struct StepFlow {
+  int32_t n_bins;
+  uint64_t *area;   // per set: counter, give-up flag, then from kFlowHead the words
+  int64_t astride;  // words between the sets' areas
+  uint32_t *fail;   // host word: a wait gave up
+};
+constexpr int kFlowHead = 16;
+// polls (0.6 us each) after which a wait gives up: the kernel ends, with an error
+constexpr int kFlowPolls = 1 << 22;
+
+__device__ __forceinline__ uint64_t flow_load(const uint64_t *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void flow_store(uint64_t *p, uint64_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ void flow_put(uint64_t *w, uint32_t tag, double v) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v), t = (uint64_t)tag << 32;
+  flow_store(w, t | (b & 0xFFFFFFFFu));
+  flow_store(w + 1, t | (b >> 32));
+}
+
+__device__ __forceinline__ double flow_get(const StepFlow &f, uint64_t *area, const uint64_t *w,
+                                           uint32_t tag) {
+  uint64_t lo, hi;
+  for (int i = 0;; ++i) {
+    lo = flow_load(w);
+    hi = flow_load(w + 1);
+    if ((uint32_t)(lo >> 32) == tag && (uint32_t)(hi >> 32) == tag) break;
+    if ((i & 1023) == 1023 && (i >= kFlowPolls || flow_load(area + 1) != 0)) {
+      // another workgroup's wait gave up, or this one: all give up
+      flow_store(area + 1, 1);
+      __hip_atomic_store(f.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      break;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  return __longlong_as_double((long long)((hi << 32) | (lo & 0xFFFFFFFFu)));
+}
+
+// One slot's update in route_step_kernel.
+struct StepLane {
+  int32_t lag, nc, c0;
+  bool link, cut;
+  double qo, qtin, c2, musk;
+  double q;       // qTR of the step (a proxy's: the upstream tile root's)
+  double sum;     // qTIN of the step
+};
+
+// The levels of one wave's slots that are due, lowest lag first.  Every slot
+// is computed on every level, from what its upstream slots hold by then: once
+// those are final (after as many levels as the slot lies above the wave's
+// lowest) so is it, and computing it again gives the same value.  That leaves
+// the loop without masks or comparisons, and levels too many do no harm.
+// LDS accesses of a wave happen in order.
+template <int NCW, bool RARE>
+__device__ __forceinline__ void step_levels(StepLane &u, double *qtr, const double *const *up,
+                                            int levels) {
+  const int s = threadIdx.x;
+  auto level = [&]() {
+    double v[NCW];
+#pragma unroll
+    for (int c = 0; c < NCW; ++c) v[c] = *up[c];
+    // upstream qTR in routing rank, then the node's own qOUT
+    double sum = v[0];
+#pragma unroll
+    for (int c = 1; c < NCW; ++c) sum = sum + v[c];
+    if (RARE) {
+#pragma nounroll
+      for (int c = NCW; c < u.nc; ++c) sum = sum + qtr[u.c0 + c];
+    }
+    sum = sum + u.qo;
+    double q = u.musk + u.c2 * (sum - u.qtin);
+    if (RARE && u.cut) q = 0.0;
+    qtr[s] = q;
+    u.q = q;
+    u.sum = sum;
+    // the next level's reads stay behind this level's writes
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
+#pragma nounroll
+  for (int i = 0; i < levels; i += 2) {
+    level();
+    level();
+  }
+}
+
+// r.pub: the qTR row in use, updated in place.  r.t_lo = 0, r.t_hi = 1, a ring
+// of one step (rows by lag).
+template <bool ACC>
+__global__ __launch_bounds__(kTileSlots) void route_step_kernel(RouteArgs r, TileArgs g, StepFlow f) {
+  constexpr int W = kTileSlots;
+  __shared__ double qtr[W + 1];
+  __shared__ uint64_t ticket;
+  const int s = threadIdx.x, set = blockIdx.y;
+  uint64_t *area = f.area + (int64_t)set * f.astride;
+  if (s == 0) {
+    const uint64_t t = __hip_atomic_fetch_add(area, (uint64_t)1, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT);
+    if ((uint32_t)t == (uint32_t)f.n_bins - 1) flow_store(area, ((t >> 32) + 1) << 32);
+    ticket = t;
+    qtr[W] = 0.0;
+  }
+  lds_barrier();
+  const uint64_t t = ticket;
+  const uint32_t tag = __builtin_amdgcn_readfirstlane((uint32_t)(t >> 32) + 1);
+  const int bin = __builtin_amdgcn_readfirstlane(f.n_bins - 1 - (int32_t)(uint32_t)t);
+  const BinInfo bi = g.bin[bin];
+  const SlotMeta m = g.slot[(int64_t)bin * W + s];
+  const bool real = (m.a & SF_REAL) != 0, proxy = (m.a & SF_PROXY) != 0;
+  const int32_t tau = m.b >> 16;
+  const int64_t ld = (int64_t)r.n_sets * r.sstride;
+  const uint32_t bv = real ? (uint32_t)(set * r.sstride + m.pos) * 8u : 0u;
+  uint64_t *word = area + kFlowHead + 2 * (int64_t)(m.bnd >= 0 ? m.bnd : 0);
+  StepLane u{};
+  u.lag = m.a & 0xFFF;
+  u.nc = (m.a >> 12) & 0xF;
+  u.c0 = m.b & 0xFFFF;
+  u.link = (m.a & NF_LINK) != 0;
+  u.cut = real && (m.a & NF_CUT);
+  const bool troot = real && (m.a & SF_TROOT);
+  double qo = 0.0;
+  int32_t gauge = -1;
+  if (real) {
+    qo = ldr(r.ring + (int64_t)u.lag * ld, bv);
+    u.qtin = ldr(r.qTIN, bv);
+    if (m.a & NF_GAUGE) gauge = g.node_gauge[m.pos];
+    if (u.link) {
+      const double qtr1 = ldr(r.pub, bv), c1 = ldr(r.C1, bv);
+      u.c2 = ldr(r.C2, bv);
+      // qTR(IT1) + C1 (qTIN(IT1) - qTR(IT1))
+      u.musk = qtr1 + c1 * (u.qtin - qtr1);
+    }
+    u.qo = (m.a & NF_QOUT) ? qo : 0.0;
+  }
+  const int wave = __builtin_amdgcn_readfirstlane(s / 64);
+  // everything that needs no upstream value comes before the wait for one
+  const double *up[5];  // the upstream slots; the zero slot W for missing ones
+#pragma unroll
+  for (int c = 0; c < 5; ++c) up[c] = qtr + (c < u.nc ? u.c0 + c : W);
+  const int form = __any(u.nc > 5 || u.cut) ? 2 : __any(u.nc > 3) ? 1 : 0;
+  for (int32_t k = bi.tau_hi; k >= bi.tau_lo; --k) {
+    const bool due = real && tau == k;
+    const uint64_t mask = __ballot(due);
+    int levels = 0;  // of the wave's slots that are due
+    if (mask != 0)
+      levels = 1 + __builtin_amdgcn_readlane(u.lag, __builtin_ctzll(mask)) -
+               __builtin_amdgcn_readlane(u.lag, 63 - __builtin_clzll(mask));
+    if (proxy && tau == k) qtr[s] = flow_get(f, area, word, tag);
+#pragma nounroll
+    for (int turn = W / 64 - 1; turn >= 0; --turn) {
+      if (turn == wave && due) {
+        if (form == 2) step_levels<5, true>(u, qtr, up, levels);
+        else if (form == 1) step_levels<5, false>(u, qtr, up, levels);
+        else step_levels<3, false>(u, qtr, up, levels);
+        if (troot) flow_put(word, tag, u.q);
+      }
+      if (turn > 0) lds_barrier();
+    }
+  }
+  if (real) {
+    str(r.qTIN, bv, u.sum);
+    if (u.link) str(r.pub, bv, u.q);
+    if (r.qOUT) str(r.qOUT, bv, qo);
+    // gauges: the node's first gauge only (the host copies it to the others)
+    if (gauge >= 0) r.gauge_out[(int64_t)set * r.n_gauges + gauge] = u.sum;
+    if (ACC) str(r.qacc, bv, ldr(r.qacc, bv) + u.sum);
+  }
+}
+
 // Forcing on the meteo grid (L2) to the L1 cells of one domain, as
 // meteo_forcings_wrapper maps it (mo_meteo_helper.f90:119-143).  One thread
 // per (L1 cell, day).  Aggregation (L1 coarser, mo_meteo_spatial_tools.f90:
@@ -1661,6 +1860,23 @@ hipError_t launch_route_tile(const RouteArgs &r, const TileArgs &g, int64_t bin_
   else
     hipLaunchKernelGGL((route_tile_kernel<false, false>), grid, dim3(kTileSlots), shm, s, r, g, L,
                        (int32_t)bin_lo);
+  return hipGetLastError();
+}
+
+hipError_t launch_route_step(const RouteArgs &r, const TileArgs &g, int64_t n_bins, uint64_t *area,
+                             int64_t astride, uint32_t *fail, hipStream_t s) {
+  // one step of a one-step ring; a set's area holds the words of its boundary
+  // rows; 32-bit tickets and byte offsets
+  if (n_bins < 1 || n_bins > 0x7FFFFFFF || r.ring_len != 1 || r.t_lo != 0 || r.t_hi != 1 ||
+      r.t_base != 0 || !area || !fail || astride < kFlowHead + 2 * g.n_bnd ||
+      (uint64_t)r.n_sets * (uint64_t)r.sstride * 8u > 0xFFFFFFFFull)
+    return hipErrorInvalidValue;
+  const StepFlow f{(int32_t)n_bins, area, astride, fail};
+  dim3 grid((unsigned)n_bins, (unsigned)r.n_sets);
+  if (r.qacc)
+    hipLaunchKernelGGL(route_step_kernel<true>, grid, dim3(kTileSlots), 0, s, r, g, f);
+  else
+    hipLaunchKernelGGL(route_step_kernel<false>, grid, dim3(kTileSlots), 0, s, r, g, f);
   return hipGetLastError();
 }
 

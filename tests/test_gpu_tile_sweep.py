@@ -69,3 +69,43 @@ def test_tile_loops_match_the_wavefront(height, window, inflow):
     for a, b in zip(r1, r3):
         for k in a:
             assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("height,inflow,packed", [(2, True, 0), (16, False, 0), (16, True, 0),
+                                                  (64, True, 0), (16, False, 30), (16, False, 530)])
+def test_step_by_step_matches_the_windows(height, inflow, packed):
+    """mrm_step's one-launch routing (kernels.hip: route_step_kernel), with the
+    windowed run in between, gives the windowed run's series bit for bit: the
+    same operations per node.  packed: that many basins of a few cells more,
+    all in tiles of depth 0 (530: more bins than the one launch is used for)."""
+    print(f"case: steps, tile height {height}, inflow {inflow}, {packed} more basins", flush=True)
+    sys.stdout.flush()
+    n, got = 25, []
+    small = [synth.make_domain(2, 3, seed=60 + i) for i in range(packed)]
+    for per_step in (False, True):
+        doms = ([] if packed > 512 else [_domain()]) + small
+        kw = {"inflow": _inflow(doms[0], n)} if inflow else {}
+        model, _, steps, _ = make_pair(doms, n_sets=2, n_steps=n, seed=13, tile_height=height, **kw)
+        run = dict(mode=1, steps_per_launch=6, route_mode=3, route_window=5)
+        if per_step:
+            def walk(a, b):
+                out = []
+                for k in range(a, b):
+                    if inflow:
+                        model.set_inflow(kw["inflow"]["q"][k:k + 1])
+                    model.mhm_step(steps[k])
+                    out.append(model.mrm_step(steps[k]))
+                return out
+            g = walk(0, 9)
+            if inflow:
+                model.set_inflow(kw["inflow"]["q"][9:16])
+            g = np.concatenate([np.stack(g), model.run(steps[9:16], **run), np.stack(walk(16, n))])
+        else:
+            g = model.run(steps, **run)
+        got.append((g, [model.routing_state(s) for s in range(2)]))
+        model.close()
+    (g1, r1), (g2, r2) = got
+    assert np.array_equal(g1, g2)
+    for a, b in zip(r1, r2):
+        for k in a:
+            assert np.array_equal(a[k], b[k]), k
