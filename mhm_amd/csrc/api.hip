@@ -241,6 +241,18 @@ struct mhmhip_ctx {
   GraphKey gkey;
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
+  // device index of every reference cell / node / link in pinned host memory, for the
+  // rows that row_gather_kernel brings in the reference's order (get_row);
+  // built by the first download after the order changed
+  struct HostOrder {
+    int32_t *pos = nullptr;
+    int64_t n = 0;
+    bool stale = true;
+  };
+  HostOrder cell_order, node_order, link_order;
+  static constexpr int kRowParts = 8;
+  hipEvent_t row_ev[kRowParts] = {};  // the parts of a row under way
+
   // one-launch routing of mhmhip_mrm_step (launch_route_step): its counters
   // and words lie in d_bnd, which the windowed routing overwrites
   bool flow_ready = false;        // cleared since
@@ -508,6 +520,11 @@ extern "C" int mhmhip_destroy(mhmhip_ctx *x) {
   for (hipEvent_t e : x->stage_ev)
     if (e) (void)hipEventDestroy(e);
   if (x->stage) (void)hipHostFree(x->stage);
+  if (x->cell_order.pos) (void)hipHostFree(x->cell_order.pos);
+  if (x->node_order.pos) (void)hipHostFree(x->node_order.pos);
+  if (x->link_order.pos) (void)hipHostFree(x->link_order.pos);
+  for (hipEvent_t e : x->row_ev)
+    if (e) (void)hipEventDestroy(e);
   if (x->cstream) (void)hipStreamSynchronize(x->cstream);
   for (int i = 0; i < 2; ++i) {
     if (x->fstage_h[i]) (void)hipHostFree(x->fstage_h[i]);
@@ -550,7 +567,7 @@ namespace {
 
 // The next pinned staging row, free once its previous upload has left it.
 // Positions past `used` (the stride's padding) keep the zeros they were
-// cleared to; a download through the row clears them again.
+// cleared to (a download through the row writes no more than the cells).
 int stage_take(mhmhip_ctx *x, double **row) {
   const int i = x->stage_next;
   x->stage_next = (i + 1) % mhmhip_ctx::kStageSlots;
@@ -588,16 +605,67 @@ int put_node_row(mhmhip_ctx *x, double *dst, const double *src) {
   return stage_send(x, dst, row);
 }
 
-int get_row(mhmhip_ctx *x, const double *srcdev, double *dst) {
+// n values of a device row in the reference's order (fill writes the device
+// index of every cell, node or link) to the host: gathered on the device into a pinned staging row
+// and copied from there.  A row of 64k values or more is split, so that the
+// host copies one part while the next ones cross the link (1M cells: 340 us
+// with 8 parts, 470 with one; at 65k cells 34 and 36).
+template <typename Fn>
+int get_ordered(mhmhip_ctx *x, const double *srcdev, mhmhip_ctx::HostOrder &o, int64_t n, Fn fill,
+                double *dst) {
+  if (n < 1) return MHMHIP_OK;
+  if (o.stale || o.n != n) {
+    if (o.pos) (void)hipHostFree(o.pos);
+    o.pos = nullptr;
+    o.n = n;
+    o.stale = true;
+    if (hipHostMalloc((void **)&o.pos, sizeof(int32_t) * n, hipHostMallocDefault) != hipSuccess)
+      return x->fail(MHMHIP_ENOMEM, "download: pinned cell order allocation failed");
+    fill(o.pos);
+    o.stale = false;
+  }
   double *row = nullptr;
   CHECK_RC(stage_take(x, &row));
-  CHECK_HIP(x, hipMemcpyAsync(row, srcdev, sizeof(double) * x->sstride, hipMemcpyDeviceToHost,
-                              x->stream),
-            "download");
-  CHECK_HIP(x, hipStreamSynchronize(x->stream), "download");
-  for (int64_t c = 0; c < x->n_cells; ++c) dst[c] = row[x->pos[c]];
-  std::fill(row + x->n_cells, row + x->sstride, 0.0);  // the padding a cell row leaves
+  const int parts = (int)std::max<int64_t>(1, std::min<int64_t>(n / 65536, mhmhip_ctx::kRowParts));
+  const int64_t len = (n + parts - 1) / parts;
+  for (int i = 0; i < parts; ++i) {
+    CHECK_HIP(x, launch_row_gather(srcdev, o.pos, row, i * len, std::min(n, (i + 1) * len),
+                                   x->stream),
+              "download");
+    if (!x->row_ev[i])
+      CHECK_HIP(x, hipEventCreateWithFlags(&x->row_ev[i], hipEventDisableTiming), "download");
+    if (i < parts - 1) CHECK_HIP(x, hipEventRecord(x->row_ev[i], x->stream), "download");
+  }
+  for (int i = 0; i < parts; ++i) {
+    if (i < parts - 1)
+      CHECK_HIP(x, hipEventSynchronize(x->row_ev[i]), "download");
+    else
+      CHECK_HIP(x, hipStreamSynchronize(x->stream), "download");
+    std::memcpy(dst + i * len, row + i * len,
+                sizeof(double) * (std::min(n, (i + 1) * len) - i * len));
+  }
   return MHMHIP_OK;
+}
+
+int get_row(mhmhip_ctx *x, const double *srcdev, double *dst) {
+  return get_ordered(x, srcdev, x->cell_order, x->n_cells, [x](int32_t *p) {
+    for (int64_t c = 0; c < x->n_cells; ++c) p[c] = (int32_t)x->pos[c];
+  }, dst);
+}
+
+// one row of node values -> reference node order
+int get_node_row(mhmhip_ctx *x, const double *srcdev, double *dst) {
+  return get_ordered(x, srcdev, x->node_order, x->n_nodes, [x](int32_t *p) {
+    for (int64_t k = 0; k < x->n_nodes; ++k) p[k] = (int32_t)x->npos[k];
+  }, dst);
+}
+
+// one row of link values (at their source nodes) -> the links' order
+int get_link_row(mhmhip_ctx *x, const double *srcdev, double *dst) {
+  return get_ordered(x, srcdev, x->link_order, x->lay.n_links_total, [x](int32_t *p) {
+    for (int64_t q = 0; q < x->n_nodes; ++q)
+      if (x->lay.link_of_node[q] >= 0) p[x->lay.link_of_node[q]] = (int32_t)q;
+  }, dst);
 }
 
 int var_cols(const mhmhip_ctx *x, int var) {
@@ -1685,6 +1753,7 @@ extern "C" int mhmhip_bind_network(mhmhip_ctx *x, const mhmhip_network *net) {
   }
   x->pos = cpos;
   x->d_pos_stale = true;
+  x->cell_order.stale = true;
   if (moved) x->mpr_stale = true;
   const int64_t old_nodes = x->n_nodes;
 
@@ -1742,6 +1811,7 @@ extern "C" int mhmhip_bind_network(mhmhip_ctx *x, const mhmhip_network *net) {
   const int64_t nn = net->n_nodes;
   x->n_nodes = nn;
   x->npos = lay.pos;
+  x->node_order.stale = x->link_order.stale = true;
   x->dom_node_start = ds;
   x->coarse = coarse;
   CHECK_RC(x->dalloc(&x->d_meta, nn, "alloc meta"));
@@ -2128,19 +2198,11 @@ extern "C" int mhmhip_get_routing_state(mhmhip_ctx *x, int32_t set, double *qOUT
   CHECK_HIP(x, hipSetDevice(x->cfg.device), "get_routing_state");
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "get_routing_state");
   const int64_t off = (int64_t)set * x->sstride;
-  std::vector<double> buf(x->sstride);
-  auto node_out = [&](const double *dev, double *dst) -> int {
-    if (!dst) return MHMHIP_OK;
-    CHECK_HIP(x, sync_copy(x, buf.data(), dev, sizeof(double) * x->sstride, hipMemcpyDeviceToHost), "download");
-    for (int64_t k = 0; k < x->n_nodes; ++k) dst[k] = buf[x->npos[k]];
-    return MHMHIP_OK;
+  auto node_out = [&](const double *dev, double *dst) {
+    return dst ? get_node_row(x, dev, dst) : MHMHIP_OK;
   };
-  auto link_out = [&](const double *dev, double *dst) -> int {
-    if (!dst) return MHMHIP_OK;
-    CHECK_HIP(x, sync_copy(x, buf.data(), dev, sizeof(double) * x->sstride, hipMemcpyDeviceToHost), "download");
-    for (int64_t q = 0; q < x->n_nodes; ++q)
-      if (x->lay.link_of_node[q] >= 0) dst[x->lay.link_of_node[q]] = buf[q];
-    return MHMHIP_OK;
+  auto link_out = [&](const double *dev, double *dst) {
+    return dst ? get_link_row(x, dev, dst) : MHMHIP_OK;
   };
   CHECK_RC(node_out(x->d_qOUT + off, qOUT));
   CHECK_RC(node_out(x->d_qTIN + off, qTIN));
@@ -2180,13 +2242,7 @@ extern "C" int mhmhip_get_qmod_sum(mhmhip_ctx *x, int32_t set, double *sum, int6
   if (set < 0 || set >= x->n_sets) return x->fail(MHMHIP_EINVAL, "get_qmod_sum: bad set");
   CHECK_HIP(x, hipSetDevice(x->cfg.device), "get_qmod_sum");
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "get_qmod_sum");
-  if (sum) {
-    std::vector<double> buf(x->sstride);
-    CHECK_HIP(x, sync_copy(x, buf.data(), x->d_qacc + (int64_t)set * x->sstride,
-                           sizeof(double) * x->sstride, hipMemcpyDeviceToHost),
-              "download");
-    for (int64_t k = 0; k < x->n_nodes; ++k) sum[k] = buf[x->npos[k]];
-  }
+  if (sum) CHECK_RC(get_node_row(x, x->d_qacc + (int64_t)set * x->sstride, sum));
   if (count) *count = x->qacc_count;
   return MHMHIP_OK;
 }

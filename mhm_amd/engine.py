@@ -101,7 +101,7 @@ class Model:
     def get(self, name, set_=0):
         var = N.S[name] if name in N.S else N.X[name]
         ncols = self.n_horizons if name in N.HORIZON_VARS else 1
-        out = np.zeros((ncols, self.n_cells))
+        out = np.empty((ncols, self.n_cells))
         self._chk(N.lib().mhmhip_get_cell_var(self._ctx, var, set_, N.dptr(out), self.n_cells,
                                               ncols))
         return out[0] if ncols == 1 else out.T.copy()
@@ -267,7 +267,7 @@ class Model:
     def routing_state(self, set_=0):
         n = self.n_nodes
         nl = self._net_arrays["netPerm"].shape[0]
-        out = {k: np.zeros(n) for k in ("qOUT", "qTIN", "qTR", "Qmod")}
+        out = {k: np.empty(n) for k in ("qOUT", "qTIN", "qTR", "Qmod")}
         out["C1"] = np.zeros(max(nl, 1))
         out["C2"] = np.zeros(max(nl, 1))
         self._chk(N.lib().mhmhip_get_routing_state(self._ctx, set_, *[N.dptr(out[k]) for k in
@@ -289,7 +289,7 @@ class Model:
 
     def qmod_sum(self, set_=0):
         """(per-node Qmod sum in reference node order, steps added)."""
-        out = np.zeros(self.n_nodes)
+        out = np.empty(self.n_nodes)
         cnt = C.c_int64()
         self._chk(N.lib().mhmhip_get_qmod_sum(self._ctx, set_, N.dptr(out), C.byref(cnt)))
         return out, cnt.value
@@ -308,7 +308,7 @@ class Model:
 
     def output_sum(self, k, horizon=1, set_=0):
         """(per-cell sum of output k in reference cell order, steps added)."""
-        out = np.zeros(self.n_cells)
+        out = np.empty(self.n_cells)
         cnt = C.c_int64()
         self._chk(N.lib().mhmhip_get_output_sum(self._ctx, int(k), int(horizon), set_,
                                                 N.dptr(out), C.byref(cnt)))
