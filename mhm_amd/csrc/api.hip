@@ -797,31 +797,20 @@ extern "C" int mhmhip_default_states(mhmhip_ctx *x, const double *hd) {
   if (!hd && x->nh > 1) return x->fail(MHMHIP_EINVAL, "default_states: horizon depths required");
   x->s_dirty = x->x_dirty = true;
   CHECK_HIP(x, hipSetDevice(x->cfg.device), "default_states");
-  std::vector<double> v(x->n_cells);
-  auto fill = [&](double val) { std::fill(v.begin(), v.end(), val); };
-  auto id = [](double a) { return a; };
-  for (int s = 0; s < x->n_sets; ++s) {
-    const int64_t off = (int64_t)s * x->sstride;
-    // mo_init_states.f90:273-287 with mo_mpr_constants P1..P5, C1_InitStateSM
-    fill(0.0);
-    CHECK_RC(put_row(x, x->S + SR_INTER * x->ld + off, v.data(), id));
-    CHECK_RC(put_row(x, x->S + SR_SEAL * x->ld + off, v.data(), id));
-    fill(15.0);
-    CHECK_RC(put_row(x, x->S + SR_SNOW * x->ld + off, v.data(), id));
-    fill(10.0);
-    CHECK_RC(put_row(x, x->S + SR_UNSAT * x->ld + off, v.data(), id));
-    fill(75.0);
-    CHECK_RC(put_row(x, x->S + SR_SAT * x->ld + off, v.data(), id));
-    for (int h = 0; h < x->nh - 1; ++h) {
-      fill((h == 0 ? hd[0] : hd[h] - hd[h - 1]) * 0.25);
-      CHECK_RC(put_row(x, x->S + (SR_NSCALAR + h) * x->ld + off, v.data(), id));
-    }
-    fill((1500.0 - (x->nh >= 2 ? hd[x->nh - 2] : 0.0)) * 0.25);
-    CHECK_RC(put_row(x, x->S + (SR_NSCALAR + x->nh - 1) * x->ld + off, v.data(), id));
-    fill(0.0);
-    for (int r = 0; r < x->n_xrows; ++r)
-      CHECK_RC(put_row(x, x->X + r * x->ld + off, v.data(), id));
-  }
+  // mo_init_states.f90:273-287 with mo_mpr_constants P1..P5, C1_InitStateSM
+  StateValues v{};
+  v.row[SR_INTER] = v.row[SR_SEAL] = 0.0;
+  v.row[SR_SNOW] = 15.0;
+  v.row[SR_UNSAT] = 10.0;
+  v.row[SR_SAT] = 75.0;
+  for (int h = 0; h < x->nh - 1; ++h)
+    v.row[SR_NSCALAR + h] = (h == 0 ? hd[0] : hd[h] - hd[h - 1]) * 0.25;
+  v.row[SR_NSCALAR + x->nh - 1] = (1500.0 - (x->nh >= 2 ? hd[x->nh - 2] : 0.0)) * 0.25;
+  CHECK_HIP(x, launch_state_rows(x->S, v, sr_count(x->nh), x->n_cells, x->sstride, x->ld,
+                                 x->n_sets, x->stream),
+            "default_states");
+  CHECK_HIP(x, hipMemsetAsync(x->X, 0, sizeof(double) * x->n_xrows * x->ld, x->stream),
+            "default_states");
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "default_states");
   return MHMHIP_OK;
 }

@@ -48,6 +48,10 @@ __host__ __device__ constexpr int pr_count(int nh) { return PR_NSCALAR + 5 * nh 
 
 enum SRow { SR_INTER = 0, SR_SNOW, SR_SEAL, SR_UNSAT, SR_SAT, SR_NSCALAR };
 __host__ __device__ constexpr int sr_count(int nh) { return SR_NSCALAR + nh; }
+// a value for every state row
+struct StateValues {
+  double row[SR_NSCALAR + MHMHIP_MAX_HORIZONS];
+};
 
 enum XRow {
   XR_PET = 0, XR_TEMP, XR_PREC, XR_THROUGHFALL, XR_AETCAN, XR_DEGDAY, XR_MELT, XR_PEFF,

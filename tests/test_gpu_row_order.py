@@ -48,3 +48,31 @@ def test_rows_come_back_in_order(nrows, ncols, refine):
         assert np.array_equal(got["C1"], c1) and np.array_equal(got["C2"], c2)
     assert np.array_equal(model.get("SNOWPACK", 1), snow[-1])
     model.close()
+
+
+@pytest.mark.parametrize("nrows,ncols,n_sets,nh", [(1, 1, 1, 1), (5, 13, 3, 2), (16, 16, 1, 3),
+                                                   (17, 19, 70, 5)])
+def test_default_states_fill_every_set(nrows, ncols, n_sets, nh):
+    """mo_init_states.f90:273-287: the same value for every cell of every set,
+    zero fluxes, whatever was there before."""
+    print(f"case: default states {nrows}x{ncols}, {n_sets} sets, {nh} horizons", flush=True)
+    sys.stdout.flush()
+    dom = synth.make_domain(nrows, ncols, seed=84)
+    dom.horizon_depth = np.linspace(100.0, 100.0 * nh, nh)
+    model = engine.Model([dom], n_sets=n_sets, n_forcing_days=1, route=False)
+    n = model.n_cells
+    for s in (0, n_sets - 1):
+        for k in ("INTER", "SNOWPACK", "SEALSTW", "UNSATSTW", "SATSTW"):
+            model.set_var(k, np.full(n, -3.0), s)
+        model.set_var("SOILMOIST", np.full((n, nh), -3.0), s)
+    model.default_states()
+    hd = dom.horizon_depth
+    edge = np.concatenate([[0.0], hd[:-1], [1500.0]])
+    want = {"INTER": 0.0, "SNOWPACK": 15.0, "SEALSTW": 0.0, "UNSATSTW": 10.0, "SATSTW": 75.0,
+            "TOTAL_RUNOFF": 0.0}
+    for s in (0, n_sets // 2, n_sets - 1):
+        for k, v in want.items():
+            assert np.array_equal(model.get(k, s), np.full(n, v)), (k, s)
+        soil = model.get("SOILMOIST", s).reshape(n, nh)
+        assert np.array_equal(soil, np.tile((edge[1:] - edge[:-1]) * 0.25, (n, 1))), s
+    model.close()
