@@ -191,7 +191,7 @@ struct mhmhip_ctx {
   int32_t *d_gauge_node = nullptr, *d_inflow_node = nullptr, *d_inflow_hw = nullptr;
   int32_t *d_node_gauge = nullptr;  // [n_cells] first gauge at the node, -1: none
   uint8_t *d_lag = nullptr;         // [n_cells] ring lag of each node (its tile slot's lag)
-  int32_t *d_slot_out = nullptr;    // [n_slots] LDS output rows of the tiled kernel
+  int32_t *d_spare = nullptr;       // [n_slots] tile roots, proxies: the root's first upstream node
   // L1 output sums (mhmhip_output_accumulate)
   double *d_out = nullptr;
   int64_t out_rows_cap = 0;
@@ -201,7 +201,7 @@ struct mhmhip_ctx {
   double *d_qacc = nullptr;         // [ld] Qmod summed over routed steps (output aggregation)
   bool qacc_on = false;
   int64_t qacc_count = 0;
-  int32_t tile_out_rows = 0;        // most output rows of a bin
+  int32_t most_proxies = 0, most_outputs = 0;  // tile roots and gauges; of any bin
   std::vector<std::pair<int32_t, int32_t>> gauge_dup;  // (gauge, earlier gauge at its node)
   std::vector<int32_t> h_inflow_node_dev, h_inflow_hw;
   double *d_inflow_q = nullptr;
@@ -253,9 +253,9 @@ struct mhmhip_ctx {
   static constexpr int kRowParts = 8;
   hipEvent_t row_ev[kRowParts] = {};  // the parts of a row under way
 
-  // one-launch routing of mhmhip_mrm_step (launch_route_step): its counters
-  // and words lie in d_bnd, which the windowed routing overwrites
-  bool flow_ready = false;        // cleared since
+  // the routing launches' counters and a step's boundary words lie in d_bnd
+  // (cleared before they are used after the windowed routing, which writes it)
+  bool flow_ready = false;
   uint32_t *flow_fail = nullptr;  // pinned host word past the staging: a wait gave up
 
   // kernel timing (mhmhip_set_profiling)
@@ -505,7 +505,7 @@ extern "C" int mhmhip_destroy(mhmhip_ctx *x) {
   (void)hipFree(x->d_gauge_node);
   (void)hipFree(x->d_node_gauge);
   (void)hipFree(x->d_lag);
-  (void)hipFree(x->d_slot_out);
+  (void)hipFree(x->d_spare);
   (void)hipFree(x->d_qacc);
   (void)hipFree(x->d_out);
   (void)hipFree(x->d_qsub);
@@ -1349,20 +1349,80 @@ int64_t ring_need(const mhmhip_ctx *x, int kind, int S, int32_t B, int64_t nstep
   return std::min((int64_t)S + x->lay.dmax + 2, nsteps);
 }
 
-TileArgs tile_args(const mhmhip_ctx *x, int32_t B, int64_t nsteps) {
+TileArgs tile_args(const mhmhip_ctx *x) {
   TileArgs g{};
   g.slot = x->d_slots;
   g.bin = x->d_bins;
   g.node_gauge = x->d_node_gauge;
-  g.slot_out = x->d_slot_out;
-  g.out_rows = x->tile_out_rows;
-  g.bnd = x->d_bnd;
+  g.spare = x->d_spare;
   g.n_bnd = std::max<int64_t>(1, x->lay.n_bnd);
-  g.tau_max = x->lay.tau_max;
-  g.B = B;
-  g.nwin = (int32_t)((nsteps + B - 1) / B);
-  g.bstride = kTileWindowMax;
   return g;
+}
+
+FlowArgs flow_args(const mhmhip_ctx *x) {
+  FlowArgs f{};
+  f.area = reinterpret_cast<uint64_t *>(x->d_bnd);
+  f.astride = 2 * std::max<int64_t>(1, x->lay.n_bnd) * kTileWindowMax;  // a set's share of d_bnd
+  f.fail = x->flow_fail;
+  f.lag = x->d_lag;
+  f.n_bins = (int32_t)x->lay.bins.size();
+  f.tickets = x->lay.tau_max > 0;
+  f.proxy_waves = (x->most_proxies + 63) / 64;
+  f.out_waves = (x->most_outputs + 63) / 64;
+  return f;
+}
+
+WindowArgs window_args(const mhmhip_ctx *x, int32_t B, int64_t nsteps) {
+  WindowArgs v{};
+  v.bnd = x->d_bnd;
+  v.tau_max = x->lay.tau_max;
+  v.B = B;
+  v.nwin = (int32_t)((nsteps + B - 1) / B);
+  v.bstride = kTileWindowMax;
+  v.out_rows = x->most_outputs;
+  return v;
+}
+
+// Before launches that hand tiles on (not under capture).
+int flow_begin(mhmhip_ctx *x, const char *who) {
+  if (x->flow_ready) return MHMHIP_OK;
+  CHECK_HIP(x, hipMemsetAsync(x->d_bnd, 0, sizeof(double) * x->n_bnd_dev, x->stream), who);
+  x->flow_ready = true;
+  return MHMHIP_OK;
+}
+
+// After a join: did a wait of a routing launch give up?
+int flow_check(mhmhip_ctx *x, const char *who) {
+  if (!*x->flow_fail) return MHMHIP_OK;
+  *x->flow_fail = 0;
+  x->flow_ready = false;
+  return x->fail(MHMHIP_EHIP, std::string(who) + ": the wait for an upstream tile gave up");
+}
+
+// Does the tiled routing of nr steps through a ring of ring_rows pay in one
+// launch (route_stream_kernel) rather than in windows of B steps
+// (route_tile_kernel)?  In us:
+//   one launch: the chain of steps and levels at 0.2 a diagonal, a level of a
+//     tile boundary costing five more, once per filling of the ring; with the
+//     chip full 0.73e-3 per workgroup and diagonal (handing a step on costs
+//     whole memory transactions for two 8-byte words);
+//   windows: (windows + tile depth) launches, each a window that fills and
+//     drains over the tile's height at 0.2 a diagonal, 8 at least; with the
+//     chip full 0.39e-3 per workgroup and diagonal besides those 8.
+// Measured, workgroups and steps: one launch / windows [us]: 59 x 480 (B 32)
+// 139 / 294, 296 x 720 (8) 579 / 979, 152 x 960 (8) 936 / 1504, 20 x 8760 (64)
+// 2034 / 2636, 1474 x 720 (64) 840 / 955, 2833 x 48 (8) 509 / 781, 4693 x 1440 (64) 4912 / 4305, 5120 x 1095
+// (64) 6365 / 3211.
+bool one_launch_pays(const mhmhip_ctx *x, int32_t B, int64_t nr, int64_t ring_rows) {
+  const double groups = (double)x->lay.bins.size() * x->n_sets, H = x->tile_h;
+  const double fills = std::ceil((double)nr / (double)std::max<int64_t>(1, ring_rows));
+  const double nwin = std::ceil((double)nr / (double)B), steps = (double)nr;
+  const double one = std::max(0.2 * (steps + fills * (x->lay.dmax + 5.0 * x->lay.tau_max)),
+                              0.73e-3 * groups * (steps + fills * H));
+  const double launches = nwin + x->lay.tau_max;
+  const double win = std::max(launches * std::max(8.0, 3.0 + 0.2 * (B + H)),
+                              launches * 8.0 + 0.39e-3 * groups * nwin * (B + H));
+  return one <= win;
 }
 
 hipError_t ev_get(mhmhip_ctx *x, hipEvent_t *e) {
@@ -1479,36 +1539,44 @@ int route_diagonals(mhmhip_ctx *x, const RouteArgs &r, int64_t d_lo, int64_t d_h
 // Tiled routing launches [L_lo, L_hi) of a call.
 // Launch L handles window k = L - (tau_max - tau) of each tile: only the bins
 // holding tiles of depth tau_max - L .. tau_max - L + nwin - 1 are launched.
-int route_tiles(mhmhip_ctx *x, const RouteArgs &r, const TileArgs &g, int32_t L_lo, int32_t L_hi,
-                hipStream_t s = nullptr) {
-  if (!s) s = x->stream;
+int route_tiles(mhmhip_ctx *x, const RouteArgs &r, const TileArgs &g, const WindowArgs &v,
+                int32_t L_lo, int32_t L_hi, hipStream_t s) {
   const int64_t nb = (int64_t)x->lay.bins.size();
   for (int32_t L = L_lo; L < L_hi; ++L) {
     int64_t lo, hi;
-    tile_bin_range(x->lay, g.tau_max - L, g.tau_max - L + g.nwin - 1, lo, hi);
+    tile_bin_range(x->lay, v.tau_max - L, v.tau_max - L + v.nwin - 1, lo, hi);
     if (hi <= lo) continue;
     CHECK_HIP(x, timed(x, MHMHIP_K_ROUTE_TILE, 0.0, [&] {
-                return launch_route_tile(r, g, lo, hi, nb, L, s);
+                return launch_route_tile(r, g, v, lo, hi, nb, L, s);
               }, s),
               "route_tile");
   }
   return MHMHIP_OK;
 }
 
-// One step (t_lo = 0, a ring of one step) in one launch; qTR in its current
-// parity slot, updated there.
-int route_one_step(mhmhip_ctx *x, RouteArgs r, const TileArgs &g) {
-  r.pub = x->d_pub + x->qtr_slot * x->ld;
-  const int64_t astride = 2 * g.n_bnd * kTileWindowMax;  // a set's share of d_bnd
-  if (!x->flow_ready) {
-    CHECK_HIP(x, hipMemsetAsync(x->d_bnd, 0, sizeof(double) * x->n_bnd_dev, x->stream), "route_step");
-    x->flow_ready = true;
+// The steps [t_lo, t_hi) of the ring, a launch for each stretch of rows that
+// does not wrap; run_end: the last step of the run.
+int route_steps(mhmhip_ctx *x, RouteArgs r, const TileArgs &g, int64_t t_lo, int64_t t_hi,
+                int64_t run_end, hipStream_t s) {
+  FlowArgs f = flow_args(x);
+  while (t_lo < t_hi) {
+    r.t_lo = t_lo;
+    r.t_hi = t_lo = std::min(t_hi, t_lo + r.ring_len - t_lo % r.ring_len);
+    f.last = r.t_hi == run_end;
+    CHECK_HIP(x, timed(x, MHMHIP_K_ROUTE_TILE, 0.0, [&] { return launch_route_stream(r, g, f, s); }, s),
+              "route_stream");
   }
-  CHECK_HIP(x, timed(x, MHMHIP_K_ROUTE_TILE, 0.0, [&] {
-              return launch_route_step(r, g, (int64_t)x->lay.bins.size(),
-                                       reinterpret_cast<uint64_t *>(x->d_bnd), astride,
-                                       x->flow_fail, x->stream);
-            }),
+  return MHMHIP_OK;
+}
+
+// One step (t_lo = 0, a ring of one step); qTR in its current parity slot,
+// updated there.
+int route_one_step(mhmhip_ctx *x, RouteArgs r, const TileArgs &g) {
+  CHECK_RC(flow_begin(x, "route_step"));
+  r.pub = x->d_pub + x->qtr_slot * x->ld;
+  const FlowArgs f = flow_args(x);
+  CHECK_HIP(x, timed(x, MHMHIP_K_ROUTE_TILE, 0.0,
+                     [&] { return launch_route_step(r, g, f, x->stream); }),
             "route_step");
   return MHMHIP_OK;
 }
@@ -1781,7 +1849,7 @@ extern "C" int mhmhip_bind_network(mhmhip_ctx *x, const mhmhip_network *net) {
   x->dfree(x->d_dom_dmax, x->n_domains);
   x->dfree(x->d_child_list, x->n_child_dev);
   x->dfree(x->d_slots, x->n_slots_dev);
-  x->dfree(x->d_slot_out, x->n_slots_dev);
+  x->dfree(x->d_spare, x->n_slots_dev);
   x->dfree(x->d_bins, x->n_bins_dev);
   x->dfree(x->d_bnd, x->n_bnd_dev);
   x->n_child_dev = x->n_slots_dev = x->n_bins_dev = x->n_bnd_dev = 0;
@@ -1821,33 +1889,41 @@ extern "C" int mhmhip_bind_network(mhmhip_ctx *x, const mhmhip_network *net) {
   // the slot flags carry the node flags (gauges, inflow, cut links set above)
   for (SlotMeta &m : lay.slots)
     if (m.a & SF_REAL) m.a |= lay.packed[m.pos] & NF_MASK;
-  // output rows of the tiled kernel, per bin: its tile roots, then its gauge
-  // nodes (the kernel stages their series in LDS)
-  std::vector<int32_t> slot_out(lay.slots.size(), -1);  // both fields 0xFFFF
-  int32_t out_rows = 0;
-  for (size_t b = 0; b < lay.bins.size(); ++b) {
-    int32_t n = 0;
-    for (int i = 0; i < kTileSlots; ++i)
-      if (lay.slots[b * kTileSlots + i].a & SF_TROOT)
-        slot_out[b * kTileSlots + i] = (int32_t)(0xFFFF0000u | (uint32_t)n++);
-    for (int i = 0; i < kTileSlots; ++i) {
-      const int32_t a = lay.slots[b * kTileSlots + i].a;
-      if ((a & SF_REAL) && (a & NF_GAUGE)) {
-        int32_t &v = slot_out[b * kTileSlots + i];
-        v = (int32_t)(((uint32_t)v & 0xFFFFu) | ((uint32_t)n++ << 16));
-      }
-    }
-    lay.bins[b].out_rows = n;
-    out_rows = std::max(out_rows, n);
+  // a tile root hands its steps on in its own ring entries and those of its
+  // first upstream node (a tile that drains into another has two levels); its
+  // proxy finds both by its slot
+  std::vector<int32_t> spare(lay.slots.size(), -1);
+  std::vector<int32_t> root(lay.n_bnd, -1);
+  for (size_t i = 0; i < lay.slots.size(); ++i) {
+    const SlotMeta &m = lay.slots[i];
+    if (!(m.a & SF_TROOT)) continue;
+    if (nm_nchild(lay.packed[m.pos]) < 1) return x->fail(MHMHIP_EINVAL, "bind_network: tile partition failed");
+    spare[i] = lay.child_list[lay.child[m.pos]];
+    root[m.bnd] = m.pos;
   }
+  int32_t most_proxies = 0, most_outputs = 0;
+  for (size_t b = 0; b < lay.bins.size(); ++b) {
+    int32_t proxies = 0, outputs = 0;
+    for (size_t i = b * kTileSlots; i < (b + 1) * kTileSlots; ++i) {
+      SlotMeta &m = lay.slots[i];
+      outputs += ((m.a & SF_TROOT) != 0) + ((m.a & SF_REAL) && (m.a & NF_GAUGE));
+      if (!(m.a & SF_PROXY)) continue;
+      ++proxies;
+      m.pos = root[m.bnd];
+      spare[i] = lay.child_list[lay.child[m.pos]];
+    }
+    most_proxies = std::max(most_proxies, proxies);
+    most_outputs = std::max(most_outputs, outputs);
+  }
+  x->most_proxies = most_proxies;
+  x->most_outputs = most_outputs;
   const int64_t n_child = std::max<int64_t>(1, (int64_t)lay.child_list.size());
   const int64_t n_bnd = 2 * (int64_t)x->n_sets * std::max<int64_t>(1, lay.n_bnd) * kTileWindowMax;
   CHECK_RC(x->dalloc(&x->d_child_list, n_child, "alloc child list"));
   x->n_child_dev = n_child;
   CHECK_RC(x->dalloc(&x->d_slots, (int64_t)lay.slots.size(), "alloc tiles"));
-  CHECK_RC(x->dalloc(&x->d_slot_out, (int64_t)lay.slots.size(), "alloc tiles"));
+  CHECK_RC(x->dalloc(&x->d_spare, (int64_t)lay.slots.size(), "alloc tiles"));
   x->n_slots_dev = (int64_t)lay.slots.size();
-  x->tile_out_rows = out_rows;
   CHECK_RC(x->dalloc(&x->d_bins, (int64_t)lay.bins.size(), "alloc tiles"));
   x->n_bins_dev = (int64_t)lay.bins.size();
   CHECK_RC(x->dalloc(&x->d_bnd, n_bnd, "alloc tile boundaries"));
@@ -1856,7 +1932,7 @@ extern "C" int mhmhip_bind_network(mhmhip_ctx *x, const mhmhip_network *net) {
     CHECK_HIP(x, sync_copy(x, x->d_child_list, lay.child_list.data(),
                            sizeof(int32_t) * lay.child_list.size(), hipMemcpyHostToDevice),
               "upload child list");
-  CHECK_HIP(x, sync_copy(x, x->d_slot_out, slot_out.data(), sizeof(int32_t) * slot_out.size(),
+  CHECK_HIP(x, sync_copy(x, x->d_spare, spare.data(), sizeof(int32_t) * spare.size(),
                          hipMemcpyHostToDevice),
             "upload tiles");
   CHECK_HIP(x, sync_copy(x, x->d_slots, lay.slots.data(), sizeof(SlotMeta) * lay.slots.size(),
@@ -2397,17 +2473,13 @@ extern "C" int mhmhip_mrm_step(mhmhip_ctx *x, const mhmhip_step *st, double *gau
     }
   }
   const int kind = MHMHIP_K_ROUTE_TILE;
-  const TileArgs g = tile_args(x, 1, 1);
+  const TileArgs g = tile_args(x);
   const int64_t ng = (int64_t)x->n_sets * x->n_gauges;
   std::vector<double> gsum(loops > 1 ? ng : 0, 0.0), gone(loops > 1 ? ng : 0);
   if (loops > 1) {
     if (!x->d_qsub) CHECK_RC(x->dalloc(&x->d_qsub, x->ld, "alloc Qmod sub-step sums"));
     CHECK_HIP(x, hipMemsetAsync(x->d_qsub, 0, sizeof(double) * x->ld, x->stream), "mrm_step");
   }
-  // One launch, whose workgroups hand tiles on and take a ticket each (12 ns
-  // per bin and set, sets side by side), instead of one launch per tile depth
-  // (6.5 to 9 us): where there are fewer than 512 bins per launch saved.
-  const bool flow = (int64_t)x->lay.bins.size() <= 512 * ((int64_t)g.tau_max + 1);
   // this step is step 0 of a one-step ring: mhm_step wrote its qOUT to ring
   // row lag (the tiles' layout), or, on a coarser routing grid, its
   // L1_total_runoff, which L11_runoff_acc aggregates into that row here
@@ -2424,12 +2496,7 @@ extern "C" int mhmhip_mrm_step(mhmhip_ctx *x, const mhmhip_step *st, double *gau
                 "runoff_agg");
     if (x->n_inflow > 0 && it == 0)
       CHECK_HIP(x, launch_inflow_patch(r, x->d_ring, x->d_lag, 0, 1, x->stream), "inflow_patch");
-    if (flow) return route_one_step(x, r, g);
-    CHECK_RC(normalize_qtr(x));
-    x->flow_ready = false;
-    CHECK_RC(route_tiles(x, r, g, 0, g.nwin + g.tau_max));
-    x->qtr_slot = 0;
-    return MHMHIP_OK;
+    return route_one_step(x, r, g);
   };
   // loops routings of this step's qOUT (mRM_routing, mo_mrm_routing.f90:224-284):
   // the states advance each time, Qmod is their average
@@ -2455,11 +2522,7 @@ extern "C" int mhmhip_mrm_step(mhmhip_ctx *x, const mhmhip_step *st, double *gau
     }
   }
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "mrm_step");
-  if (*x->flow_fail) {
-    *x->flow_fail = 0;
-    x->flow_ready = false;
-    return x->fail(MHMHIP_EHIP, "mrm_step: the wait for an upstream tile gave up");
-  }
+  CHECK_RC(flow_check(x, "mrm_step"));
   if (gauge_out) copy_dup_gauges(x, gauge_out, 1);
   return prof_collect(x);
 }
@@ -2578,6 +2641,13 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
   // tiled routing: windows of B steps (the plain path routes in windows too)
   const int32_t B = tile_window(o.route_window);
   const int64_t ring_rows = route ? ring_need(x, kind, S * rep, B, nr) : 0;
+  const int64_t groups = route ? (int64_t)x->lay.bins.size() * x->n_sets : 0;
+  const bool tiled = route && kind == MHMHIP_K_ROUTE_TILE;
+  const bool flow = tiled && one_launch_pays(x, B, nr, ring_rows), windows = tiled && !flow;
+  // the ring's rows in use: whole cell launches, so that no routing launch's
+  // rows wrap
+  const int64_t ring_len = flow && ring_rows < nr ? ring_rows / ((int64_t)S * rep) * S * rep
+                                                  : ring_rows;
   ScratchSwap swap(x);
   if (noalloc) {
     // graph capture and instantiation, the routing stream and the timing
@@ -2636,7 +2706,7 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
   CellArgs a = cell_args(x, route);
   RouteArgs r = route_args(x, 0, nr, 0);
   if (route) {
-    a.ring_len = r.ring_len = ring_rows;  // this call's rows of the ring
+    a.ring_len = r.ring_len = ring_len;  // this call's rows of the ring
     a.ring_rep = r.rep = rep;
     if (kind == MHMHIP_K_ROUTE_TILE) a.lag = x->d_lag;  // qOUT written lag rows late
     if (rep > 1) {
@@ -2657,36 +2727,66 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
     a.ring_rep = 1;
     a.raw_total = 1;
   }
-  const TileArgs g = tile_args(x, B, nr);
-  const int32_t L_end = g.nwin + g.tau_max;
+  const TileArgs g = tile_args(x);
   const bool graph = o.use_graph && o.mode == MHMHIP_RUN_FUSED;
-  // A captured fused run puts the tiled routing on a stream of its own: a
-  // routing launch waits for the cell launch that completes its window, and
-  // the cell launches run on while the routing of earlier windows proceeds.
-  // When the ring is shorter than the call, a cell launch also waits for the
-  // routing launch that last reads the rows it overwrites.
-  const bool two = graph && route && kind == MHMHIP_K_ROUTE_TILE;
+  // A captured fused run puts routing that leaves room on the chip, or comes
+  // in many launches, on a stream of its own beside the cell launches that
+  // follow.  One that fills the chip for a few launches waits instead until
+  // the ring is full or the call ends.
+  const bool two = graph && tiled && (!flow || groups <= 256);
   if (two && !x->rstream)
     CHECK_HIP(x, hipStreamCreateWithFlags(&x->rstream, hipStreamNonBlocking), "routing stream");
-  const bool wrap = ring_rows < nr;
+  if (flow) CHECK_RC(flow_begin(x, "run"));
+  const WindowArgs win = window_args(x, B, nr);
+  const int32_t L_end = win.nwin + win.tau_max;
   // the whole loop, in steps relative to this call (replayable as a graph)
   auto enqueue = [&]() -> int {
-    int32_t L = 0;  // next tiled routing launch
+    int32_t L = 0;       // next launch of the windowed routing
+    int64_t routed = 0;  // steps whose routing in one launch is enqueued
     hipStream_t rs = two ? x->rstream : x->stream;
-    std::vector<hipEvent_t> evL(two && wrap ? L_end : 0, nullptr);  // routing launch L done
+    // two: events on the routing stream and the last steps whose ring rows
+    // are read before them
+    std::vector<std::pair<int64_t, hipEvent_t>> read;
     if (two) CHECK_RC(capture_edge(x, x->stream, rs));  // the routing stream joins the capture
+    auto mark = [&](int64_t t) -> int {
+      hipEvent_t e = nullptr;
+      if (ring_len < nr) {
+        CHECK_RC(capture_edge(x, rs, nullptr, &e));
+        read.emplace_back(t, e);
+      }
+      return MHMHIP_OK;
+    };
+    // the tiled routing that the steps before t allow
+    auto route_to = [&](int64_t t) -> int {
+      if (flow) {
+        if (t <= routed) return MHMHIP_OK;
+        if (two) CHECK_RC(capture_edge(x, x->stream, rs));
+        CHECK_RC(route_steps(x, r, g, routed, t, nr, rs));
+        routed = t;
+        return two ? mark(t) : MHMHIP_OK;
+      }
+      // launch L needs the steps of window L (its deepest tiles' window)
+      int32_t L1 = L;
+      while (L1 < L_end && std::min<int64_t>((int64_t)(L1 + 1) * B, nr) <= t) ++L1;
+      if (two && L1 > L) CHECK_RC(capture_edge(x, x->stream, rs));
+      for (; L < L1; ++L) {
+        CHECK_RC(route_tiles(x, r, g, win, L, L + 1, rs));
+        // launch L is the last that reads the rows of window L - tau_max
+        if (two && L >= win.tau_max) CHECK_RC(mark((int64_t)(L - win.tau_max + 1) * B));
+      }
+      return MHMHIP_OK;
+    };
     for (int32_t k = 0; k < nsteps; k += S) {
       const int n = std::min<int32_t>(S, nsteps - k);
-      // the launch's routing steps [u0, u1)
+      // the launch's routing steps [u0, u1), whose rows held those of
+      // ring_len steps before
       const int64_t u0 = (int64_t)k * rep, u1 = (int64_t)(k + n) * rep;
-      if (two && wrap && u1 - 1 - ring_rows >= 0) {
-        // rows of the routing steps up to u1 - 1 - R are overwritten: the
-        // last routing launch reading them is enqueued already
-        const int64_t Ln = (u1 - 1 - ring_rows) / B + g.tau_max;
-        if (Ln >= L) return x->fail(MHMHIP_EINVAL, "run: ring shorter than the routing lag");
-        int64_t Lw = Ln;
-        while (Lw >= 0 && !evL[Lw]) --Lw;  // a launch with no bin due reads nothing
-        if (Lw >= 0) CHECK_HIP(x, hipStreamWaitEvent(x->stream, evL[Lw], 0), "capture edge");
+      if (flow && u1 - routed > ring_len) CHECK_RC(route_to(u0));
+      if (two && u1 > ring_len) {
+        size_t i = 0;
+        while (i < read.size() && read[i].first < u1 - ring_len) ++i;
+        if (i == read.size()) return x->fail(MHMHIP_EINVAL, "run: ring shorter than the routing lag");
+        CHECK_HIP(x, hipStreamWaitEvent(x->stream, read[i].second, 0), "capture edge");
       }
       if (o.mode == MHMHIP_RUN_PLAIN) {
         CHECK_HIP(x, timed(x, MHMHIP_K_CELL_STEP, (double)x->n_cells * x->n_sets, [&] {
@@ -2703,41 +2803,21 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
       if (x->coarse)
         CHECK_HIP(x, launch_runoff_agg(x->d_cring, S, x->d_agg_start, x->d_area, x->n_nodes,
                                        x->sstride, x->ld, x->n_sets, x->d_ring, node_lag,
-                                       ring_rows, rep, k, n,
+                                       ring_len, rep, k, n,
                                        kHourSecs * (double)x->cfg.timestep, x->stream),
                   "runoff_agg");
       if (kind == MHMHIP_K_ROUTE_TILE && x->n_inflow > 0)
         CHECK_HIP(x, launch_inflow_patch(r, x->d_ring, x->d_lag, u0, u1, x->stream, rep),
                   "inflow_patch");
-      if (kind == MHMHIP_K_ROUTE_TILE) {
-        // launch L needs the steps of window L (its deepest tiles' window)
-        int32_t L1 = L;
-        while (L1 < L_end && std::min<int64_t>((int64_t)(L1 + 1) * B, nr) <= u1) ++L1;
-        if (two && L1 > L) {
-          CHECK_RC(capture_edge(x, x->stream, rs));
-          for (int32_t l = L; l < L1; ++l) {
-            CHECK_RC(route_tiles(x, r, g, l, l + 1, rs));
-            if (wrap) CHECK_RC(capture_edge(x, rs, nullptr, &evL[l]));
-          }
-        } else if (!two) {
-          CHECK_RC(route_tiles(x, r, g, L, L1));
-        }
-        L = L1;
-      } else {
-        CHECK_RC(route_diagonals(x, r, u0, u1, false, wg));
-      }
+      if (windows || (two && tiled)) CHECK_RC(route_to(u1));
+      if (!tiled) CHECK_RC(route_diagonals(x, r, u0, u1, false, wg));
     }
-    if (route && kind == MHMHIP_K_ROUTE_TILE) {
-      if (two) {
-        if (L < L_end) {
-          CHECK_RC(capture_edge(x, x->stream, rs));
-          CHECK_RC(route_tiles(x, r, g, L, L_end, rs));
-        }
-        CHECK_RC(capture_edge(x, rs, x->stream));  // join
-      } else {
-        CHECK_RC(route_tiles(x, r, g, L, L_end));
-      }
+    if (flow) CHECK_RC(route_to(nr));
+    if (windows && L < L_end) {
+      if (two) CHECK_RC(capture_edge(x, x->stream, rs));
+      CHECK_RC(route_tiles(x, r, g, win, L, L_end, rs));
     }
+    if (two) CHECK_RC(capture_edge(x, rs, x->stream));  // join
     if (route && kind != MHMHIP_K_ROUTE_TILE) CHECK_RC(route_diagonals(x, r, nr, 0, true, wg));
     return MHMHIP_OK;
   };
@@ -2753,7 +2833,7 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
     key.gauge = route ? x->d_gauge_buf : nullptr;
     key.steps = x->d_steps;
     key.inflow = x->d_inflow_q;
-    key.ring_len = ring_rows;
+    key.ring_len = ring_len;
     key.B = B;
     key.qacc = r.qacc;
     key.out = a.out.sum;
@@ -2784,7 +2864,7 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
   }
   if (route) {
     credit_route(x, kind, nr);
-    x->flow_ready = false;
+    if (windows) x->flow_ready = false;
     x->qtr_slot = (int)((nr - 1) & 1);
     if (x->qacc_on) x->qacc_count += nsteps;
     x->qsub_loops = rep;
@@ -2800,6 +2880,7 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
               "download gauges");
   }
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "run");
+  if (route) CHECK_RC(flow_check(x, "run"));
   if (!gsub.empty()) {
     // qAcc = qAcc + Qmod over the sub-steps, then Qmod = qAcc / rout_loop
     // (mo_mrm_routing.f90:246-284), per gauge

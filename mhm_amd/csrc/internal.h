@@ -250,12 +250,8 @@ struct BinInfo {
   int32_t height;    // tallest tile in the bin
   int32_t tau_lo;    // smallest / largest tile depth in the bin
   int32_t tau_hi;
-  int32_t out_rows;  // tile roots + gauge nodes of the bin (LDS output rows)
+  int32_t pad;
 };
-// LDS a tiled launch may use to stage its tile-root series and gauge sums;
-// past it the kernel stores them directly
-constexpr size_t kTileStageLds = 64 * 1024;
-
 struct RouteArgs {
   const NodeMeta *meta;    // [n_nodes]
   const int32_t *child_list;  // upstream device indices, NodeMeta.child offsets
@@ -303,21 +299,39 @@ struct MprLiteArgs {
   double gamma[kMprNGamma];
 };
 
-// Extra arguments of the tiled routing kernel.
+// Extra arguments of the tiled routing kernels.
 struct TileArgs {
-  const SlotMeta *slot;    // [n_bins * kTileSlots]
+  const SlotMeta *slot;    // [n_bins * kTileSlots]; a proxy's pos: the upstream tile's root
   const BinInfo *bin;      // [n_bins]
   const int32_t *node_gauge;  // [n_nodes] first gauge at the node (device index), -1: none
-  const int32_t *slot_out;    // [n_bins * kTileSlots] output rows: tile root (bits 0..15),
-                              // gauge (16..31), 0xFFFF: none
+  const int32_t *spare;    // [n_bins * kTileSlots] tile roots and their proxies: the root's
+                           // first upstream node
+  int64_t n_bnd;           // tile boundaries
+};
+
+// The windows of the windowed tiled routing.
+struct WindowArgs {
   double *bnd;             // [2][n_sets][n_bnd][bstride] tile-root outflow by window parity
-  int64_t n_bnd;
   int32_t tau_max;         // deepest tile
   int32_t B;               // steps per window
   int32_t nwin;            // windows in [t_lo, t_hi)
   int32_t bstride;         // boundary series length (kTileWindowMax)
-  int32_t out_rows;        // largest BinInfo.out_rows
-  int32_t pad;
+  int32_t out_rows;        // most tile roots + gauge nodes of a bin (LDS output rows)
+};
+// LDS a launch may use to stage its tile-root series and gauge sums; past it
+// the kernel stores them directly
+constexpr size_t kTileStageLds = 64 * 1024;
+
+// How the workgroups of a routing launch hand tiles on.
+struct FlowArgs {
+  uint64_t *area;     // per set: counter, give-up flag, words of a step's boundaries
+  int64_t astride;    // words between the sets' areas
+  uint32_t *fail;     // host word: a wait gave up
+  const uint8_t *lag; // [n_nodes] lag of the node in its tile
+  int32_t n_bins;
+  int32_t tickets;    // 0: no tile boundaries
+  int32_t proxy_waves, out_waves;  // per workgroup, beside the slots' (steps of the ring)
+  int32_t last;       // the launch ends the run
 };
 
 }  // namespace mhmhip

@@ -1115,6 +1115,13 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Diagonals that a tiled kernel fetches ahead of use.
+constexpr int kTileAhead = 4;
+// LDS parity buffers, in doubles: a value per slot and for the zero slot W,
+// whose +0.0 stands for a node's missing upstream slots (adding it leaves the
+// running sum's value unchanged).
+constexpr int kTileBuf = kTileSlots + 1;
+
 // ---------------------------------------------------------------------------
 // Tiled routing: launch L handles, for every tile of depth tau, the window
 // k = L - (tau_max - tau) of B steps.  Tile-root outflow of window k is
@@ -1147,8 +1154,6 @@ __device__ __forceinline__ void lds_barrier() {
 // 19.4 us; 8 fetches ahead instead of 4 gave the same.  Four steps per diagonal
 // (one LDS round trip for four steps) were slower where many bins are due (68
 // us: a window fills and drains over four times the steps), 17.7 us for eleven.
-constexpr int kTileAhead = 4;
-
 struct TileLane {
   const double *p;      // series element of window step 0
   uint64_t stride;      // bytes between consecutive elements of the series (0: idle)
@@ -1170,11 +1175,6 @@ struct TileOutRow {
   int32_t stride;  // elements between consecutive steps
   int32_t nb;      // steps to write
 };
-
-// LDS parity buffers, in doubles: a value per slot and for the zero slot W,
-// whose +0.0 stands for a node's missing upstream slots (adding it leaves the
-// running sum's value unchanged).
-constexpr int kTileBuf = kTileSlots + 1;
 
 // The diagonals [lo, hi) of the bin's nd (a multiple of kTileAhead) that a
 // wave's slots handle, lo a multiple of kTileAhead.
@@ -1276,28 +1276,30 @@ __device__ __forceinline__ void tile_sweep(const RouteArgs &r, TileLane &u, doub
   for (; d0 < w.nd; ++d0) lds_barrier();
 }
 
-// LDS: the parity buffers, then (STAGE) the bin's output rows: g.out_rows
-// TileOutRow, then g.out_rows x (B + 1) values and a scratch value per slot.
+// LDS: the parity buffers, then (STAGE) the bin's output rows: v.out_rows
+// TileOutRow, then v.out_rows x (B + 1) values and a scratch value per slot.
 // ACC: Qmod summed per node (r.qacc).
 template <bool STAGE, bool ACC>
 __global__ __launch_bounds__(kTileSlots) void route_tile_kernel(RouteArgs r, TileArgs g,
-                                                                int32_t L, int32_t bin0) {
+                                                                WindowArgs v, int32_t L,
+                                                                int32_t bin0) {
   extern __shared__ double lds[];
+  __shared__ int32_t n_rows;  // output rows given out
   constexpr int W = kTileSlots;
   const int bin = bin0 + blockIdx.x, set = blockIdx.y, s = threadIdx.x;
   const BinInfo bi = g.bin[bin];
   // whole bin idle in this launch: every thread leaves before any barrier
-  if (L - (g.tau_max - bi.tau_hi) < 0 || L - (g.tau_max - bi.tau_lo) >= g.nwin) return;
+  if (L - (v.tau_max - bi.tau_hi) < 0 || L - (v.tau_max - bi.tau_lo) >= v.nwin) return;
   const SlotMeta m = g.slot[(int64_t)bin * W + s];
   TileLane u;
-  const int32_t k = L - (g.tau_max - (m.b >> 16));
+  const int32_t k = L - (v.tau_max - (m.b >> 16));
   u.a = m.a;
   u.set = set;
   u.real = (m.a & SF_REAL) != 0;
   u.proxy = (m.a & SF_PROXY) != 0;
-  const bool act = (u.real || u.proxy) && k >= 0 && k < g.nwin;
-  u.t0 = r.t_lo + (int64_t)k * g.B;
-  u.nb = act ? (int)min((int64_t)g.B, r.t_hi - u.t0) : 0;
+  const bool act = (u.real || u.proxy) && k >= 0 && k < v.nwin;
+  u.t0 = r.t_lo + (int64_t)k * v.B;
+  u.nb = act ? (int)min((int64_t)v.B, r.t_hi - u.t0) : 0;
   u.lag = m.a & 0xFFF;
   u.nc = (m.a >> 12) & 0xF;
   u.c0 = m.b & 0xFFFF;
@@ -1318,40 +1320,38 @@ __global__ __launch_bounds__(kTileSlots) void route_tile_kernel(RouteArgs r, Til
       u.c2 = ldr(r.C2, u.bv);
     }
   } else if (act) {
-    u.p = g.bnd + (bseries + m.bnd) * g.bstride;
+    u.p = v.bnd + (bseries + m.bnd) * v.bstride;
     u.stride = 8;
   } else {
-    u.p = g.bnd;
+    u.p = v.bnd;
     u.stride = 0;
   }
-  u.bout = (act && (m.a & SF_TROOT)) ? g.bnd + (bseries + m.bnd) * g.bstride : nullptr;
+  u.bout = (act && (m.a & SF_TROOT)) ? v.bnd + (bseries + m.bnd) * v.bstride : nullptr;
   // gauges: the node's first gauge only (the host copies it to the others)
   u.gauge = (act && u.real && (m.a & NF_GAUGE)) ? g.node_gauge[m.pos] : -1;
   u.orow_t = u.orow_g = -1;
   u.qacc = ACC && act && u.real ? ldr(r.qacc, u.bv) : 0.0;
   double *qtr = lds;
   TileOutRow *rows = reinterpret_cast<TileOutRow *>(lds + 2 * kTileBuf);
-  double *out = reinterpret_cast<double *>(rows + g.out_rows);
+  double *out = reinterpret_cast<double *>(rows + v.out_rows);
   if (STAGE) {
-    // the slot's output rows (host-numbered inside the bin); an idle owner
-    // leaves its row empty
-    const int32_t so = g.slot_out[(int64_t)bin * W + s];
-    const int32_t rt = so & 0xFFFF, rg = (so >> 16) & 0xFFFF;
-    if (rt != 0xFFFF) {
-      u.orow_t = rt;
-      rows[rt] = TileOutRow{u.bout ? u.bout : g.bnd, 1, u.bout ? u.nb : 0};
+    // a row for each tile-root series and gauge, in any order
+    if (s == 0) n_rows = 0;
+    lds_barrier();
+    if (u.bout) {
+      u.orow_t = atomicAdd(&n_rows, 1);
+      rows[u.orow_t] = TileOutRow{u.bout, 1, u.nb};
     }
-    if (rg != 0xFFFF) {
-      u.orow_g = rg;
+    if (u.gauge >= 0) {
       const int64_t gi = ((u.t0 - r.t_base) * r.n_sets + set) * r.n_gauges + u.gauge;
-      rows[rg] = TileOutRow{u.gauge >= 0 ? r.gauge_out + gi : g.bnd, r.n_sets * r.n_gauges,
-                            u.gauge >= 0 ? u.nb : 0};
+      u.orow_g = atomicAdd(&n_rows, 1);
+      rows[u.orow_g] = TileOutRow{r.gauge_out + gi, r.n_sets * r.n_gauges, u.nb};
     }
   }
   if (s < 2) qtr[s * kTileBuf + W] = 0.0;
   lds_barrier();
   TileSpan w;
-  w.nd = (bi.height + g.B - 1 + kTileAhead - 1) / kTileAhead * kTileAhead;
+  w.nd = (bi.height + v.B - 1 + kTileAhead - 1) / kTileAhead * kTileAhead;
   int lo = u.nb > 0 ? u.lag : 0x7FFFFFFF, hi = u.nb > 0 ? u.lag + u.nb : 0;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
@@ -1362,19 +1362,19 @@ __global__ __launch_bounds__(kTileSlots) void route_tile_kernel(RouteArgs r, Til
   w.lo = min(__builtin_amdgcn_readfirstlane(lo), w.hi) & ~(kTileAhead - 1);
   const bool rare = u.nc > 5 || (u.real && (!(u.a & NF_QOUT) || (u.a & NF_CUT)));
   if (__any(rare))
-    tile_sweep<5, true, true, STAGE, ACC>(r, u, qtr, w, out, g.out_rows, g.B);
+    tile_sweep<5, true, true, STAGE, ACC>(r, u, qtr, w, out, v.out_rows, v.B);
   else if (__any(u.bout != nullptr || u.gauge >= 0))
-    tile_sweep<5, true, false, STAGE, ACC>(r, u, qtr, w, out, g.out_rows, g.B);
+    tile_sweep<5, true, false, STAGE, ACC>(r, u, qtr, w, out, v.out_rows, v.B);
   else if (__any(u.nc > 3))
-    tile_sweep<5, false, false, STAGE, ACC>(r, u, qtr, w, out, g.out_rows, g.B);
+    tile_sweep<5, false, false, STAGE, ACC>(r, u, qtr, w, out, v.out_rows, v.B);
   else
-    tile_sweep<3, false, false, STAGE, ACC>(r, u, qtr, w, out, g.out_rows, g.B);
+    tile_sweep<3, false, false, STAGE, ACC>(r, u, qtr, w, out, v.out_rows, v.B);
   if (STAGE) {
     // the sweep's last barrier follows its last rows
-    for (int idx = s; idx < bi.out_rows * g.B; idx += W) {
-      const int rr = idx / g.B, j = idx - rr * g.B;
+    for (int idx = s; idx < n_rows * v.B; idx += W) {
+      const int rr = idx / v.B, j = idx - rr * v.B;
       const TileOutRow o = rows[rr];
-      if (j < o.nb) o.base[(int64_t)j * o.stride] = out[rr * (g.B + 1) + j];
+      if (j < o.nb) o.base[(int64_t)j * o.stride] = out[rr * (v.B + 1) + j];
     }
   }
   if (act && u.real) {
@@ -1414,12 +1414,6 @@ __global__ __launch_bounds__(kTileSlots) void route_tile_kernel(RouteArgs r, Til
 // this launch's; relaxed device-scope accesses suffice.  The counter holds
 // the launch number and the tickets taken; who takes the last ticket sets it
 // for the next launch.
-struct StepFlow {
-  int32_t n_bins;
-  uint64_t *area;   // per set: counter, give-up flag, then from kFlowHead the words
-  int64_t astride;  // words between the sets' areas
-  uint32_t *fail;   // host word: a wait gave up
-};
 constexpr int kFlowHead = 16;
 // polls (0.6 us each) after which a wait gives up: the kernel ends, with an error
 constexpr int kFlowPolls = 1 << 22;
@@ -1431,25 +1425,38 @@ __device__ __forceinline__ void flow_store(uint64_t *p, uint64_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Workgroup's ticket (32 bits) under the launch number; without tile
+// boundaries nobody waits, and the block index serves.
+__device__ __forceinline__ uint64_t flow_ticket(const FlowArgs &f, uint64_t *area) {
+  if (!f.tickets) return blockIdx.x;
+  const uint64_t t = __hip_atomic_fetch_add(area, (uint64_t)1, __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT);
+  if ((uint32_t)t == (uint32_t)f.n_bins - 1) flow_store(area, ((t >> 32) + 1) << 32);
+  return t;
+}
+
+// A wait that took too long: all waits give up, and the host is told.
+__device__ __forceinline__ bool flow_gives_up(const FlowArgs &f, uint64_t *area, int polls) {
+  if ((polls & 1023) != 1023 || (polls < kFlowPolls && flow_load(area + 1) == 0)) return false;
+  flow_store(area + 1, 1);
+  __hip_atomic_store(f.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  return true;
+}
+
 __device__ __forceinline__ void flow_put(uint64_t *w, uint32_t tag, double v) {
   const uint64_t b = (uint64_t)__double_as_longlong(v), t = (uint64_t)tag << 32;
   flow_store(w, t | (b & 0xFFFFFFFFu));
   flow_store(w + 1, t | (b >> 32));
 }
 
-__device__ __forceinline__ double flow_get(const StepFlow &f, uint64_t *area, const uint64_t *w,
+__device__ __forceinline__ double flow_get(const FlowArgs &f, uint64_t *area, const uint64_t *w,
                                            uint32_t tag) {
   uint64_t lo, hi;
   for (int i = 0;; ++i) {
     lo = flow_load(w);
     hi = flow_load(w + 1);
     if ((uint32_t)(lo >> 32) == tag && (uint32_t)(hi >> 32) == tag) break;
-    if ((i & 1023) == 1023 && (i >= kFlowPolls || flow_load(area + 1) != 0)) {
-      // another workgroup's wait gave up, or this one: all give up
-      flow_store(area + 1, 1);
-      __hip_atomic_store(f.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      break;
-    }
+    if (flow_gives_up(f, area, i)) break;
     __builtin_amdgcn_s_sleep(1);
   }
   return __longlong_as_double((long long)((hi << 32) | (lo & 0xFFFFFFFFu)));
@@ -1505,17 +1512,14 @@ __device__ __forceinline__ void step_levels(StepLane &u, double *qtr, const doub
 // r.pub: the qTR row in use, updated in place.  r.t_lo = 0, r.t_hi = 1, a ring
 // of one step (rows by lag).
 template <bool ACC>
-__global__ __launch_bounds__(kTileSlots) void route_step_kernel(RouteArgs r, TileArgs g, StepFlow f) {
+__global__ __launch_bounds__(kTileSlots) void route_step_kernel(RouteArgs r, TileArgs g, FlowArgs f) {
   constexpr int W = kTileSlots;
   __shared__ double qtr[W + 1];
   __shared__ uint64_t ticket;
   const int s = threadIdx.x, set = blockIdx.y;
   uint64_t *area = f.area + (int64_t)set * f.astride;
   if (s == 0) {
-    const uint64_t t = __hip_atomic_fetch_add(area, (uint64_t)1, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-    if ((uint32_t)t == (uint32_t)f.n_bins - 1) flow_store(area, ((t >> 32) + 1) << 32);
-    ticket = t;
+    ticket = flow_ticket(f, area);
     qtr[W] = 0.0;
   }
   lds_barrier();
@@ -1582,6 +1586,328 @@ __global__ __launch_bounds__(kTileSlots) void route_step_kernel(RouteArgs r, Til
     // gauges: the node's first gauge only (the host copies it to the others)
     if (gauge >= 0) r.gauge_out[(int64_t)set * r.n_gauges + gauge] = u.sum;
     if (ACC) str(r.qacc, bv, ldr(r.qacc, bv) + u.sum);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Routing of the steps [t_lo, t_hi) of the ring in one launch: every workgroup
+// routes one bin of one set, all steps, as soon as the tiles upstream of it
+// hand their steps on.  The workgroup walks its own (depth, step) diagonals:
+// the slot with lag g handles step j on diagonal j + g, its upstream slots
+// (lag g - 1) produced step j on the diagonal before, and a two-entry LDS
+// parity buffer keeps it readable while they write step j + 1.  The tiles of a
+// bin that lie s levels of tile depth below its deepest ones run s (height +
+// kStreamSkew) diagonals late: by then the tiles they may wait for in the same
+// bin have handed the step on.
+// Same per-node arithmetic as route_node (mo_mrm_routing.f90:425-472).
+//
+// Waves by role.  0..3, a slot per lane: each real slot streams its qOUT from
+// the ring (inflow gauges already applied by inflow_patch_kernel), kTileAhead
+// diagonals ahead of use.  Then f.proxy_waves: each lane takes a proxy's steps
+// from the upstream tile.  Then f.out_waves: each lane hands a tile root's
+// steps on or stores a gauge's.  Loads, waits for other workgroups and stores
+// would hold up the slots' diagonals in one wave (stores and loads share a
+// counter, so a wait for a fetched value would wait for later stores).
+//
+// Hand-over: a root's step as two words in the ring, in the entries of that
+// step of the root itself and of its first upstream node, which nobody reads
+// any more: both hold 32 bits of the value under a tag.  The tags are
+// signalling NaNs, which no arithmetic yields, so that an entry's qOUT is
+// never taken for a word; an entry gets its next qOUT from a cell kernel after
+// this launch.  Tickets as in route_step_kernel.
+//
+// What bounds it: where the bins fill the chip, the ring's reads; else the
+// chain of diagonals, steps + levels of them (0.2 us each: LDS write, barrier
+// and read, 146 cycles, eight dependent FP64 operations, and whatever else a
+// wave issues).  Against the windowed launches: 150x220 nodes, 960 routing
+// steps through a ring of 192 rows 1504 -> 936 us; 215x301 nodes, 720 steps
+// 979 -> 579 us; 64x64 nodes, a year 2636 -> 2034 us; with the chip full no
+// gain (one_launch_pays in api.hip).
+constexpr int kStreamSkew = 8;
+constexpr uint32_t kTagLo = 0x7FF5A5A1u, kTagHi = 0x7FF5A5A2u;
+
+struct StreamLane {
+  const char *p;    // series element of step 0
+  uint64_t stride;  // bytes between consecutive elements
+  int32_t lag, n;   // n: steps, 0: idle
+  int32_t nc, c0;
+  bool noq, cut;
+  double qtin1, qtr1, c1, c2;
+  double qlast;     // qOUT of the last step
+  double qacc;      // Qmod summed over the steps (ACC)
+};
+
+// What a proxy or output lane does (LDS lists).
+struct StreamItem {
+  int32_t slot, lag;
+  int32_t a, b;  // nodes whose ring entries hold the words; output: b = -1: gauge a
+};
+
+// A wave's slots over the nd diagonals (a multiple of kTileAhead); NCW bounds
+// the upstream slots read together.  RARE: a slot has more than NCW upstream
+// slots, does not add its own qOUT or is cut by an inflow gauge.  Slots outside
+// their steps are masked; before the first and after the last diagonal that
+// one of its slots handles [lo, hi) the wave only keeps the barriers.
+template <int NCW, bool RARE, bool ACC>
+__device__ __forceinline__ void stream_slots(const RouteArgs &r, StreamLane &u, double *qtr,
+                                             double *gsum, bool gauges, int nd) {
+  constexpr int W = kTileSlots, A = kTileAhead;
+  const int s = threadIdx.x;
+  int lo = u.n > 0 ? u.lag : 0x7FFFFFFF, hi = u.n > 0 ? u.lag + u.n : 0;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = min(lo, __shfl_xor(lo, o));
+    hi = max(hi, __shfl_xor(hi, o));
+  }
+  hi = __builtin_amdgcn_readfirstlane(hi);
+  lo = min(__builtin_amdgcn_readfirstlane(lo), hi) & ~(A - 1);
+  const double *up[NCW];  // the upstream slots in buffer 0
+#pragma unroll
+  for (int c = 0; c < NCW; ++c) up[c] = qtr + (c < u.nc ? u.c0 + c : W);
+  // value for diagonal d: the slot's step d - lag, its first or last one
+  // outside its diagonals
+  const char *p = u.p;
+  const uint32_t moves = u.n > 0 ? u.n - 1 : 0;
+  double qq[A];
+  auto fetch = [&](int d, double &q) {
+    if ((uint32_t)(d - u.lag - 1) < moves) p += u.stride;
+    q = *reinterpret_cast<const double *>(p);
+  };
+  double musk = u.qtr1 + u.c1 * (u.qtin1 - u.qtr1);  // qTR(IT1) + C1 (qTIN(IT1) - qTR(IT1))
+  // Diagonal d reads parity buffer (d + 1) & 1, written on diagonal d - 1, and
+  // writes buffer d & 1 (wb).
+  auto diagonal = [&](int d, int wb, double qo) {
+    const int j = d - u.lag;
+    if ((uint32_t)j >= (uint32_t)u.n) return;
+    double v[NCW];
+#pragma unroll
+    for (int c = 0; c < NCW; ++c) v[c] = up[c][(wb ^ 1) * kTileBuf];
+    // upstream qTR in routing rank, then the node's own qOUT
+    double sum = v[0];
+#pragma unroll
+    for (int c = 1; c < NCW; ++c) sum = sum + v[c];
+    if (RARE) {
+#pragma nounroll
+      for (int c = NCW; c < u.nc; ++c) sum = sum + qtr[(wb ^ 1) * kTileBuf + u.c0 + c];
+    }
+    sum = sum + (RARE && u.noq ? 0.0 : qo);
+    // musk = qTR(IT1) + C1 (qTIN(IT1) - qTR(IT1)), formed on the diagonal before
+    double q = musk + u.c2 * (sum - u.qtin1);
+    if (RARE && u.cut) q = 0.0;
+    qtr[wb * kTileBuf + s] = q;
+    if (gauges) gsum[wb * W + s] = sum;
+    u.qtr1 = q;
+    u.qtin1 = sum;
+    u.qlast = qo;
+    musk = q + u.c1 * (sum - q);
+    // Qmod of step j, added in step order
+    if (ACC && r.t_lo + j >= r.acc_from) u.qacc = u.qacc + sum;
+  };
+#pragma unroll
+  for (int i = 0; i < A; ++i) fetch(lo + i, qq[i]);
+#pragma nounroll
+  for (int d = 0; d < lo; ++d) lds_barrier();
+  int d0 = lo;
+#pragma nounroll
+  for (; d0 < hi; d0 += A) {
+#pragma unroll
+    for (int i = 0; i < A; ++i) {
+      // every lane waits for this diagonal's value here, whether it uses it
+      // or not: the register is free for the next fetch
+      settle(qq[i]);
+      diagonal(d0 + i, i & 1, qq[i]);
+      lds_barrier();
+      fetch(d0 + i + A, qq[i]);
+    }
+  }
+#pragma nounroll
+  for (; d0 < nd; ++d0) lds_barrier();
+}
+
+// A proxy wave: each lane brings an upstream tile root's steps into its
+// proxy's slot, kTileAhead diagonals ahead of use, and waits for a step that
+// was not there yet.
+__device__ __forceinline__ void stream_proxies(const RouteArgs &r, const FlowArgs &f, uint64_t *area,
+                                               const StreamItem &m, bool have, int n,
+                                               const char *pa, const char *pb, uint64_t stride,
+                                               double *qtr, int nd) {
+  constexpr int A = kTileAhead;
+  const char *p = pa, *p2 = pb;
+  const uint32_t moves = have ? n - 1 : 0;
+  uint64_t wa[A], wb[A];
+  bool dead = false;  // a wait gave up
+  auto fetch = [&](int d, uint64_t &a, uint64_t &b) {
+    if ((uint32_t)(d - m.lag - 1) < moves) {
+      p += stride;
+      p2 += stride;
+    }
+    a = flow_load(reinterpret_cast<const uint64_t *>(p));
+    b = flow_load(reinterpret_cast<const uint64_t *>(p2));
+  };
+  auto ready = [](uint64_t a, uint64_t b) {
+    return (uint32_t)(a >> 32) == kTagLo && (uint32_t)(b >> 32) == kTagHi;
+  };
+#pragma unroll
+  for (int i = 0; i < A; ++i) fetch(i, wa[i], wb[i]);
+#pragma nounroll
+  for (int d0 = 0; d0 < nd; d0 += A) {
+#pragma unroll
+    for (int i = 0; i < A; ++i) {
+      const int j = d0 + i - m.lag;
+      if (have && (uint32_t)j < (uint32_t)n) {
+        uint64_t a = wa[i], b = wb[i];
+        if (!ready(a, b) && !dead) {
+          const uint64_t *qa = reinterpret_cast<const uint64_t *>(pa + (uint64_t)j * stride);
+          const uint64_t *qb = reinterpret_cast<const uint64_t *>(pb + (uint64_t)j * stride);
+          for (int k = 0;; ++k) {
+            a = flow_load(qa);
+            b = flow_load(qb);
+            if (ready(a, b)) break;
+            if (flow_gives_up(f, area, k)) {
+              dead = true;
+              break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+          }
+        }
+        qtr[(i & 1) * kTileBuf + m.slot] =
+            __longlong_as_double((long long)((b << 32) | (a & 0xFFFFFFFFu)));
+      }
+      lds_barrier();
+      fetch(d0 + i + A, wa[i], wb[i]);
+    }
+  }
+}
+
+// An output wave: on the diagonal after a slot's, each lane hands its tile
+// root's step on or stores its gauge's.
+__device__ __forceinline__ void stream_outputs(const StreamItem &m, bool have, int n, char *pa,
+                                               char *pb, uint64_t stride, const double *qtr,
+                                               const double *gsum, int nd) {
+  const bool gauge = m.b < 0;
+  auto put = [&](int d, int rb) {  // diagonal d's values, in parity buffer rb
+    if (!have || (uint32_t)(d - m.lag) >= (uint32_t)n) return;
+    if (gauge) {
+      *reinterpret_cast<double *>(pa) = gsum[rb * kTileSlots + m.slot];
+    } else {
+      const uint64_t v = (uint64_t)__double_as_longlong(qtr[rb * kTileBuf + m.slot]);
+      flow_store(reinterpret_cast<uint64_t *>(pa), (uint64_t)kTagLo << 32 | (v & 0xFFFFFFFFu));
+      flow_store(reinterpret_cast<uint64_t *>(pb), (uint64_t)kTagHi << 32 | (v >> 32));
+      pb += stride;
+    }
+    pa += stride;
+  };
+  lds_barrier();  // diagonal 0
+#pragma nounroll
+  for (int d = 1; d < nd; d += 2) {
+    put(d - 1, 0);
+    lds_barrier();
+    put(d, 1);
+    if (d + 1 < nd) lds_barrier();
+  }
+}
+
+// ACC: Qmod summed per node (r.qacc).  last: t_hi ends the run (r.qOUT).
+template <bool ACC>
+__global__ __launch_bounds__(1024) void route_stream_kernel(RouteArgs r, TileArgs g, FlowArgs f) {
+  constexpr int W = kTileSlots;
+  __shared__ double qtr[2 * kTileBuf];
+  __shared__ double gsum[2 * W];
+  __shared__ StreamItem proxy[W], output[2 * W];
+  __shared__ uint64_t ticket;
+  __shared__ int32_t n_proxy, n_output;
+  const int s = threadIdx.x, set = blockIdx.y;
+  uint64_t *area = f.area + (int64_t)set * f.astride;
+  if (s == 0) {
+    ticket = flow_ticket(f, area);
+    n_proxy = n_output = 0;
+    qtr[W] = qtr[kTileBuf + W] = 0.0;
+  }
+  lds_barrier();
+  const int bin = __builtin_amdgcn_readfirstlane(f.n_bins - 1 - (int32_t)(uint32_t)ticket);
+  const BinInfo bi = g.bin[bin];
+  const int n = (int)(r.t_hi - r.t_lo);
+  const int skew = bi.height + kStreamSkew;
+  const int64_t ld = (int64_t)r.n_sets * r.sstride;
+  const int64_t row0 = ring_row(r.t_lo, 0, r.ring_len);
+  char *ring = reinterpret_cast<char *>(const_cast<double *>(r.ring) + row0 * ld +
+                                        (int64_t)set * r.sstride);
+  const int wave = __builtin_amdgcn_readfirstlane(s / 64);
+  StreamLane u{};
+  uint32_t bv = 0;
+  bool real = false, link = false, gauges = false;
+  if (wave < W / 64) {
+    const SlotMeta m = g.slot[(int64_t)bin * W + s];
+    const int32_t spare = g.spare[(int64_t)bin * W + s];
+    real = (m.a & SF_REAL) != 0;
+    link = (m.a & NF_LINK) != 0;
+    const int32_t lag = m.a & 0xFFF;
+    u.lag = lag + (bi.tau_hi - (m.b >> 16)) * skew;
+    u.nc = (m.a >> 12) & 0xF;
+    u.c0 = m.b & 0xFFFF;
+    u.noq = real && !(m.a & NF_QOUT);
+    u.cut = real && (m.a & NF_CUT);
+    u.p = ring;
+    if (m.a & SF_PROXY) proxy[atomicAdd(&n_proxy, 1)] = StreamItem{s, u.lag, m.pos, spare};
+    if (real) {
+      u.n = n;
+      u.p = ring + ((int64_t)lag * ld + m.pos) * 8;
+      u.stride = (uint64_t)ld * 8u;
+      bv = (uint32_t)(set * r.sstride + m.pos) * 8u;
+      u.qtin1 = ldr(r.qTIN, bv);
+      if (link) {
+        u.qtr1 = ldr(r.pub + ((r.t_lo - 1) & 1) * ld, bv);
+        u.c1 = ldr(r.C1, bv);
+        u.c2 = ldr(r.C2, bv);
+      }
+      if (ACC) u.qacc = ldr(r.qacc, bv);
+      if (m.a & SF_TROOT) output[atomicAdd(&n_output, 1)] = StreamItem{s, u.lag, m.pos, spare};
+      // gauges: the node's first gauge only (the host copies it to the others)
+      if (m.a & NF_GAUGE)
+        output[atomicAdd(&n_output, 1)] = StreamItem{s, u.lag, g.node_gauge[m.pos], -1};
+    }
+    gauges = __any(real && (m.a & NF_GAUGE));
+  }
+  lds_barrier();
+  const int nd = (n + bi.height - 1 + (bi.tau_hi - bi.tau_lo) * skew + kTileAhead - 1) /
+                 kTileAhead * kTileAhead;
+  if (wave < W / 64) {
+    if (__any(u.nc > 5 || u.noq || u.cut)) stream_slots<5, true, ACC>(r, u, qtr, gsum, gauges, nd);
+    else if (__any(u.nc > 3)) stream_slots<5, false, ACC>(r, u, qtr, gsum, gauges, nd);
+    else stream_slots<3, false, ACC>(r, u, qtr, gsum, gauges, nd);
+    if (real) {
+      str(r.qTIN, bv, u.qtin1);
+      if (link) str(r.pub + ((r.t_hi - 1) & 1) * ld, bv, u.qtr1);
+      if (f.last && r.qOUT) str(r.qOUT, bv, u.qlast);
+      if (ACC) str(r.qacc, bv, u.qacc);
+    }
+  } else if (wave < W / 64 + f.proxy_waves) {
+    const int i = s - W;
+    const bool have = i < n_proxy;
+    const StreamItem m = have ? proxy[i] : StreamItem{0, 0, 0, 0};
+    if (__any(have))
+      stream_proxies(r, f, area, m, have, n, ring + ((int64_t)f.lag[m.a] * ld + m.a) * 8,
+                     ring + ((int64_t)f.lag[m.b] * ld + m.b) * 8, have ? (uint64_t)ld * 8u : 0,
+                     qtr, nd);
+    else
+      for (int d = 0; d < nd; ++d) lds_barrier();
+  } else {
+    const int i = s - W - 64 * f.proxy_waves;
+    const bool have = i < n_output;
+    const StreamItem m = have ? output[i] : StreamItem{0, 0, 0, 0};
+    const bool gauge = m.b < 0;
+    char *pa = ring + ((int64_t)f.lag[gauge ? 0 : m.a] * ld + m.a) * 8;
+    char *pb = ring + ((int64_t)f.lag[gauge ? 0 : m.b] * ld + m.b) * 8;
+    uint64_t stride = (uint64_t)ld * 8u;
+    if (gauge) {
+      pa = reinterpret_cast<char *>(
+          r.gauge_out + ((r.t_lo - r.t_base) * r.n_sets + set) * r.n_gauges + m.a);
+      stride = (uint64_t)r.n_sets * r.n_gauges * 8u;
+    }
+    if (__any(have))
+      stream_outputs(m, have, n, pa, pb, stride, qtr, gsum, nd);
+    else
+      for (int d = 0; d < nd; ++d) lds_barrier();
   }
 }
 
@@ -1879,50 +2205,72 @@ hipError_t launch_route_diag(const RouteArgs &r, int64_t d, int64_t p_lo, int64_
   return hipGetLastError();
 }
 
-hipError_t launch_route_tile(const RouteArgs &r, const TileArgs &g, int64_t bin_lo, int64_t bin_hi,
+hipError_t launch_route_tile(const RouteArgs &r, const TileArgs &g, const WindowArgs &v,
+                             int64_t bin_lo, int64_t bin_hi,
                              int64_t n_bins, int32_t L, hipStream_t s) {
   // a window's rows do not wrap (ring length and window starts are multiples
   // of B; the ring has kTileHeight rows past its length), and a ring row's
   // bytes fit the kernel's 32-bit stride
-  if (bin_lo < 0 || bin_hi > n_bins || bin_hi <= bin_lo || g.B < 1 || g.B > g.bstride ||
-      g.bstride > kTileWindowMax || g.nwin < 1 || r.ring_len % g.B != 0 || r.t_lo % g.B != 0 ||
+  if (bin_lo < 0 || bin_hi > n_bins || bin_hi <= bin_lo || v.B < 1 || v.B > v.bstride ||
+      v.bstride > kTileWindowMax || v.nwin < 1 || r.ring_len % v.B != 0 || r.t_lo % v.B != 0 ||
       (uint64_t)r.n_sets * (uint64_t)r.sstride * 8u > 0xFFFFFFFFull)
     return hipErrorInvalidValue;
   dim3 grid((unsigned)(bin_hi - bin_lo), (unsigned)r.n_sets);
   const size_t base = sizeof(double) * 2 * (size_t)kTileBuf;
-  const size_t stage = (size_t)g.out_rows * (sizeof(TileOutRow) + sizeof(double) * (g.B + 1)) +
+  const size_t stage = (size_t)v.out_rows * (sizeof(TileOutRow) + sizeof(double) * (v.B + 1)) +
                        sizeof(double) * kTileSlots;
   const bool st = base + stage <= kTileStageLds;
   const size_t shm = st ? base + stage : base;
   if (st && r.qacc)
-    hipLaunchKernelGGL((route_tile_kernel<true, true>), grid, dim3(kTileSlots), shm, s, r, g, L,
+    hipLaunchKernelGGL((route_tile_kernel<true, true>), grid, dim3(kTileSlots), shm, s, r, g, v, L,
                        (int32_t)bin_lo);
   else if (st)
-    hipLaunchKernelGGL((route_tile_kernel<true, false>), grid, dim3(kTileSlots), shm, s, r, g, L,
+    hipLaunchKernelGGL((route_tile_kernel<true, false>), grid, dim3(kTileSlots), shm, s, r, g, v, L,
                        (int32_t)bin_lo);
   else if (r.qacc)
-    hipLaunchKernelGGL((route_tile_kernel<false, true>), grid, dim3(kTileSlots), shm, s, r, g, L,
+    hipLaunchKernelGGL((route_tile_kernel<false, true>), grid, dim3(kTileSlots), shm, s, r, g, v, L,
                        (int32_t)bin_lo);
   else
-    hipLaunchKernelGGL((route_tile_kernel<false, false>), grid, dim3(kTileSlots), shm, s, r, g, L,
+    hipLaunchKernelGGL((route_tile_kernel<false, false>), grid, dim3(kTileSlots), shm, s, r, g, v, L,
                        (int32_t)bin_lo);
   return hipGetLastError();
 }
 
-hipError_t launch_route_step(const RouteArgs &r, const TileArgs &g, int64_t n_bins, uint64_t *area,
-                             int64_t astride, uint32_t *fail, hipStream_t s) {
-  // one step of a one-step ring; a set's area holds the words of its boundary
-  // rows; 32-bit tickets and byte offsets
-  if (n_bins < 1 || n_bins > 0x7FFFFFFF || r.ring_len != 1 || r.t_lo != 0 || r.t_hi != 1 ||
-      r.t_base != 0 || !area || !fail || astride < kFlowHead + 2 * g.n_bnd ||
-      (uint64_t)r.n_sets * (uint64_t)r.sstride * 8u > 0xFFFFFFFFull)
+namespace {
+// a set's area holds the words of its boundary rows; 32-bit byte offsets
+bool flow_fits(const RouteArgs &r, const TileArgs &g, const FlowArgs &f) {
+  return f.n_bins >= 1 && f.area && f.fail && f.lag && f.astride >= kFlowHead + 2 * g.n_bnd &&
+         (uint64_t)r.n_sets * (uint64_t)r.sstride * 8u <= 0xFFFFFFFFull;
+}
+}  // namespace
+
+hipError_t launch_route_step(const RouteArgs &r, const TileArgs &g, const FlowArgs &f,
+                             hipStream_t s) {
+  // one step of a one-step ring
+  if (!flow_fits(r, g, f) || r.ring_len != 1 || r.t_lo != 0 || r.t_hi != 1 || r.t_base != 0)
     return hipErrorInvalidValue;
-  const StepFlow f{(int32_t)n_bins, area, astride, fail};
-  dim3 grid((unsigned)n_bins, (unsigned)r.n_sets);
+  dim3 grid((unsigned)f.n_bins, (unsigned)r.n_sets);
   if (r.qacc)
     hipLaunchKernelGGL(route_step_kernel<true>, grid, dim3(kTileSlots), 0, s, r, g, f);
   else
     hipLaunchKernelGGL(route_step_kernel<false>, grid, dim3(kTileSlots), 0, s, r, g, f);
+  return hipGetLastError();
+}
+
+hipError_t launch_route_stream(const RouteArgs &r, const TileArgs &g, const FlowArgs &f,
+                               hipStream_t s) {
+  // the steps' rows do not wrap (the ring has the tiles' height in rows past
+  // its length), and the proxies and outputs of a bin have a lane each
+  if (!flow_fits(r, g, f) || r.t_lo < 0 || r.t_hi <= r.t_lo || r.t_hi - r.t_lo > 0x3FFFFFFF ||
+      r.t_lo % r.ring_len + (r.t_hi - r.t_lo) > r.ring_len || f.proxy_waves < 0 ||
+      f.out_waves < 0 || f.proxy_waves > 4 || f.out_waves > 8)
+    return hipErrorInvalidValue;
+  dim3 grid((unsigned)f.n_bins, (unsigned)r.n_sets);
+  dim3 block((unsigned)(kTileSlots + 64 * (f.proxy_waves + f.out_waves)));
+  if (r.qacc)
+    hipLaunchKernelGGL(route_stream_kernel<true>, grid, block, 0, s, r, g, f);
+  else
+    hipLaunchKernelGGL(route_stream_kernel<false>, grid, block, 0, s, r, g, f);
   return hipGetLastError();
 }
 

@@ -14,10 +14,13 @@ hipError_t launch_cell_fused(int nh, const CellArgs &a, int64_t t0, int nsteps, 
                              int block, int n_sets, hipStream_t s);
 hipError_t launch_route_diag(const RouteArgs &r, int64_t d, int64_t p_lo, int64_t p_hi,
                              hipStream_t s);
-hipError_t launch_route_step(const RouteArgs &r, const TileArgs &g, int64_t n_bins, uint64_t *area,
-                             int64_t astride, uint32_t *fail, hipStream_t s);
-hipError_t launch_route_tile(const RouteArgs &r, const TileArgs &g, int64_t bin_lo, int64_t bin_hi,
-                             int64_t n_bins, int32_t L, hipStream_t s);
+hipError_t launch_route_tile(const RouteArgs &r, const TileArgs &g, const WindowArgs &v,
+                             int64_t bin_lo, int64_t bin_hi, int64_t n_bins, int32_t L,
+                             hipStream_t s);
+hipError_t launch_route_step(const RouteArgs &r, const TileArgs &g, const FlowArgs &f,
+                             hipStream_t s);
+hipError_t launch_route_stream(const RouteArgs &r, const TileArgs &g, const FlowArgs &f,
+                               hipStream_t s);
 hipError_t launch_inflow_patch(const RouteArgs &r, double *ring, const uint8_t *lag, int64_t t_lo,
                                int64_t t_hi, hipStream_t s, int32_t rep = 1);
 hipError_t launch_meteo_l2(const double *data2, const uint8_t *mask2, int32_t nr2, int64_t n2,

@@ -109,3 +109,33 @@ def test_step_by_step_matches_the_windows(height, inflow, packed):
     for a, b in zip(r1, r2):
         for k in a:
             assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("height,window,n,windows", [(16, 64, 320, True), (16, 50, 333, True),
+                                                     (24, 64, 330, True), (16, 4, 43, False)])
+def test_many_sets_match_the_wavefront(height, window, n, windows):
+    """Enough workgroups (bins times sets) to fill the chip: long windows go to
+    the windowed launches (kernels.hip: route_tile_kernel), short ones to the
+    one launch; with an inflow gauge, in pieces that end inside a window, and
+    Qmod sums; bit for bit the wavefront's."""
+    print(f"case: 100 sets, tile height {height}, window {window}, {n} steps", flush=True)
+    sys.stdout.flush()
+    got = []
+    for mode, h in ((1, 0), (3, height)):
+        dom = synth.make_domain(61, 60, seed=52)
+        dom.gauge_nodes = (np.argsort(dom.depth)[[0, 1, 15, 16, 17, 900, 2500]] + 1).astype(np.int32)
+        model, _, steps, _ = make_pair([dom], n_sets=100, n_steps=n, seed=14, tile_height=h,
+                                       inflow=_inflow(dom, n))
+        model.qmod_accumulate()
+        model.set_profiling(True, 1)
+        g = model.run(steps, mode=1, steps_per_launch=24, route_mode=mode,
+                      route_window=window if mode == 3 else 0)
+        if mode == 3:
+            assert (model.profile()["route_tile"][1] > 3) == windows
+        got.append((g, [model.routing_state(s) for s in (0, 77, 99)], model.qmod_sum(77)[0]))
+        model.close()
+    (g1, r1, q1), (g3, r3, q3) = got
+    assert np.array_equal(g1, g3) and np.array_equal(q1, q3)
+    for a, b in zip(r1, r3):
+        for k in a:
+            assert np.array_equal(a[k], b[k]), k
