@@ -250,6 +250,9 @@ struct mhmhip_ctx {
     bool stale = true;
   };
   HostOrder cell_order, node_order, link_order;
+  // links' length, slope, sealed flood plain fraction and domain's largest
+  // slope in pinned host memory (reg_rout)
+  double *link_in = nullptr;
   static constexpr int kRowParts = 8;
   hipEvent_t row_ev[kRowParts] = {};  // the parts of a row under way
 
@@ -523,6 +526,7 @@ extern "C" int mhmhip_destroy(mhmhip_ctx *x) {
   if (x->cell_order.pos) (void)hipHostFree(x->cell_order.pos);
   if (x->node_order.pos) (void)hipHostFree(x->node_order.pos);
   if (x->link_order.pos) (void)hipHostFree(x->link_order.pos);
+  if (x->link_in) (void)hipHostFree(x->link_in);
   for (hipEvent_t e : x->row_ev)
     if (e) (void)hipEventDestroy(e);
   if (x->cstream) (void)hipStreamSynchronize(x->cstream);
@@ -605,8 +609,24 @@ int put_node_row(mhmhip_ctx *x, double *dst, const double *src) {
   return stage_send(x, dst, row);
 }
 
-// n values of a device row in the reference's order (fill writes the device
-// index of every cell, node or link) to the host: gathered on the device into a pinned staging row
+// The device index of the n cells, nodes or links (fill writes them) in pinned
+// memory, current.
+template <typename Fn>
+int host_order(mhmhip_ctx *x, mhmhip_ctx::HostOrder &o, int64_t n, Fn fill) {
+  if (!o.stale && o.n == n) return MHMHIP_OK;
+  CHECK_HIP(x, hipStreamSynchronize(x->stream), "pinned order");  // kernels may read the old one
+  if (o.pos) (void)hipHostFree(o.pos);
+  o.pos = nullptr;
+  o.n = n;
+  o.stale = true;
+  if (hipHostMalloc((void **)&o.pos, sizeof(int32_t) * n, hipHostMallocDefault) != hipSuccess)
+    return x->fail(MHMHIP_ENOMEM, "pinned order allocation failed");
+  fill(o.pos);
+  o.stale = false;
+  return MHMHIP_OK;
+}
+
+// n values of a device row in the reference's order (host_order) to the host: gathered on the device into a pinned staging row
 // and copied from there.  A row of 64k values or more is split, so that the
 // host copies one part while the next ones cross the link (1M cells: 340 us
 // with 8 parts, 470 with one; at 65k cells 34 and 36).
@@ -614,16 +634,7 @@ template <typename Fn>
 int get_ordered(mhmhip_ctx *x, const double *srcdev, mhmhip_ctx::HostOrder &o, int64_t n, Fn fill,
                 double *dst) {
   if (n < 1) return MHMHIP_OK;
-  if (o.stale || o.n != n) {
-    if (o.pos) (void)hipHostFree(o.pos);
-    o.pos = nullptr;
-    o.n = n;
-    o.stale = true;
-    if (hipHostMalloc((void **)&o.pos, sizeof(int32_t) * n, hipHostMallocDefault) != hipSuccess)
-      return x->fail(MHMHIP_ENOMEM, "download: pinned cell order allocation failed");
-    fill(o.pos);
-    o.stale = false;
-  }
+  CHECK_RC(host_order(x, o, n, fill));
   double *row = nullptr;
   CHECK_RC(stage_take(x, &row));
   const int parts = (int)std::max<int64_t>(1, std::min<int64_t>(n / 65536, mhmhip_ctx::kRowParts));
@@ -660,12 +671,16 @@ int get_node_row(mhmhip_ctx *x, const double *srcdev, double *dst) {
   }, dst);
 }
 
+// device index of every link's source node
+void link_nodes(const mhmhip_ctx *x, int32_t *p) {
+  for (int64_t q = 0; q < x->n_nodes; ++q)
+    if (x->lay.link_of_node[q] >= 0) p[x->lay.link_of_node[q]] = (int32_t)q;
+}
+
 // one row of link values (at their source nodes) -> the links' order
 int get_link_row(mhmhip_ctx *x, const double *srcdev, double *dst) {
-  return get_ordered(x, srcdev, x->link_order, x->lay.n_links_total, [x](int32_t *p) {
-    for (int64_t q = 0; q < x->n_nodes; ++q)
-      if (x->lay.link_of_node[q] >= 0) p[x->lay.link_of_node[q]] = (int32_t)q;
-  }, dst);
+  return get_ordered(x, srcdev, x->link_order, x->lay.n_links_total,
+                     [x](int32_t *p) { link_nodes(x, p); }, dst);
 }
 
 int var_cols(const mhmhip_ctx *x, int var) {
@@ -1820,6 +1835,11 @@ extern "C" int mhmhip_bind_network(mhmhip_ctx *x, const mhmhip_network *net) {
   for (int d = 0; d < x->n_domains; ++d)
     x->dom_link_start[d + 1] = x->dom_link_start[d] + (ds[d + 1] - ds[d]) - x->h_nout[d];
   const int64_t nLtot = x->dom_link_start[x->n_domains];
+  if (x->link_in) {
+    CHECK_HIP(x, hipStreamSynchronize(x->stream), "bind_network");
+    (void)hipHostFree(x->link_in);
+    x->link_in = nullptr;
+  }
   x->h_length.assign(net->length, net->length + nLtot);
   x->h_slope.assign(net->slope, net->slope + nLtot);
   x->h_fFPimp.assign(net->fFPimp, net->fFPimp + nLtot);
@@ -2036,25 +2056,37 @@ int upload_coefs(mhmhip_ctx *x, int32_t set, Fn coef) {
   return MHMHIP_OK;
 }
 
-// reg_rout (mo_mrm_mpr.f90:61-119) over the links [l0, l1) of one domain,
-// TS = real(timestep) [h]
-void reg_rout(const mhmhip_ctx *x, const double *p, int64_t l0, int64_t l1, double *c1,
-              double *c2) {
-  if (l1 <= l0) return;
-  const double TS = (double)x->cfg.timestep;
-  double ssMax = x->h_slope[l0];
-  for (int64_t i = l0 + 1; i < l1; ++i)
-    if (x->h_slope[i] > ssMax) ssMax = x->h_slope[i];
-  for (int64_t i = l0; i < l1; ++i) {
-    double K = p[0] + p[1] * (x->h_length[i] * 0.001) + p[2] * x->h_slope[i] + p[3] * x->h_fFPimp[i];
-    double xi = p[4] * (1.0 + x->h_slope[i] / ssMax);
-    if (xi > 0.5) xi = 0.5;
-    if (xi < 0.005) xi = 0.005;
-    if (K > 0.5 * TS / xi) K = 0.5 * TS / xi;
-    if (K < 0.5 * TS / (1.0 - xi)) K = 0.5 * TS / (1.0 - xi);
-    c1[i] = TS / (K * (1.0 - xi) + 0.5 * TS);
-    c2[i] = 1.0 - c1[i] * K / TS;
+// reg_rout (mo_mrm_mpr.f90:61-119) of one set over the links [l0, l1)
+int reg_rout(mhmhip_ctx *x, int32_t set, const double *p, int64_t l0, int64_t l1) {
+  if (l1 <= l0) return MHMHIP_OK;
+  const int64_t n = x->lay.n_links_total;
+  CHECK_RC(host_order(x, x->link_order, n, [x](int32_t *q) { link_nodes(x, q); }));
+  if (!x->link_in) {
+    if (hipHostMalloc((void **)&x->link_in, sizeof(double) * 4 * n, hipHostMallocDefault) !=
+        hipSuccess)
+      return x->fail(MHMHIP_ENOMEM, "reg_rout: pinned link inputs allocation failed");
+    for (int64_t i = 0; i < n; ++i) {
+      x->link_in[i] = x->h_length[i];
+      x->link_in[n + i] = x->h_slope[i];
+      x->link_in[2 * n + i] = x->h_fFPimp[i];
+    }
+    for (int d = 0; d < x->n_domains; ++d) {
+      const int64_t a = x->dom_link_start[d], b = x->dom_link_start[d + 1];
+      if (b <= a) continue;
+      double ss_max = x->h_slope[a];
+      for (int64_t i = a + 1; i < b; ++i)
+        if (x->h_slope[i] > ss_max) ss_max = x->h_slope[i];
+      std::fill(x->link_in + 3 * n + a, x->link_in + 3 * n + b, ss_max);
+    }
   }
+  RegRout g;
+  for (int i = 0; i < 5; ++i) g.p[i] = p[i];
+  g.ts = (double)x->cfg.timestep;
+  const int64_t off = (int64_t)set * x->sstride;
+  CHECK_HIP(x, launch_reg_rout(x->link_in, n, x->link_order.pos, l0, l1, g, x->d_C1 + off,
+                               x->d_C2 + off, x->stream),
+            "reg_rout");
+  return MHMHIP_OK;
 }
 
 // A routed step with read_states = 0 evaluates reg_rout from the routing1
@@ -2063,26 +2095,21 @@ void reg_rout(const mhmhip_ctx *x, const double *p, int64_t l0, int64_t l1, doub
 // pairs already hold reg_rout's (or mrm_update_param's) values.
 int refresh_reg_rout(mhmhip_ctx *x) {
   for (int s = 0; s < x->n_sets; ++s) {
-    bool any = false;
-    for (int d = 0; d < x->n_domains; ++d) {
-      const size_t k = (size_t)s * x->n_domains + d;
-      if (!x->coef_restart[k] || x->ts_rout[k] > 0.0) continue;
-      if (x->dom_link_start[d + 1] <= x->dom_link_start[d]) continue;
-      if (!x->gam_set[k])
-        return x->fail(MHMHIP_EINVAL,
-                       "read_states = 0 recomputes C1/C2 by reg_rout from the routing "
-                       "parameters (mo_mrm_routing.f90:211-218): set them first, or route "
-                       "with read_states = 1 to keep the restart's C1/C2");
-      any = true;
-    }
-    if (!any) continue;
-    CHECK_RC(upload_coefs(x, s, [&](int d, int64_t l0, int64_t l1, double *c1, double *c2) {
-      const size_t k = (size_t)s * x->n_domains + d;
-      if (!x->coef_restart[k] || x->ts_rout[k] > 0.0) return false;
-      reg_rout(x, &x->gam5[k * 5], l0, l1, c1, c2);
-      x->coef_restart[k] = 0;
-      return true;
-    }));
+    for (int pass = 0; pass < 2; ++pass)  // all parameters known before any is used
+      for (int d = 0; d < x->n_domains; ++d) {
+        const size_t k = (size_t)s * x->n_domains + d;
+        if (!x->coef_restart[k] || x->ts_rout[k] > 0.0) continue;
+        const int64_t l0 = x->dom_link_start[d], l1 = x->dom_link_start[d + 1];
+        if (pass == 1) {
+          CHECK_RC(reg_rout(x, s, &x->gam5[k * 5], l0, l1));
+          x->coef_restart[k] = 0;
+        } else if (l1 > l0 && !x->gam_set[k]) {
+          return x->fail(MHMHIP_EINVAL,
+                         "read_states = 0 recomputes C1/C2 by reg_rout from the routing "
+                         "parameters (mo_mrm_routing.f90:211-218): set them first, or route "
+                         "with read_states = 1 to keep the restart's C1/C2");
+        }
+      }
   }
   return MHMHIP_OK;
 }
@@ -2098,17 +2125,16 @@ extern "C" int mhmhip_set_routing_params(mhmhip_ctx *x, int32_t set, int32_t dom
   CHECK_HIP(x, hipSetDevice(x->cfg.device), "set_routing_params");
   // The reference re-evaluates reg_rout every step with unchanged inputs
   // (mo_mrm_routing.f90:211-218); evaluating it once gives the same C1, C2.
-  CHECK_RC(upload_coefs(x, set, [&](int d, int64_t l0, int64_t l1, double *c1, double *c2) {
-    if (domain >= 0 && d != domain) return false;
+  for (int d = 0; d < x->n_domains; ++d) {
+    if (domain >= 0 && d != domain) continue;
     const size_t k = (size_t)set * x->n_domains + d;
     x->ts_rout[k] = 0.0;  // processCase 1
     for (int i = 0; i < 5; ++i) x->gam5[k * 5 + i] = p[i];
     x->gam_set[k] = 1;
     x->coef_restart[k] = 0;
-    reg_rout(x, p, l0, l1, c1, c2);
-    return true;
-  }));
-  return MHMHIP_OK;
+  }
+  return reg_rout(x, set, p, x->dom_link_start[domain >= 0 ? domain : 0],
+                  x->dom_link_start[domain >= 0 ? domain + 1 : x->n_domains]);
 }
 
 namespace {

@@ -299,6 +299,12 @@ struct MprLiteArgs {
   double gamma[kMprNGamma];
 };
 
+// reg_rout's parameters and time step [h].
+struct RegRout {
+  double p[5];
+  double ts;
+};
+
 // Extra arguments of the tiled routing kernels.
 struct TileArgs {
   const SlotMeta *slot;    // [n_bins * kTileSlots]; a proxy's pos: the upstream tile's root
