@@ -2755,11 +2755,16 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
   }
   const TileArgs g = tile_args(x);
   const bool graph = o.use_graph && o.mode == MHMHIP_RUN_FUSED;
-  // A captured fused run puts routing that leaves room on the chip, or comes
-  // in many launches, on a stream of its own beside the cell launches that
-  // follow.  One that fills the chip for a few launches waits instead until
-  // the ring is full or the call ends.
-  const bool two = graph && tiled && (!flow || groups <= 256);
+  // A captured run puts the routing on a stream of its own beside the cell
+  // launches that follow: the windowed launches as their windows fill, the
+  // one launch, where it leaves room on the chip, whenever half the steps that
+  // fill its chain (or half the ring) are there (a year of 64x64 12.1 -> 10.3
+  // ms, five horizons on 96x130 1.50 -> 1.40 ms).  Otherwise it waits until the
+  // ring is full or the call ends: outside a graph the waits between streams
+  // cost more than they hide (150x220, ten launches: 1.94 -> 2.12 ms).
+  const int64_t flush =  // steps that make a launch beside the cells
+      std::max<int64_t>(1, std::min<int64_t>(x->lay.dmax + 5 * x->lay.tau_max, ring_len) / 2);
+  const bool two = graph && tiled && (!flow || (groups <= 256 && nr > flush));
   if (two && !x->rstream)
     CHECK_HIP(x, hipStreamCreateWithFlags(&x->rstream, hipStreamNonBlocking), "routing stream");
   if (flow) CHECK_RC(flow_begin(x, "run"));
@@ -2835,7 +2840,7 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
       if (kind == MHMHIP_K_ROUTE_TILE && x->n_inflow > 0)
         CHECK_HIP(x, launch_inflow_patch(r, x->d_ring, x->d_lag, u0, u1, x->stream, rep),
                   "inflow_patch");
-      if (windows || (two && tiled)) CHECK_RC(route_to(u1));
+      if (windows || (two && u1 - routed >= flush)) CHECK_RC(route_to(u1));
       if (!tiled) CHECK_RC(route_diagonals(x, r, u0, u1, false, wg));
     }
     if (flow) CHECK_RC(route_to(nr));
