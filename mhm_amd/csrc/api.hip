@@ -1200,7 +1200,8 @@ extern "C" int mhmhip_set_meteo_weights(mhmhip_ctx *x, const double *pre_w,
 
 namespace {
 
-int make_step(mhmhip_ctx *x, const mhmhip_step &s, StepDev &d) {
+// prev: the step before, whose day's terms serve when the day is the same
+int make_step(mhmhip_ctx *x, const mhmhip_step &s, StepDev &d, const StepDev *prev = nullptr) {
   if (s.tt < 1 || s.month < 1 || s.month > 12 || s.hour < 0 || s.hour > 23 || s.doy < 1 ||
       s.doy > 366 || s.iMeteoTS < 1)
     return x->fail(MHMHIP_EINVAL, "step: tt/month/hour/doy/iMeteoTS out of range");
@@ -1212,12 +1213,19 @@ int make_step(mhmhip_ctx *x, const mhmhip_step &s, StepDev &d) {
                                       std::to_string(x->cfg.n_forcing_days) +
                                       " columns; stream the day first)");
   // mo_pet.f90:339-340, evaluated with the same libm as the reference
-  const double doy = (double)s.doy;
-  d.dr = 1.0 + 0.0330 * std::cos(kTwoPiD * doy / kYearDays);
-  const double delta = 0.4090 * std::sin(kTwoPiD * doy / kYearDays - 1.3900);
-  d.tand = std::tan(delta);
-  d.sind = std::sin(delta);
-  d.cosd = std::cos(delta);
+  if (prev && prev->doy == s.doy) {
+    d.dr = prev->dr;
+    d.tand = prev->tand;
+    d.sind = prev->sind;
+    d.cosd = prev->cosd;
+  } else {
+    const double doy = (double)s.doy;
+    d.dr = 1.0 + 0.0330 * std::cos(kTwoPiD * doy / kYearDays);
+    const double delta = 0.4090 * std::sin(kTwoPiD * doy / kYearDays - 1.3900);
+    d.tand = std::tan(delta);
+    d.sind = std::sin(delta);
+    d.cosd = std::cos(delta);
+  }
   d.day = col;
   d.month0 = s.month - 1;
   d.isday = (s.hour > 6) && (s.hour <= 18);  // mo_meteo_handler.f90:1048
@@ -2647,7 +2655,8 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
   CHECK_HIP(x, hipSetDevice(x->cfg.device), "run");
   if (route && !steps[0].read_states) CHECK_RC(refresh_reg_rout(x));
   std::vector<StepDev> hs(nsteps);
-  for (int32_t k = 0; k < nsteps; ++k) CHECK_RC(make_step(x, steps[k], hs[k]));
+  for (int32_t k = 0; k < nsteps; ++k)
+    CHECK_RC(make_step(x, steps[k], hs[k], k > 0 ? &hs[k - 1] : nullptr));
   // what each step changes: a step whose forcing column, day and day/night
   // factors (and, with meteo weights, month and hour) equal the step before's
   // has the same disaggregated meteo values (the fused kernel keeps them; its
