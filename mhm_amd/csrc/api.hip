@@ -226,7 +226,7 @@ struct mhmhip_ctx {
   // time loop captured as a hipGraph, replayed while its key matches
   struct GraphKey {
     int32_t nsteps = -1, mode = -1, S = -1, block = -1, wg = -1, prof = -1, B = -1, out_n = -1,
-            rep = -1;
+            rep = -1, sun = -1;
     uint64_t out_mask = 0;
     const void *ring = nullptr, *gauge = nullptr, *steps = nullptr, *inflow = nullptr,
                *qacc = nullptr, *out = nullptr, *cring = nullptr;
@@ -235,7 +235,8 @@ struct mhmhip_ctx {
       return nsteps == o.nsteps && mode == o.mode && S == o.S && block == o.block && wg == o.wg &&
              prof == o.prof && B == o.B && ring == o.ring && gauge == o.gauge && steps == o.steps &&
              inflow == o.inflow && qacc == o.qacc && ring_len == o.ring_len && out == o.out &&
-             out_n == o.out_n && out_mask == o.out_mask && rep == o.rep && cring == o.cring;
+             out_n == o.out_n && out_mask == o.out_mask && rep == o.rep && sun == o.sun &&
+             cring == o.cring;
     }
   };
   GraphKey gkey;
@@ -2775,6 +2776,14 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
     a.raw_total = 1;
   }
   const TileArgs g = tile_args(x);
+  // Sets of one cell share its days' sun terms (sun_kernel), kept in the flux
+  // rows until the call's last step, which becomes a launch of its own: where a
+  // day begins on most steps and at least four sets share a term.
+  int64_t days = 0;
+  for (const StepDev &d : hs) days += (d.change & SC_DAY) != 0;
+  const bool sun = o.mode == MHMHIP_RUN_FUSED && x->cfg.process_pet == 1 && x->n_sets >= 4 &&
+                   nsteps > 8 && 2 * days > nsteps && S <= 65535 &&
+                   2 * (int64_t)S <= x->n_xrows * x->n_sets;
   const bool graph = o.use_graph && o.mode == MHMHIP_RUN_FUSED;
   // A captured run puts the routing on a stream of its own beside the cell
   // launches that follow: the windowed launches as their windows fill, the
@@ -2828,8 +2837,9 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
       }
       return MHMHIP_OK;
     };
-    for (int32_t k = 0; k < nsteps; k += S) {
-      const int n = std::min<int32_t>(S, nsteps - k);
+    for (int32_t k = 0, n; k < nsteps; k += n) {
+      n = std::min<int32_t>(S, nsteps - k);
+      if (sun && k + n == nsteps && n > 1) --n;  // the last step writes the flux rows
       // the launch's routing steps [u0, u1), whose rows held those of
       // ring_len steps before
       const int64_t u0 = (int64_t)k * rep, u1 = (int64_t)(k + n) * rep;
@@ -2846,6 +2856,13 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
                   }),
                   "cell_step");
       } else {
+        // only the call's last step leaves its fluxes (1024x1024 cells, ten
+        // launches: 15.8 -> 15.6 ms); the rows hold the sun terms of launches
+        // before that step's
+        a.skip_fluxes = k + n < nsteps;
+        a.sun = sun && a.skip_fluxes ? x->X : nullptr;
+        a.sun_step0 = k;
+        if (a.sun) CHECK_HIP(x, launch_sun(a, k, n, x->X, x->stream), "sun");
         CHECK_HIP(x, timed(x, MHMHIP_K_CELL_FUSED, (double)x->n_cells * x->n_sets * n, [&] {
                     return launch_cell_fused(x->nh, a, k, n, k, block, x->n_sets, x->stream);
                   }),
@@ -2892,6 +2909,7 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
     key.out_n = a.out.sum ? a.out.n : 0;
     key.out_mask = a.out.sum ? a.out.mask : 0;
     key.rep = rep;
+    key.sun = sun;
     key.cring = route && x->coarse ? x->d_cring : nullptr;
     if (!x->graph_exec || !(key == x->gkey)) {
       drop_graph(x);

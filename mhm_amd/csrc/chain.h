@@ -762,19 +762,34 @@ __device__ __forceinline__ bool ordinary_states(double pack, double unsat, doubl
 // value within a few ulp (the factored form keeps its relative accuracy as
 // arg nears +-1), for a square root instead of a sine's range reduction and
 // series.
-__device__ MHMHIP_OUTLINE double pet_hargreaves(double coeff, double tavg, double tmax,
-                                                 double tmin, double tanlat, double sinlat,
-                                                 double coslat, double dr, double tand,
-                                                 double sind, double cosd) {
+//
+// The sun's part of it, the same for every parameter set: extraterrestrial
+// radiation and sqrt(tmax - tmin), the latter -1 where the PET is 0.
+struct SunTerms {
+  double ra, sq;
+};
+__device__ __forceinline__ SunTerms sun_terms(double tavg, double tmax, double tmin, double tanlat,
+                                              double sinlat, double coslat, double dr, double tand,
+                                              double sind, double cosd) {
   const double dT = tmax - tmin;
-  if (le_eps(dT, 0.0) || le_eps(tavg, -kHarSamConst)) return 0.0;
+  if (le_eps(dT, 0.0) || le_eps(tavg, -kHarSamConst)) return {0.0, -1.0};
   double arg = -tanlat * tand;
   if (arg < -1.0) arg = -1.0;
   if (arg > 1.0) arg = 1.0;
   const double omega = acos(arg);
   const double sin_omega = sqrt((1.0 - arg) * (1.0 + arg));
   const double ra = kRadConst * dr * (omega * sinlat * sind + coslat * cosd * sin_omega);
-  return coeff * ra * (tavg + kHarSamConst) * sqrt(dT);
+  return {ra, sqrt(dT)};
+}
+__device__ __forceinline__ double pet_of_sun(double coeff, double tavg, SunTerms t) {
+  return t.sq < 0.0 ? 0.0 : coeff * t.ra * (tavg + kHarSamConst) * t.sq;
+}
+__device__ MHMHIP_OUTLINE double pet_hargreaves(double coeff, double tavg, double tmax,
+                                                 double tmin, double tanlat, double sinlat,
+                                                 double coslat, double dr, double tand,
+                                                 double sind, double cosd) {
+  return pet_of_sun(coeff, tavg, sun_terms(tavg, tmax, tmin, tanlat, sinlat, coslat, dr, tand,
+                                           sind, cosd));
 }
 
 // FORCES mo_constants: DaySecs, SpecHeatET_dp, Psychro_dp, rho0_dp, cp0_dp, T0_dp;

@@ -142,6 +142,11 @@ struct CellArgs {
   double nT;               // steps per day as real (nTstepDay_dp)
   double rnT;              // RN(1 / nT)
   OutAcc out;              // output sums (out.sum null: none)
+  // the days' sun terms of this launch's steps (sun_kernel), null: each lane
+  // evaluates its own
+  const double *sun;
+  int32_t sun_step0;       // step of its first pair of rows
+  int32_t skip_fluxes;     // 1: a later launch of the call writes the flux rows
   // meteo weights [3][12 * 24][sstride] (pre, temp, pet), null: the day/night
   // factors disaggregate
   const double *W;

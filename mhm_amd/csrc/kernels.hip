@@ -90,6 +90,7 @@ __device__ __forceinline__ CellArgs read_args(ConstArgs *p) {
   a.forcing_days = p->forcing_days, a.ring_len = p->ring_len, a.pet_case = p->pet_case;
   a.jarvis = p->jarvis, a.hourly = p->hourly, a.ring_rep = p->ring_rep;
   a.raw_total = p->raw_total, a.nT = p->nT, a.rnT = p->rnT, a.W = p->W;
+  a.sun = p->sun, a.sun_step0 = p->sun_step0, a.skip_fluxes = p->skip_fluxes;
   return a;
 }
 
@@ -701,6 +702,7 @@ struct FusedLane {
   double scale;        // runoff_scale
   double *ring;        // ring row 0 of the node (its lag folded in), null: no routing
   int64_t roff;        // element offset of the step's first ring row
+  int32_t sun;         // 1: the wave reads its days' sun terms (sun_kernel)
 };
 
 // The step's qOUT to its rep ring rows.
@@ -726,13 +728,23 @@ __device__ __forceinline__ void disagg_at(const CellArgs &a, const StepDev &st, 
 }
 
 // The daily PET into its slot, out of line and from its own loads: the time
-// loop around it holds no register for it.
+// loop around it holds no register for it.  shared: the sun terms are there.
 template <int NH>
 __device__ __attribute__((noinline)) void day_pet(ConstArgs *args, uint32_t bc, uint32_t bv,
-                                                  uint32_t slot, const ConstStep *step) {
+                                                  uint32_t slot, const ConstStep *step,
+                                                  int32_t shared) {
   const CellArgs a = read_args(uniform(args));
-  const StepDev st = read_step((const ConstStep *)uniform((ConstArgs *)step));
+  const ConstStep *p = (const ConstStep *)uniform((ConstArgs *)step);
+  const StepDev st = read_step(p);
   const double tavg = ldr(frow_ptr(a, MHMHIP_F_TAVG, st.day), bc);
+  if (__builtin_amdgcn_readfirstlane(shared)) {
+    auto P = [&](int r) { return ldr(a.P + (int64_t)r * a.ld, bv); };
+    const int32_t i = (int32_t)(p - (const ConstStep *)a.steps) - a.sun_step0;
+    const double *row = a.sun + (int64_t)(2 * i) * a.sstride;
+    const SunTerms t{ldr(row, bc), ldr(row + a.sstride, bc)};
+    s_lane[slot + LS_PD] = P(PR_FASP) * pet_of_sun(P(PR_HARSAM), tavg, t);
+    return;
+  }
   const double tmax = a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMAX, st.day), bc) : 0.0;
   const double tmin = a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMIN, st.day), bc) : 0.0;
   s_lane[slot + LS_PD] = pet_day<NH>(a, st, bv, bc, tavg, tmax, tmin);
@@ -744,7 +756,7 @@ __device__ __attribute__((noinline)) void day_pet(ConstArgs *args, uint32_t bc, 
 template <int NH>
 __device__ __forceinline__ void look_up(ConstArgs *k, const FusedLane &u, const ConstStep *p,
                                         int change, bool ordinary) {
-  if (change & SC_DAY) day_pet<NH>(k, u.bc, u.bv, u.slot, p);
+  if (change & SC_DAY) day_pet<NH>(k, u.bc, u.bv, u.slot, p, u.sun);
   const CellArgs a = read_args(rare(k));
   const StepDev st = read_step(p);
   // offsets opaque here: no per-lane address of these rows is held across
@@ -813,6 +825,38 @@ __device__ __forceinline__ Stress<NH> read_stress(uint32_t li) {
   return t;
 }
 
+// Sun terms of the steps step0 .. of a launch that begin a day (and of its
+// first), per cell: rows 2 i and 2 i + 1 of sun hold ra and sq of step
+// step0 + i.  With daily steps each lane's own were a third of a step's
+// instructions, the same for every set of a cell: 256 sets of 4096 cells, 1095
+// days, 23.7 -> 19.9 ms with every set's lanes reading them (they come from L2:
+// a step's rows are 64 KB).
+__global__ __launch_bounds__(256) void sun_kernel(CellArgs a, int32_t step0, double *sun) {
+  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
+  const StepDev st = a.steps[step0 + i];
+  if (c >= a.n_cells || !(i == 0 || (st.change & SC_DAY))) return;
+  const uint32_t bc = c * 8u;
+  auto P = [&](int r) { return ldr(a.P + (int64_t)r * a.ld, bc); };
+  const SunTerms t = sun_terms(ldr(frow_ptr(a, MHMHIP_F_TAVG, st.day), bc),
+                               ldr(frow_ptr(a, MHMHIP_F_TMAX, st.day), bc),
+                               ldr(frow_ptr(a, MHMHIP_F_TMIN, st.day), bc), P(PR_TANLAT),
+                               P(PR_SINLAT), P(PR_COSLAT), st.dr, st.tand, st.sind, st.cosd);
+  double *row = sun + (int64_t)(2 * i) * a.sstride;
+  str(row, bc, t.ra);
+  str(row + a.sstride, bc, t.sq);
+}
+
+// Whether the wave's cells have set 0's latitude, whose sun terms sun holds.
+__device__ __forceinline__ bool shares_sun(const CellArgs &a, uint32_t bc, uint32_t bv) {
+  if (!a.sun) return false;
+  bool same = true;
+  for (int r : {PR_TANLAT, PR_SINLAT, PR_COSLAT}) {
+    const double *row = a.P + (int64_t)r * a.ld;
+    same = same & (__double_as_longlong(ldr(row, bc)) == __double_as_longlong(ldr(row, bv)));
+  }
+  return __all(same);
+}
+
 // The lane's slots and its place in the ring: the lane's row offset (its lag)
 // is fixed, the step's row uniform.
 template <int NH, bool JV>
@@ -822,6 +866,7 @@ __device__ __forceinline__ void fused_lane(const CellArgs &a, uint32_t c, uint32
   u.bc = c * 8u;
   u.bv = bv;
   u.slot = slot;
+  u.sun = shares_sun(a, u.bc, bv);
 #pragma unroll
   for (int h = 0; h < NH; ++h) {
     s_lane[slot + LS_STRESS + h] = t.fr[h];
@@ -857,6 +902,7 @@ __device__ __forceinline__ void fused_ordinary(const CellArgs &a, FusedLane &u, 
   if (OUT) load_sums(k, a.ld, u.bv, u.slot + LS_STRESS + stress_slots(NH, JV));
   const int rep = a.ring_rep;
   const int64_t wrap = a.ring_len * a.ld;
+  const int32_t flux_at = a.skip_fluxes ? -2 : nsteps - 1;  // step whose fluxes are stored
   // exponents in units of 1/256 (pow_v)
   const double alpha256 = 256.0 * (1.0 + r.alpha), rc1 = JV ? 1.0 / r.c1 : 0.0;
 #pragma unroll
@@ -877,10 +923,10 @@ __device__ __forceinline__ void fused_ordinary(const CellArgs &a, FusedLane &u, 
       const uint32_t li = opaque(u.slot);
       ordinary_soil<NH, JV>(r, x, demand, s_lane[li + LS_XPE], ecan, peff, wet, pwh.v, rc1,
                             read_stress<NH, JV>(li));
-      if (last || OUT) {
+      if (s == flux_at || OUT) {
         FluxRegs<NH> y = x;
         report_sealed<NH>(r, y);
-        if (last) store_fluxes_soil<NH>(read_args(rare(k)), u.bv, y);
+        if (s == flux_at) store_fluxes_soil<NH>(read_args(rare(k)), u.bv, y);
         if (OUT) {
           o = opaque(u.slot) + LS_STRESS + stress_slots(NH, JV) + n_canopy;
           outputs_soil<NH>(r, y, ecan, out_slots(mask, o));
@@ -907,7 +953,7 @@ __device__ __forceinline__ void fused_ordinary(const CellArgs &a, FusedLane &u, 
       x.prec = s_lane[li + LS_XPREC];
       ordinary_canopy<NH>(r, x, s_lane[li + LS_XMELT], s_lane[li + LS_XCOLD],
                           s_lane[li + LS_MAXI], s_lane[li + LS_RMAXI]);
-      if (s + 2 == nsteps) {
+      if (s + 1 == flux_at) {
         last_meteo<NH>(k, u, next, x);
         store_fluxes_canopy<NH>(read_args(rare(k)), u.bv, x);
       }
@@ -940,7 +986,7 @@ __device__ __forceinline__ void fused_ordinary(const CellArgs &a, FusedLane &u, 
     if (s >= 0) {
       ordinary_post<NH>(r, x, pw_slow, x.rseal);
       put_ring(a, u, wrap, rep, x.total);
-      if (last) store_fluxes_post<NH>(read_args(rare(k)), u.bv, x);
+      if (s == flux_at) store_fluxes_post<NH>(read_args(rare(k)), u.bv, x);
       if (OUT) outputs_post<NH>(r, x, out_slots(mask, o));
     }
   }
@@ -990,7 +1036,7 @@ __device__ __attribute__((noinline)) void fused_general(ConstArgs *args, uint32_
     x.prec = s_lane[li + LS_XPREC];
     chain_step<NH, JV>(r, x, s_lane[li + LS_MAXI], s_lane[li + LS_RMAXI], p->evap, p->revap, t);
     put_ring(a, u, wrap, rep, x.total);
-    if (s == nsteps - 1) store_fluxes<NH>(a, u.bv, x);
+    if (s == nsteps - 1 && !a.skip_fluxes) store_fluxes<NH>(a, u.bv, x);
     if (OUT) add_outputs<NH>(k, a.ld, u.bv, r, x);
   }
   store_states<NH>(a, bv, r);
@@ -2228,6 +2274,13 @@ hipError_t launch_cell_fused(int nh, const CellArgs &a, int64_t t0, int nsteps, 
     case 6: return fused_nh<6>(a, t0, nsteps, step0, block, n_sets, s);
   }
   return hipErrorInvalidValue;
+}
+
+hipError_t launch_sun(const CellArgs &a, int step0, int nsteps, double *sun, hipStream_t s) {
+  if (nsteps < 1 || nsteps > 65535 || a.pet_case != 1) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(sun_kernel, dim3((unsigned)((a.n_cells + 255) / 256), (unsigned)nsteps),
+                     dim3(256), 0, s, a, step0, sun);
+  return hipGetLastError();
 }
 
 hipError_t launch_route_diag(const RouteArgs &r, int64_t d, int64_t p_lo, int64_t p_hi,

@@ -26,6 +26,7 @@ hipError_t launch_inflow_patch(const RouteArgs &r, double *ring, const uint8_t *
 hipError_t launch_meteo_l2(const double *data2, const uint8_t *mask2, int32_t nr2, int64_t n2,
                            const MeteoL2Cell *cells, int64_t ncells, int32_t ndays, double *F,
                            int64_t day_stride, bool aggregate, hipStream_t s);
+hipError_t launch_sun(const CellArgs &a, int step0, int nsteps, double *sun, hipStream_t s);
 hipError_t launch_reg_rout(const double *in, int64_t n, const int32_t *pos, int64_t l0, int64_t l1,
                            const RegRout &g, double *C1, double *C2, hipStream_t s);
 hipError_t launch_state_rows(double *S, const StateValues &v, int32_t n_rows, int64_t n_cells,
