@@ -54,8 +54,9 @@ def bytes_per_unit(kernel, steps_per_launch, steps_per_forcing, window=16, sets_
     if kernel == "cell_fused":
         # forcing once per forcing column, shared by the sets (32/(F n_sets)), qOUT
         # to the ring every step (8); once per launch: params 256 + states 64 +
-        # ring lag 1 read, states 64 + 23 fluxes 184 written (569/S)
-        return 32.0 / (steps_per_forcing * sets_sharing) + 8.0 + 569.0 / steps_per_launch
+        # ring lag 1 read, states 64 written (385/S); the 23 fluxes 184 written
+        # once per call are not counted
+        return 32.0 / (steps_per_forcing * sets_sharing) + 8.0 + 385.0 / steps_per_launch
     if kernel == "route_tile":
         # node-step: qOUT from the ring 8; once per window of B steps: slot metadata
         # 16, C1 + C2 16, qTIN read + write 16, qTR read + write 16
@@ -348,11 +349,11 @@ def bench_serving(serve, n_req, qps, pool, seed=11):
 
 def pmc_workload(args):
     """Short run for counter collection: the headline kernels on the same
-    basin (2 plain steps, then 6 fused launches routed in the headline's
+    basin (2 plain steps, then the headline's 15 fused launches routed in its
     windows), then a plain device copy of COPY_CALIB_BYTES."""
     import torch
     from mhm_amd import _native as N, workloads
-    n_steps = 2 + 6 * args.steps_per_launch  # 2 plain steps, then whole fused launches
+    n_steps = 2 + 15 * args.steps_per_launch  # 2 plain steps, then whole fused launches
     model, steps, dom, _ = workloads.plain_domain(args.grid, args.grid, n_steps, seed=1)
     model.run(steps[:2], mode=N.RUN_PLAIN)
     model.run(steps[2:], mode=N.RUN_FUSED, steps_per_launch=args.steps_per_launch,
