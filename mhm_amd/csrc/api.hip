@@ -2521,7 +2521,7 @@ extern "C" int mhmhip_mrm_step(mhmhip_ctx *x, const mhmhip_step *st, double *gau
   // the kernel writes a step's gauges straight to pinned host memory: a copy
   // costs 8 us more
   double *pinned = nullptr;
-  if (loops == 1 && gauge_out && ng > 0 && ng <= x->sstride) CHECK_RC(stage_take(x, &pinned));
+  if (loops == 1 && gauge_out && ng > 0 && ng <= x->n_cells) CHECK_RC(stage_take(x, &pinned));
   auto enqueue = [&](int32_t it) -> int {
     RouteArgs r = route_args(x, 0, 1, 0);
     if (pinned) r.gauge_out = pinned;
