@@ -627,10 +627,11 @@ int host_order(mhmhip_ctx *x, mhmhip_ctx::HostOrder &o, int64_t n, Fn fill) {
   return MHMHIP_OK;
 }
 
-// n values of a device row in the reference's order (host_order) to the host: gathered on the device into a pinned staging row
-// and copied from there.  A row of 64k values or more is split, so that the
-// host copies one part while the next ones cross the link (1M cells: 340 us
-// with 8 parts, 470 with one; at 65k cells 34 and 36).
+// n values of a device row in the reference's order (host_order) to the host:
+// gathered on the device into a pinned staging row and copied from there.  A
+// row of 128k values or more is split, so that the host copies one part while
+// the next ones cross the link (1M cells: 340 us with 8 parts, 470 with one;
+// at 65k cells two parts gain nothing: 33 against 35).
 template <typename Fn>
 int get_ordered(mhmhip_ctx *x, const double *srcdev, mhmhip_ctx::HostOrder &o, int64_t n, Fn fill,
                 double *dst) {
@@ -1435,8 +1436,8 @@ int flow_check(mhmhip_ctx *x, const char *who) {
 //     chip full 0.39e-3 per workgroup and diagonal besides those 8.
 // Measured, workgroups and steps: one launch / windows [us]: 59 x 480 (B 32)
 // 139 / 294, 296 x 720 (8) 579 / 979, 152 x 960 (8) 936 / 1504, 20 x 8760 (64)
-// 2034 / 2636, 1474 x 720 (64) 840 / 955, 2833 x 48 (8) 509 / 781, 4693 x 1440 (64) 4912 / 4305, 5120 x 1095
-// (64) 6365 / 3211.
+// 2034 / 2636, 1474 x 720 (64) 840 / 955, 2833 x 48 (8) 509 / 781, 4693 x 1440
+// (64) 4912 / 4305, 5120 x 1095 (64) 6365 / 3211.
 bool one_launch_pays(const mhmhip_ctx *x, int32_t B, int64_t nr, int64_t ring_rows) {
   const double groups = (double)x->lay.bins.size() * x->n_sets, H = x->tile_h;
   const double fills = std::ceil((double)nr / (double)std::max<int64_t>(1, ring_rows));
@@ -1926,7 +1927,8 @@ extern "C" int mhmhip_bind_network(mhmhip_ctx *x, const mhmhip_network *net) {
   for (size_t i = 0; i < lay.slots.size(); ++i) {
     const SlotMeta &m = lay.slots[i];
     if (!(m.a & SF_TROOT)) continue;
-    if (nm_nchild(lay.packed[m.pos]) < 1) return x->fail(MHMHIP_EINVAL, "bind_network: tile partition failed");
+    if (nm_nchild(lay.packed[m.pos]) < 1)
+      return x->fail(MHMHIP_EINVAL, "bind_network: tile partition failed");
     spare[i] = lay.child_list[lay.child[m.pos]];
     root[m.bnd] = m.pos;
   }
@@ -2798,6 +2800,7 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
   if (two && !x->rstream)
     CHECK_HIP(x, hipStreamCreateWithFlags(&x->rstream, hipStreamNonBlocking), "routing stream");
   if (flow) CHECK_RC(flow_begin(x, "run"));
+  if (windows) x->flow_ready = false;  // they write d_bnd
   const WindowArgs win = window_args(x, B, nr);
   const int32_t L_end = win.nwin + win.tau_max;
   // the whole loop, in steps relative to this call (replayable as a graph)
@@ -2934,7 +2937,6 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
   }
   if (route) {
     credit_route(x, kind, nr);
-    if (windows) x->flow_ready = false;
     x->qtr_slot = (int)((nr - 1) & 1);
     if (x->qacc_on) x->qacc_count += nsteps;
     x->qsub_loops = rep;
