@@ -197,11 +197,12 @@ __host__ __device__ inline DV<N> exp_fin_v(const DV<N> &zin) {
 
 // x**y for x > 0 as 2^(y log2 x), N pairs at once, table-driven (Tang's
 // method for both halves, in base 2): x = m 2^e (frexp), the row of m's
-// interval gives R and L = -log2 R (one double: R is chosen for it),
-// u = m R - 1 (one fma; |u| <= 1/128) and
-//   log2 x = e + L + u (c0 + ... + c5 u^5);
-// with y256 = 256 y, z = 256 y log2 x as y256 e + (y256 L + y256 (u ...)), two
-// fma, n = RN(z), r = z - n (exact, |r| <= 1/2):
+// interval gives R and L = -log2 R (R is chosen so that L is a multiple of
+// 2^-42), u = m R - 1 (one fma; |u| <= 1/128) and
+//   log2 x = (e + L) + u (c0 + ... + c5 u^5)
+// with e + L exact: where e and L cancel (x just above 1) nothing of the size
+// of y is rounded.  With y256 = 256 y, z = 256 y log2 x as y256 (e + L) +
+// y256 (u ...), one fma, n = RN(z), r = z - n (exact, |r| <= 1/2):
 //   x**y = 2^(n >> 8) 2^((n & 255)/256) (1 + r (d0 + ... + d3 r^3)),
 // the table's 2^(j/256) as hi + lo.  Working in units of 1/256 of a binary
 // logarithm leaves no multiplication by ln 2 or 256/ln 2 and makes the
@@ -209,8 +210,9 @@ __host__ __device__ inline DV<N> exp_fin_v(const DV<N> &zin) {
 // power on gfx950, where exp(y log x) took 37 and three.  The rows on either
 // side of x = 1 hold R = 2 and R = 1 with exact logarithms, so 1**y is 1.
 // Within (2 + 3 |y log x|) ulp of the exact power (the rounding of z,
-// amplified by the exponential); over the chain's arguments 1.3 to 1.5 ulp
-// rms against mpmath, where exp(y log x) with two such roundings had 1.7 to 1.9.
+// amplified by the exponential); against mpmath 1.2 to 1.5 ulp rms over the
+// chain's arguments (exp(y log x) had 1.7 to 1.9) and at most 2.2 ulp for x in
+// (1, 1.05], y up to 65 (43 when e and L were added after their products with y).
 // Phases run over all N values, the loads of a phase's table rows together,
 // so that N independent chains interleave and each phase waits for LDS once.
 template <int N>
@@ -239,7 +241,7 @@ __host__ __device__ __forceinline__ DV<N> pow_v(const DV<N> &y256, const DV<N> &
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     const double y = y256.v[i];
-    z.v[i] = fma(y, (double)e[i], fma(y, hi.v[i], y * (p.v[i] * u.v[i])));
+    z.v[i] = fma(y, (double)e[i] + hi.v[i], y * (p.v[i] * u.v[i]));
   }
   const char *etab = reinterpret_cast<const char *>(exptab());
 #pragma unroll

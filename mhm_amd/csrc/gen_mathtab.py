@@ -16,14 +16,16 @@ Power (pow_v in chain.h): base-2 logarithm rows {R, L} for j = 0..127, one per
 interval [(128 + j)/256, (129 + j)/256) of the frexp mantissa m: R near the
 reciprocal of the interval's middle, u = m R - 1 and log2(m) = L +
 log2(1 + u).  R is searched next to that reciprocal so that L = -log2(R) lies
-within 2^-10 of half a unit of a double's last place (the accurate tables of
-Gal, in "Computing elementary functions: a new approach for achieving high
-accuracy and good performance", LNCS 235 (1986) 1-16): one double holds it.
-The first row has R = 2 and the last R = 1, both with exact logarithms, so
-that log2 x is 0 at x = 1.  Then 2^(j/256) as above, and the coefficients of
-log2(1 + u) = u (c0 + ... + c5 u^5) on [-1/256, 1/128] and of
+within 2^-66 of a multiple of 2^-42 (the accurate tables of Gal, in "Computing
+elementary functions: a new approach for achieving high accuracy and good
+performance", LNCS 235 (1986) 1-16): one double holds it, and e + L is exact
+for the exponent e of every finite double, also where the two nearly cancel (x
+just above 1).  The first row has R = 2 and the last R = 1, both with exact
+logarithms, so that log2 x is 0 at x = 1.  Then 2^(j/256) as above, and the
+coefficients of log2(1 + u) = u (c0 + ... + c5 u^5) on [-1/256, 1/128] and of
 2^(r/256) = 1 + r (d0 + ... + d3 r^3) on [-1/2, 1/2], interpolated at Chebyshev
-nodes (relative errors below 2^-52 and 2^-58).
+nodes; main() checks that log2(1 + u) and 2^(r/256) come out with relative
+errors below 2^-51.8 and 2^-57.5.
 
 Values from mpmath at 256 bits.
 Run: python mhm_amd/csrc/gen_mathtab.py > mhm_amd/csrc/mathtab.h
@@ -60,12 +62,16 @@ def pow_row(j):
         return 2.0, -1.0
     if j == 127:
         return 1.0, 0.0
-    R = float(mp.mpf(512) / (2 * (128 + j) + 1))
-    while True:
-        L = -mp.log(mp.mpf(R), 2)
-        if abs(L - mp.mpf(float(L))) < math.ulp(float(L)) * mp.mpf(2) ** -11:
-            return R, float(L)
-        R = math.nextafter(R, 2.0)
+    # the grid's logarithms from the reciprocal's on, their powers of 2 a
+    # factor apart: the first that a double meets to 2^-66 in the logarithm
+    g = math.floor(mp.ldexp(-mp.log(mp.mpf(512) / (2 * (128 + j) + 1), 2), 42))
+    want, step = mp.power(2, mp.ldexp(-g, -42)), mp.power(2, mp.ldexp(1, -42))
+    with mp.workprec(128):
+        while abs(mp.mpf(float(want)) / want - 1) * mp.log(mp.e, 2) > mp.ldexp(1, -66):
+            g, want = g - 1, want * step
+    R, L = float(want), math.ldexp(g, -42)
+    assert abs(mp.log(mp.mpf(R), 2) + mp.mpf(L)) < mp.ldexp(1, -66) * 1.001
+    return R, L
 
 
 def chebyshev_fit(f, a, b, n):
@@ -80,6 +86,18 @@ def chebyshev_fit(f, a, b, n):
         for k in range(n):
             A[i, k] = x[i] ** k
     return [float(c) for c in mp.lu_solve(A, y)]
+
+
+def worst_error(f, c, c0, a, b):
+    """Largest relative error of c0 + t (c[0] + c[1] t + ...) against f over a
+    grid of [a, b]."""
+    worst = mp.mpf(0)
+    for i in range(2001):
+        t = a + (b - a) * i / 2000
+        if f(t) != 0:
+            p = c0 + t * mp.polyval([mp.mpf(v) for v in reversed(c)], t)
+            worst = max(worst, abs(p / f(t) - 1))
+    return worst
 
 
 def main():
@@ -113,8 +131,11 @@ def main():
         hi, lo = exp_row(j)
         print("    %s, %s," % (hi.hex(), lo.hex()))
     print("};")
-    c = chebyshev_fit(lambda u: mp.log(1 + u, 2) / u, mp.mpf(-1) / 256, mp.mpf(1) / 128, 6)
-    d = chebyshev_fit(lambda r: (mp.power(2, r / 256) - 1) / r, mp.mpf(-1) / 2, mp.mpf(1) / 2, 4)
+    half, u0, u1 = mp.mpf(1) / 2, -mp.mpf(1) / 256, mp.mpf(1) / 128
+    c = chebyshev_fit(lambda u: mp.log(1 + u, 2) / u, u0, u1, 6)
+    d = chebyshev_fit(lambda r: (mp.power(2, r / 256) - 1) / r, -half, half, 4)
+    assert worst_error(lambda u: mp.log(1 + u, 2), c, 0, u0, u1) < mp.power(2, -51.8)
+    assert worst_error(lambda r: mp.power(2, r / 256), d, 1, -half, half) < mp.power(2, -57.5)
     print("// log2(1 + u) / u and (2^(r/256) - 1) / r, constant term first")
     print("constexpr double kPowC[6] = {%s};" % ", ".join(v.hex() for v in c))
     print("constexpr double kPowD[4] = {%s};" % ", ".join(v.hex() for v in d))
