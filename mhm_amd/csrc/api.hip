@@ -339,6 +339,29 @@ static hipError_t sync_copy(mhmhip_ctx *x, void *dst, const void *src, size_t n,
 }
 
 // ---------------------------------------------------------------------------
+namespace {
+int64_t forcing_values(const mhmhip_ctx *x) {
+  return (int64_t)x->n_frows * x->cfg.n_forcing_days * x->sstride;
+}
+
+// The word after the forcing columns: not 0 once forcing, weights or factors
+// outside the usual ranges were given (CellArgs::odd_weather).  It stays, also
+// when they are replaced: launches then look at their steps' weather.
+int32_t *odd_weather(const mhmhip_ctx *x) {
+  return reinterpret_cast<int32_t *>(x->F + forcing_values(x));
+}
+
+// After n columns of a variable from col on were written on stream s.
+int scan_forcing(mhmhip_ctx *x, int32_t var, int32_t col, int32_t n, hipStream_t s) {
+  if (var != MHMHIP_F_PRE && var != MHMHIP_F_TAVG) return MHMHIP_OK;
+  const double *rows =
+      x->F + ((int64_t)x->frow[var] * x->cfg.n_forcing_days + col) * x->sstride;
+  const hipError_t e = launch_forcing_scan(rows, x->sstride, n, x->n_cells,
+                                           var == MHMHIP_F_TAVG, odd_weather(x), s);
+  return e == hipSuccess ? MHMHIP_OK : x->hipfail(e, "forcing scan");
+}
+}  // namespace
+
 extern "C" int mhmhip_create(const mhmhip_config *cfg, mhmhip_ctx **out) {
   if (!cfg || !out) {
     g_create_error = "create: null argument";
@@ -452,11 +475,19 @@ extern "C" int mhmhip_create(const mhmhip_config *cfg, mhmhip_ctx **out) {
   if ((rc = x->dalloc(&x->P, x->n_prows * x->ld, "alloc params")) ||
       (rc = x->dalloc(&x->S, x->n_srows * x->ld, "alloc states")) ||
       (rc = x->dalloc(&x->X, x->n_xrows * x->ld, "alloc fluxes")) ||
-      (rc = x->dalloc(&x->F, (int64_t)x->n_frows * c.n_forcing_days * x->sstride,
-                      "alloc forcing"))) {
+      (rc = x->dalloc(&x->F, forcing_values(x) + 1, "alloc forcing"))) {  // and odd_weather
     g_create_error = x->err;
     mhmhip_destroy(x);
     return rc;
+  }
+  bool usual = true;  // day and night shares of the precipitation, temperature shifts
+  for (int m = 0; m < 12; ++m)
+    usual = usual && c.fnight_prec[m] >= 0.0 && c.fnight_prec[m] <= 1.0 &&
+            std::isfinite(c.fnight_temp[m]);
+  if (!usual && hipMemsetAsync(odd_weather(x), 1, sizeof(int32_t), x->stream) != hipSuccess) {
+    g_create_error = "create: setting the weather word failed";
+    mhmhip_destroy(x);
+    return MHMHIP_EHIP;
   }
   if (hipHostMalloc((void **)&x->stage,
                     sizeof(double) * (x->sstride * mhmhip_ctx::kStageSlots + 1),
@@ -947,6 +978,12 @@ extern "C" int mhmhip_stream_forcing(mhmhip_ctx *x, int32_t day0, int32_t ndays,
     CHECK_HIP(x, launch_forcing_gather(x->fstage_d[i], map, ndays, x->n_cells, x->d_pos, x->F, nfd,
                                        day0 - 1, x->sstride, x->cstream),
               "stream_forcing gather");
+  const int32_t col0 = (day0 - 1) % nfd, n0 = std::min(ndays, nfd - col0);
+  for (int32_t v : {MHMHIP_F_PRE, MHMHIP_F_TAVG})
+    if (host[v]) {
+      CHECK_RC(scan_forcing(x, v, col0, n0, x->cstream));
+      CHECK_RC(scan_forcing(x, v, 0, ndays - n0, x->cstream));
+    }
   hipEvent_t done = nullptr;
   CHECK_HIP(x, hipEventCreateWithFlags(&done, hipEventDisableTiming), "stream_forcing event");
   x->chunk_ev.push_back(done);
@@ -976,6 +1013,7 @@ extern "C" int mhmhip_set_forcing(mhmhip_ctx *x, int32_t var, int32_t day0, int3
         x->F + ((int64_t)x->frow[var] * x->cfg.n_forcing_days + (day0 - 1 + j)) * x->sstride;
     CHECK_RC(put_row(x, dst, host + (int64_t)j * ld, id));
   }
+  CHECK_RC(scan_forcing(x, var, day0 - 1, ndays, x->stream));
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "set_forcing");
   return MHMHIP_OK;
 }
@@ -1106,6 +1144,7 @@ extern "C" int mhmhip_set_forcing_l2(mhmhip_ctx *x, int32_t var, int32_t domain,
   double *dst = x->F + ((int64_t)x->frow[var] * x->cfg.n_forcing_days + (day0 - 1)) * x->sstride;
   CHECK_HIP(x, launch_meteo_l2(b.data2, b.mask2, nr2, n2, b.cells, ncells, ndays, dst, x->sstride,
                                aggregate, x->stream), "set_forcing_l2 map");
+  CHECK_RC(scan_forcing(x, var, day0 - 1, ndays, x->stream));
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "set_forcing_l2");
   return MHMHIP_OK;
 }
@@ -1193,6 +1232,10 @@ extern "C" int mhmhip_set_meteo_weights(mhmhip_ctx *x, const double *pre_w,
       for (int h = 0; h < 24; ++h)
         CHECK_RC(put_row(x, x->W + ((int64_t)v * 288 + m * 24 + h) * x->sstride,
                          host[v] + ld * ((int64_t)m + 12 * h), id));
+  for (int v = 0; v < 2; ++v)  // precipitation, temperature
+    CHECK_HIP(x, launch_forcing_scan(x->W + (int64_t)v * 288 * x->sstride, x->sstride, 288,
+                                     x->n_cells, v == 1, odd_weather(x), x->stream),
+              "set_meteo_weights");
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "set_meteo_weights");
   return MHMHIP_OK;
 }
@@ -1250,6 +1293,7 @@ CellArgs cell_args(mhmhip_ctx *x, bool ring) {
   a.S = x->S;
   a.X = x->X;
   a.F = x->F;
+  a.odd_weather = odd_weather(x);
   a.ring = ring ? x->d_ring : nullptr;
   a.area = x->d_area;
   a.tst = kHourSecs * (double)x->cfg.timestep;  // mo_mrm_pre_routing.f90:110

@@ -147,6 +147,9 @@ struct CellArgs {
   const double *sun;
   int32_t sun_step0;       // step of its first pair of rows
   int32_t skip_fluxes;     // 1: a later launch of the call writes the flux rows
+  // device word, not 0: forcing or weights outside the usual ranges were
+  // uploaded (forcing_scan_kernel)
+  const int32_t *odd_weather;
   // meteo weights [3][12 * 24][sstride] (pre, temp, pet), null: the day/night
   // factors disaggregate
   const double *W;

@@ -1,0 +1,73 @@
+"""Weather for which the branch-free form of the snow (chain.h: snow_meteo) does
+not hold: precipitation so far below zero (errors, nodata of -9999) that the
+degree-day factor is negative.  A cell with such weather in a launch takes the
+branches as written, its neighbours in the wave stay as they are.  Every way
+the forcing reaches the device, daily and hourly, fused and plain, single sets
+and the daily launches that share sun terms, against the oracle to the parity
+bar of tests/test_gpu_parity.py."""
+import sys
+
+import numpy as np
+import pytest
+
+from mhm_amd import synth
+from pairs import START, compare_cells, make_pair
+
+pytestmark = pytest.mark.gpu
+
+RTOL, ATOL = 1e-10, 1e-12
+NODATA = -9999.0
+
+
+def _domain(n_days):
+    """Every second cell has odd days: -0.3 mm (the factor stays positive), -40
+    mm and nodata, on days of hard frost, of thaw and as the series has them;
+    the snow of the start lies on all cells."""
+    dom = synth.make_domain(13, 17, seed=71)
+    synth.make_forcing(dom, n_days, 72, doy0=START.timetuple().tm_yday)
+    for name, shift in (("TAVG", 0.0), ("TMIN", -5.0), ("TMAX", 5.0)):
+        for i, c in enumerate(range(1, dom.n_cells, 2)):
+            t = (-15.0, 6.0, None)[i % 3]
+            if t is not None:
+                dom.forcing[name][:, c] = t + shift
+    for i, c in enumerate(range(1, dom.n_cells, 2)):
+        day = (i // 9) % n_days
+        dom.forcing["PRE"][day, c] = (-0.3, -40.0, NODATA)[(i // 3) % 3]
+    return dom
+
+
+@pytest.mark.parametrize("how,timestep,n_sets", [("set", 1, 1), ("set", 24, 1), ("set", 24, 5),
+                                                 ("stream", 1, 2), ("l2", 24, 4), ("l2", 1, 1),
+                                                 ("weights", 1, 2)])
+def test_odd_weather_matches_oracle(how, timestep, n_sets):
+    n_steps, n_days = 96, 4
+    for mode in (1, 0):
+        print(f"case: odd weather {how} timestep={timestep} sets={n_sets} mode={mode}", flush=True)
+        sys.stdout.flush()
+        dom = _domain(n_days)
+        if how == "weights":
+            dom.forcing["PRE"] = np.abs(dom.forcing["PRE"]) % 50.0
+        model, sim, steps, recs = make_pair([dom], n_sets=n_sets, timestep=timestep,
+                                            n_steps=n_steps, seed=73, route=False,
+                                            forcing_columns=n_days if how == "stream" else None,
+                                            weights=how == "weights")
+        if how == "weights":
+            w = [np.array(v, dtype=float) for v in synth.make_meteo_weights(dom.n_cells, 974)]
+            w[0].reshape(dom.n_cells, -1)[1::4] *= -3.0
+            model.set_meteo_weights(*w)
+            sim.set_meteo_weights(*w)
+        elif how == "stream":
+            model.stream_forcing(dom.forcing, day0=1)
+        elif how == "l2":
+            model.set_forcing("PRE", np.zeros_like(dom.forcing["PRE"]))
+            # cells in Fortran order over a full grid
+            grid = dom.forcing["PRE"].reshape(-1, 17, 13).transpose(0, 2, 1)
+            ones = np.ones((13, 17), bool)
+            model.set_forcing_l2("PRE", 0, grid, ones, 1.0, ones, 1.0)
+        for a, b in ((0, n_steps // 2), (n_steps // 2, n_steps)):
+            model.run(steps[a:b], mode=mode, steps_per_launch=12, want_gauges=False)
+            for r in recs[a:b]:
+                sim.step(r)
+            bad = compare_cells(model, sim, RTOL, ATOL)
+            assert bad == [], bad
+        model.close()
