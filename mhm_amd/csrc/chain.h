@@ -726,17 +726,17 @@ __device__ __forceinline__ void runoff_slow_perc_ordinary(double k1, double kp, 
 // (a NaN is not).
 template <int NH, bool JV>
 __device__ __forceinline__ bool ordinary_params(double fS, double thrS, double incr, double dmax,
-                                                double dnp, double k0, double k1, double k2,
-                                                double kp, double karst, double alpha, double thrU,
+                                                double dnp, double tth, double k0, double k1,
+                                                double k2, double kp, double karst, double alpha, double thrU,
                                                 const double *sat, const double *fr,
                                                 const double *fc, const double *wp,
                                                 const double *bexp, double c1) {
   // no short circuits: one straight line of compares
-  bool ok = (fS >= 0.0) & (!(fS > 0.0) | (thrS > kTiny)) & (thrS < kBig) & (incr >= 0.0) &
-            (incr < kBig) & (dnp >= 0.0) & (dnp < kBig) & (dmax >= 0.0) & (dmax < kBig) &
-            (k0 >= 0.0) & (k0 < kBig) & (k1 >= 0.0) & (k1 < kBig) & (k2 >= 0.0) & (k2 <= 1.0) &
-            (kp >= 0.0) & (kp < kBig) & (karst >= 0.0) & (karst < kBig) & (alpha > -1.0) &
-            (alpha < 64.0) & (thrU > kTiny) & (thrU < kBig);
+  bool ok = (fS >= 0.0) & (!(fS > 0.0) | (thrS > kTiny)) & (fabs(thrS) < kBig) & (incr >= 0.0) &
+            (incr < kBig) & (fabs(tth) < kBig) & (dnp >= 0.0) & (dnp < kBig) & (dmax >= 0.0) &
+            (dmax < kBig) & (k0 >= 0.0) & (k0 < kBig) & (k1 >= 0.0) & (k1 < kBig) & (k2 >= 0.0) &
+            (k2 <= 1.0) & (kp >= 0.0) & (kp < kBig) & (karst >= 0.0) & (karst < kBig) &
+            (alpha > -1.0) & (alpha < 64.0) & (thrU > kTiny) & (thrU < kBig);
 #pragma unroll
   for (int h = 0; h < NH; ++h) {
     ok = ok & (sat[h] >= 1.0) & (sat[h] < kBig) & (bexp[h] >= 1.0) & (bexp[h] < 64.0) &
@@ -758,9 +758,11 @@ __device__ __forceinline__ bool ordinary_weather(double incr, double dnp, double
 }
 
 template <int NH>
-__device__ __forceinline__ bool ordinary_states(double pack, double unsat, double satS,
-                                                const double *sm, const double *sat) {
-  bool ok = (pack >= 0.0) & (unsat >= 0.0) & (unsat < kBig) & (satS >= 0.0);
+__device__ __forceinline__ bool ordinary_states(double inter, double pack, double seal,
+                                                double unsat, double satS, const double *sm,
+                                                const double *sat) {
+  bool ok = (inter < kBig) & (seal < kBig) & (pack >= 0.0) & (unsat >= 0.0) & (unsat < kBig) &
+            (satS >= 0.0);
 #pragma unroll
   for (int h = 0; h < NH; ++h) ok = ok & (sm[h] >= kEps) & (sm[h] <= sat[h]);
   return ok;

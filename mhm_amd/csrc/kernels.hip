@@ -450,14 +450,14 @@ __device__ __forceinline__ Stress<NH> stress_of(const CellRegs<NH> &c, bool ordi
 
 template <int NH, bool JV>
 __device__ __forceinline__ bool ordinary_cell(const CellRegs<NH> &c, bool init_sm) {
-  bool ok = ordinary_params<NH, JV>(c.fS, c.thrS, c.incr, c.dmaxs, c.dnps, c.k0s, c.k1s, c.k2s,
-                                    c.kps, c.karst, c.alpha, c.thrU, c.sat, c.fr, c.fc, c.wp,
-                                    c.bexp, c.c1);
+  bool ok = ordinary_params<NH, JV>(c.fS, c.thrS, c.incr, c.dmaxs, c.dnps, c.tth, c.k0s, c.k1s,
+                                    c.k2s, c.kps, c.karst, c.alpha, c.thrU, c.sat, c.fr, c.fc,
+                                    c.wp, c.bexp, c.c1);
   // a step that resets the soil moisture starts from half the field capacity
   double sm[NH];
 #pragma unroll
   for (int h = 0; h < NH; ++h) sm[h] = init_sm ? 0.5 * c.fc[h] : c.sm[h];
-  return ok && ordinary_states<NH>(c.pack, c.unsat, c.satS, sm, c.sat);
+  return ok && ordinary_states<NH>(c.inter, c.pack, c.seal, c.unsat, c.satS, sm, c.sat);
 }
 
 template <int NH, bool JV>
