@@ -85,6 +85,7 @@ struct mhmhip_ctx {
   // not read it), n_frows rows in all
   int32_t frow[MHMHIP_F_COUNT] = {};
   int32_t n_frows = 0;
+  uint8_t *d_odd = nullptr;  // [sstride] OddWeather marks of the cells
   double *W = nullptr;  // meteo weights [3][12 * 24][sstride], null: off
   // MPR-lite inputs (mhmhip_mprlite_inputs): host copies in reference cell
   // order, and the kernel's input rows laid out as the cells are (rebuilt
@@ -339,29 +340,6 @@ static hipError_t sync_copy(mhmhip_ctx *x, void *dst, const void *src, size_t n,
 }
 
 // ---------------------------------------------------------------------------
-namespace {
-int64_t forcing_values(const mhmhip_ctx *x) {
-  return (int64_t)x->n_frows * x->cfg.n_forcing_days * x->sstride;
-}
-
-// The word after the forcing columns: not 0 once forcing, weights or factors
-// outside the usual ranges were given (CellArgs::odd_weather).  It stays, also
-// when they are replaced: launches then look at their steps' weather.
-int32_t *odd_weather(const mhmhip_ctx *x) {
-  return reinterpret_cast<int32_t *>(x->F + forcing_values(x));
-}
-
-// After n columns of a variable from col on were written on stream s.
-int scan_forcing(mhmhip_ctx *x, int32_t var, int32_t col, int32_t n, hipStream_t s) {
-  if (var != MHMHIP_F_PRE && var != MHMHIP_F_TAVG) return MHMHIP_OK;
-  const double *rows =
-      x->F + ((int64_t)x->frow[var] * x->cfg.n_forcing_days + col) * x->sstride;
-  const hipError_t e = launch_forcing_scan(rows, x->sstride, n, x->n_cells,
-                                           var == MHMHIP_F_TAVG, odd_weather(x), s);
-  return e == hipSuccess ? MHMHIP_OK : x->hipfail(e, "forcing scan");
-}
-}  // namespace
-
 extern "C" int mhmhip_create(const mhmhip_config *cfg, mhmhip_ctx **out) {
   if (!cfg || !out) {
     g_create_error = "create: null argument";
@@ -475,17 +453,19 @@ extern "C" int mhmhip_create(const mhmhip_config *cfg, mhmhip_ctx **out) {
   if ((rc = x->dalloc(&x->P, x->n_prows * x->ld, "alloc params")) ||
       (rc = x->dalloc(&x->S, x->n_srows * x->ld, "alloc states")) ||
       (rc = x->dalloc(&x->X, x->n_xrows * x->ld, "alloc fluxes")) ||
-      (rc = x->dalloc(&x->F, forcing_values(x) + 1, "alloc forcing"))) {  // and odd_weather
+      (rc = x->dalloc(&x->F, (int64_t)x->n_frows * c.n_forcing_days * x->sstride,
+                      "alloc forcing")) ||
+      (rc = x->dalloc(&x->d_odd, x->sstride, "alloc weather marks"))) {
     g_create_error = x->err;
     mhmhip_destroy(x);
     return rc;
   }
-  bool usual = true;  // day and night shares of the precipitation, temperature shifts
+  bool usual = true;  // the day's and night's shares of the precipitation, temperature shifts
   for (int m = 0; m < 12; ++m)
     usual = usual && c.fnight_prec[m] >= 0.0 && c.fnight_prec[m] <= 1.0 &&
             std::isfinite(c.fnight_temp[m]);
-  if (!usual && hipMemsetAsync(odd_weather(x), 1, sizeof(int32_t), x->stream) != hipSuccess) {
-    g_create_error = "create: setting the weather word failed";
+  if (!usual && hipMemsetAsync(x->d_odd, OW_FACTOR, x->sstride, x->stream) != hipSuccess) {
+    g_create_error = "create: setting the weather marks failed";
     mhmhip_destroy(x);
     return MHMHIP_EHIP;
   }
@@ -521,6 +501,7 @@ extern "C" int mhmhip_destroy(mhmhip_ctx *x) {
   (void)hipFree(x->S);
   (void)hipFree(x->X);
   (void)hipFree(x->F);
+  (void)hipFree(x->d_odd);
   (void)hipFree(x->W);
   (void)hipFree(x->d_agg_start);
   (void)hipFree(x->d_cring);
@@ -877,6 +858,21 @@ int forcing_columns_direct(mhmhip_ctx *x, int32_t day0, int32_t ndays) {
   return MHMHIP_OK;
 }
 
+// After n columns of a variable from col on were written on stream s: marks the
+// cells with odd weather in them.  whole: the variable has no other column, so
+// that marks of what it held before go.
+int scan_forcing(mhmhip_ctx *x, int32_t var, int32_t col, int32_t n, bool whole, hipStream_t s) {
+  if (var != MHMHIP_F_PRE && var != MHMHIP_F_TAVG) return MHMHIP_OK;
+  const int32_t bit = var == MHMHIP_F_PRE ? OW_PRE : OW_TAVG;
+  if (whole) CHECK_HIP(x, launch_odd_clear(x->sstride, bit, x->d_odd, s), "forcing scan");
+  const double *rows =
+      x->F + ((int64_t)x->frow[var] * x->cfg.n_forcing_days + col) * x->sstride;
+  CHECK_HIP(x, launch_forcing_scan(rows, x->sstride, n, x->n_cells, var == MHMHIP_F_TAVG, bit,
+                                   x->d_odd, s),
+            "forcing scan");
+  return MHMHIP_OK;
+}
+
 // The compute stream waits for the streamed chunks that wrote the columns
 // the steps read (chunks complete in order on the copy stream: waiting for
 // the newest is enough).
@@ -981,8 +977,8 @@ extern "C" int mhmhip_stream_forcing(mhmhip_ctx *x, int32_t day0, int32_t ndays,
   const int32_t col0 = (day0 - 1) % nfd, n0 = std::min(ndays, nfd - col0);
   for (int32_t v : {MHMHIP_F_PRE, MHMHIP_F_TAVG})
     if (host[v]) {
-      CHECK_RC(scan_forcing(x, v, col0, n0, x->cstream));
-      CHECK_RC(scan_forcing(x, v, 0, ndays - n0, x->cstream));
+      CHECK_RC(scan_forcing(x, v, col0, n0, ndays == nfd, x->cstream));
+      CHECK_RC(scan_forcing(x, v, 0, ndays - n0, false, x->cstream));
     }
   hipEvent_t done = nullptr;
   CHECK_HIP(x, hipEventCreateWithFlags(&done, hipEventDisableTiming), "stream_forcing event");
@@ -1013,7 +1009,7 @@ extern "C" int mhmhip_set_forcing(mhmhip_ctx *x, int32_t var, int32_t day0, int3
         x->F + ((int64_t)x->frow[var] * x->cfg.n_forcing_days + (day0 - 1 + j)) * x->sstride;
     CHECK_RC(put_row(x, dst, host + (int64_t)j * ld, id));
   }
-  CHECK_RC(scan_forcing(x, var, day0 - 1, ndays, x->stream));
+  CHECK_RC(scan_forcing(x, var, day0 - 1, ndays, ndays == x->cfg.n_forcing_days, x->stream));
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "set_forcing");
   return MHMHIP_OK;
 }
@@ -1144,7 +1140,8 @@ extern "C" int mhmhip_set_forcing_l2(mhmhip_ctx *x, int32_t var, int32_t domain,
   double *dst = x->F + ((int64_t)x->frow[var] * x->cfg.n_forcing_days + (day0 - 1)) * x->sstride;
   CHECK_HIP(x, launch_meteo_l2(b.data2, b.mask2, nr2, n2, b.cells, ncells, ndays, dst, x->sstride,
                                aggregate, x->stream), "set_forcing_l2 map");
-  CHECK_RC(scan_forcing(x, var, day0 - 1, ndays, x->stream));
+  CHECK_RC(scan_forcing(x, var, day0 - 1, ndays,
+                        x->n_domains == 1 && ndays == x->cfg.n_forcing_days, x->stream));
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "set_forcing_l2");
   return MHMHIP_OK;
 }
@@ -1217,6 +1214,8 @@ extern "C" int mhmhip_set_meteo_weights(mhmhip_ctx *x, const double *pre_w,
   CHECK_HIP(x, hipSetDevice(x->cfg.device), "set_meteo_weights");
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "set_meteo_weights");
   drop_graph(x);  // a captured run holds the kernels' arguments
+  CHECK_HIP(x, launch_odd_clear(x->sstride, OW_PRE_WEIGHT | OW_TEMP_WEIGHT, x->d_odd, x->stream),
+            "set_meteo_weights");
   if (given == 0) {
     x->dfree(x->W, (int64_t)3 * 12 * 24 * x->sstride);
     x->W = nullptr;
@@ -1234,7 +1233,8 @@ extern "C" int mhmhip_set_meteo_weights(mhmhip_ctx *x, const double *pre_w,
                          host[v] + ld * ((int64_t)m + 12 * h), id));
   for (int v = 0; v < 2; ++v)  // precipitation, temperature
     CHECK_HIP(x, launch_forcing_scan(x->W + (int64_t)v * 288 * x->sstride, x->sstride, 288,
-                                     x->n_cells, v == 1, odd_weather(x), x->stream),
+                                     x->n_cells, v == 1, v == 0 ? OW_PRE_WEIGHT : OW_TEMP_WEIGHT,
+                                     x->d_odd, x->stream),
               "set_meteo_weights");
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "set_meteo_weights");
   return MHMHIP_OK;
@@ -1293,7 +1293,7 @@ CellArgs cell_args(mhmhip_ctx *x, bool ring) {
   a.S = x->S;
   a.X = x->X;
   a.F = x->F;
-  a.odd_weather = odd_weather(x);
+  a.odd_weather = x->d_odd;
   a.ring = ring ? x->d_ring : nullptr;
   a.area = x->d_area;
   a.tst = kHourSecs * (double)x->cfg.timestep;  // mo_mrm_pre_routing.f90:110
@@ -1874,6 +1874,12 @@ extern "C" int mhmhip_bind_network(mhmhip_ctx *x, const mhmhip_network *net) {
     if (x->x_dirty) CHECK_RC(relayout(x->X, x->n_xrows, x->ld, x->n_sets));
     if (x->f_dirty)
       CHECK_RC(relayout(x->F, (int64_t)x->n_frows * x->cfg.n_forcing_days, x->sstride, 1));
+    if (x->f_dirty || x->W) {  // weather marks
+      std::vector<uint8_t> m(x->sstride), n(x->sstride, 0);
+      CHECK_HIP(x, sync_copy(x, m.data(), x->d_odd, m.size(), hipMemcpyDeviceToHost), "relayout");
+      for (int64_t c = 0; c < x->n_cells; ++c) n[cpos[c]] = m[old_pos[c]];
+      CHECK_HIP(x, sync_copy(x, x->d_odd, n.data(), n.size(), hipMemcpyHostToDevice), "relayout");
+    }
     if (x->W) CHECK_RC(relayout(x->W, (int64_t)3 * 12 * 24, x->sstride, 1));
     if (x->d_out) CHECK_RC(relayout(x->d_out, x->out_rows_cap, x->ld, x->n_sets));  // output sums
   }

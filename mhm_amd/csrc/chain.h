@@ -588,12 +588,12 @@ __device__ __forceinline__ double total_runoff(double fS, double fast, double sl
 // (every type at one wave instruction per four cycles), and about half of the
 // functions above is compares, 64-bit selects (two instructions each) and
 // copies at the ends of divergent branches.  For parameters, states and
-// weather in their physical ranges (ordinary_params, ordinary_states,
-// ordinary_weather: non-negative rates, field capacity above wilting point, a
-// store within its bounds, a degree-day factor not below zero, ...) every
-// branch is a minimum, a maximum or has a known outcome.  A cell outside these
-// ranges takes the functions above; which of the two a cell takes depends on
-// that cell alone.  The values are those of the functions above:
+// weather in their physical ranges (ordinary_params, ordinary_states and
+// forcing_scan_kernel: non-negative rates, field capacity above wilting point,
+// a store within its bounds, precipitation not below zero, ...) every branch is
+// a minimum, a maximum or has a known outcome.  A cell outside these ranges
+// takes the functions above; which of the two a cell takes depends on that
+// cell alone.  The values are those of the functions above:
 // equal bits, except that where two branches meet (a store filled or emptied
 // exactly, the degree-day factor reaching its maximum, field capacity) the
 // result may be the other branch's, one rounding away.
@@ -632,8 +632,9 @@ __device__ __forceinline__ void canopy_ordinary(double pet, double interc_max, d
 
 // snow_accum_melt, first what the meteo values alone give: the degree-day
 // factor (its rise ends where it meets its maximum), the melt a large enough
-// pack would give (a cold step's product is negative and melts nothing) and
-// whether precipitation is snow (1) or rain (0).
+// pack would give (a cold step's product is negative and melts nothing; with a
+// factor below zero, for precipitation below -dnp / incr, it would be positive)
+// and whether precipitation is snow (1) or rain (0).
 struct SnowMeteo {
   double ddf, melt, cold;
 };
@@ -746,15 +747,6 @@ __device__ __forceinline__ bool ordinary_params(double fS, double thrS, double i
   }
   if constexpr (JV) ok = ok & (c1 > kTiny) & (c1 < kBig);
   return ok;
-}
-
-// Whether a step's precipitation and temperature are in the ranges the
-// functions above assume: below -dnp / incr the degree-day factor is negative,
-// a frost would melt snow and a thaw would add to it (the reference's branches
-// have neither).
-__device__ __forceinline__ bool ordinary_weather(double incr, double dnp, double prec,
-                                                 double temp) {
-  return (dnp + incr * prec >= 0.0) & (prec < kBig) & (fabs(temp) < kBig);
 }
 
 template <int NH>

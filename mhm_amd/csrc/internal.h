@@ -71,6 +71,8 @@ enum StepChange {
   SC_INIT = 8,   // the step resets the soil moisture (init_sm)
 };
 
+enum OddWeather { OW_PRE = 1, OW_TAVG = 2, OW_PRE_WEIGHT = 4, OW_TEMP_WEIGHT = 8, OW_FACTOR = 16 };
+
 // Per-step scalars on the device (host-evaluated from the step clock).
 struct StepDev {
   double dr, tand, sind, cosd;  // extraterr_rad_approx day-of-year terms
@@ -147,9 +149,9 @@ struct CellArgs {
   const double *sun;
   int32_t sun_step0;       // step of its first pair of rows
   int32_t skip_fluxes;     // 1: a later launch of the call writes the flux rows
-  // device word, not 0: forcing or weights outside the usual ranges were
-  // uploaded (forcing_scan_kernel)
-  const int32_t *odd_weather;
+  // [n_cells] OddWeather bits: what was given for the cell outside the ranges
+  // that the branch-free form covers (forcing_scan_kernel); 0: nothing
+  const uint8_t *odd_weather;
   // meteo weights [3][12 * 24][sstride] (pre, temp, pet), null: the day/night
   // factors disaggregate
   const double *W;

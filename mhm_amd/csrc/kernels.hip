@@ -91,7 +91,6 @@ __device__ __forceinline__ CellArgs read_args(ConstArgs *p) {
   a.jarvis = p->jarvis, a.hourly = p->hourly, a.ring_rep = p->ring_rep;
   a.raw_total = p->raw_total, a.nT = p->nT, a.rnT = p->rnT, a.W = p->W;
   a.sun = p->sun, a.sun_step0 = p->sun_step0, a.skip_fluxes = p->skip_fluxes;
-  a.odd_weather = p->odd_weather;
   return a;
 }
 
@@ -448,11 +447,14 @@ __device__ __forceinline__ Stress<NH> stress_of(const CellRegs<NH> &c, bool ordi
   return t;
 }
 
+// odd: the cell's weather mark (CellArgs::odd_weather)
 template <int NH, bool JV>
-__device__ __forceinline__ bool ordinary_cell(const CellRegs<NH> &c, bool init_sm) {
-  bool ok = ordinary_params<NH, JV>(c.fS, c.thrS, c.incr, c.dmaxs, c.dnps, c.tth, c.k0s, c.k1s,
-                                    c.k2s, c.kps, c.karst, c.alpha, c.thrU, c.sat, c.fr, c.fc,
-                                    c.wp, c.bexp, c.c1);
+__device__ __forceinline__ bool ordinary_cell(const CellRegs<NH> &c, bool init_sm, uint32_t odd) {
+  // no branch on odd: the loads it would hold back are as far away as its own
+  const bool ok = (odd == 0) & ordinary_params<NH, JV>(
+                                   c.fS, c.thrS, c.incr, c.dmaxs, c.dnps, c.tth, c.k0s, c.k1s,
+                                   c.k2s, c.kps, c.karst, c.alpha, c.thrU, c.sat, c.fr, c.fc,
+                                   c.wp, c.bexp, c.c1);
   // a step that resets the soil moisture starts from half the field capacity
   double sm[NH];
 #pragma unroll
@@ -638,64 +640,11 @@ __device__ __attribute__((noinline)) void general_step(ConstArgs *args, uint32_t
                         a.ring && a.lag ? a.lag[c] : 0, r, x);
 }
 
-// An ordinary cell's step, its loads issued.
-template <int NH, bool JV, bool OUT>
-__device__ __forceinline__ void step_ordinary(ConstArgs *k, const CellArgs &a, const StepArgs &sa,
-                                              uint32_t c, uint32_t bv, double pre, double tavg,
-                                              double tmax, double tmin, CellRegs<NH> &r,
-                                              FluxRegs<NH> &x) {
-  const StepDev &st = sa.st;
-  const uint32_t bc = c * 8u;
-  double scale = a.ring ? runoff_scale(a, bc) : 0.0;
-  int32_t g = a.ring && a.lag ? a.lag[c] : 0;
-  step_start<NH>(a, st, bc, bv, pre, tavg, tmax, tmin, r, x);
-  double maxinter = ldr(a.P + (int64_t)(pr_maxinter(NH) + st.month0) * a.ld, bv);
-  // no load is waited for once the stores start: they share a counter
-  settle(maxinter);
-  settle(scale);
-  asm volatile("" : "+v"(g));
-  settle_all<NH>(r);
-  ordinary_step<NH, JV>(a, bv, r, x, maxinter, maxinter > kEps ? 1.0 / maxinter : 0.0,
-                        div_rcp(x.pet, st.evap, st.revap), stress_of<NH, JV>(r, true));
-  step_end<NH, JV, OUT>(k, a, c, bv, sa.t, scale, g, r, x);
-}
-
-// A step whose forcing may hold weather that the branch-free form does not
-// cover (CellArgs::odd_weather): looks at the cell's first.  Out of line and
-// the only thing such a step does: the look in every step's kernel cost 2 to
-// 15 of 67 us in spilled registers.
-template <int NH, bool JV, bool OUT>
-__device__ __attribute__((noinline)) void step_odd(ConstArgs *args, uint32_t c, uint32_t bv) {
-  ConstArgs *k = uniform(args);
-  const CellArgs a = read_args(k);
-  const __attribute__((address_space(4))) StepArgs *p =
-      (const __attribute__((address_space(4))) StepArgs *)(k + 1);
-  const StepArgs sa{read_step(&p->st), p->t};
-  const StepDev &st = sa.st;
-  const uint32_t bc = c * 8u;
-  const double pre = ldr(frow_ptr(a, MHMHIP_F_PRE, st.day), bc);
-  const double tavg = ldr(frow_ptr(a, MHMHIP_F_TAVG, st.day), bc);
-  CellRegs<NH> r;
-  FluxRegs<NH> x;
-  load_params<NH, JV>(a, bv, r);
-  load_states<NH>(a, bv, r);
-  disagg_step<NH>(a, st, bc, 0.0, tavg, pre, x.pet, x.temp, x.prec);
-  if (ordinary_weather(r.incr, r.dnps, x.prec, x.temp) &&
-      ordinary_cell<NH, JV>(r, st.init_sm != 0)) {
-    const double tmax = a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMAX, st.day), bc) : 0.0;
-    const double tmin = a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMIN, st.day), bc) : 0.0;
-    step_ordinary<NH, JV, OUT>(k, a, sa, c, bv, pre, tavg, tmax, tmin, r, x);
-  } else {
-    general_step<NH, JV, OUT>(k, c, bv);
-  }
-}
-
 template <int NH, bool JV, bool OUT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NH > 3 ? 2 : OUT ? 3 : 4)))
 void cell_step_kernel(CellArgs a, StepArgs sa) {
   static_assert(sizeof(CellArgs) % alignof(StepArgs) == 0, "StepArgs follows CellArgs");
   const StepDev &st = sa.st;
-  const int32_t odd = *(const __attribute__((address_space(4))) int32_t *)a.odd_weather;
   const uint32_t c0 = blockIdx.x * blockDim.x + threadIdx.x;
   const bool act = c0 < a.n_cells;
   const uint32_t c = act ? c0 : 0u;  // an idle lane loads cell 0 and leaves after the fill
@@ -709,15 +658,24 @@ void cell_step_kernel(CellArgs a, StepArgs sa) {
   const double tavg = ldr(frow_ptr(a, MHMHIP_F_TAVG, st.day), bc);
   const double tmax = a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMAX, st.day), bc) : 0.0;
   const double tmin = a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMIN, st.day), bc) : 0.0;
+  const uint32_t odd = a.odd_weather[c];
   mathtab_fill();  // the chain's powers read it (every thread, before any returns)
   if (!act) return;
-  if (__builtin_expect(odd, 0)) {
-    step_odd<NH, JV, OUT>(kernel_args(), opaque(c), opaque(bv));
-    return;
+  const bool ordinary = ordinary_cell<NH, JV>(r, st.init_sm != 0, odd);
+  if (ordinary) {
+    double scale = a.ring ? runoff_scale(a, bc) : 0.0;
+    int32_t g = a.ring && a.lag ? a.lag[c] : 0;
+    step_start<NH>(a, st, bc, bv, pre, tavg, tmax, tmin, r, x);
+    double maxinter = ldr(a.P + (int64_t)(pr_maxinter(NH) + st.month0) * a.ld, bv);
+    // no load is waited for once the stores start: they share a counter
+    settle(maxinter);
+    settle(scale);
+    asm volatile("" : "+v"(g));
+    settle_all<NH>(r);
+    ordinary_step<NH, JV>(a, bv, r, x, maxinter, maxinter > kEps ? 1.0 / maxinter : 0.0,
+                          div_rcp(x.pet, st.evap, st.revap), stress_of<NH, JV>(r, true));
+    step_end<NH, JV, OUT>(kernel_args(), a, c, bv, sa.t, scale, g, r, x);
   }
-  const bool ordinary = ordinary_cell<NH, JV>(r, st.init_sm != 0);
-  if (ordinary)
-    step_ordinary<NH, JV, OUT>(kernel_args(), a, sa, c, bv, pre, tavg, tmax, tmin, r, x);
   // last, where the call finds no other value in use
   if (!ordinary) general_step<NH, JV, OUT>(kernel_args(), opaque(c), opaque(bv));
 }
@@ -968,9 +926,10 @@ constexpr int kAllChanged = SC_METEO | SC_DAY | SC_MONTH;
 // independent chains, and a wave in which no lane has water to infiltrate at
 // step s + 1 leaves the horizon powers out.  The first turn only starts.
 template <int NH, bool JV, bool OUT, bool DY>
-__device__ __forceinline__ void fused_ordinary(ConstArgs *k, const CellArgs &a, FusedLane &u,
-                                               CellRegs<NH> &r, const ConstStep *steps,
-                                               int32_t nsteps, const DayParams &day) {
+__device__ __forceinline__ void fused_ordinary(const CellArgs &a, FusedLane &u, CellRegs<NH> &r,
+                                               const ConstStep *steps, int32_t nsteps,
+                                               const DayParams &day) {
+  ConstArgs *k = kernel_args();
   const uint64_t mask = OUT ? k->out.mask : 0;
   const int n_canopy = __builtin_popcountll(mask & 0x1F);  // outputs_canopy's bits
   if (OUT) load_sums(k, a.ld, u.bv, u.slot + LS_STRESS + stress_slots(NH, JV));
@@ -1121,60 +1080,6 @@ __device__ __attribute__((noinline)) void fused_general(ConstArgs *args, uint32_
   store_states<NH>(a, bv, r);
 }
 
-// A cell's launch if it is an ordinary one; false: it is not, nothing was done.
-template <int NH, bool JV, bool OUT, bool DY>
-__device__ __forceinline__ bool fused_cell(ConstArgs *k, const CellArgs &a, const FusedArgs &fa,
-                                           uint32_t c, uint32_t bv, uint32_t slot) {
-  const ConstStep *steps = (const ConstStep *)(a.steps + fa.step0);
-  CellRegs<NH> r;
-  load_params<NH, JV>(a, bv, r);
-  load_states<NH>(a, bv, r);
-  const bool ordinary = ordinary_cell<NH, JV>(r, steps->init_sm != 0);
-  if (ordinary) {
-    FusedLane u;
-    fused_lane<NH, JV>(a, c, bv, slot, fa.t0, stress_of<NH, JV>(r, true), u);
-    settle(u.scale);
-    settle_all<NH>(r);
-    DayParams day{};
-    if (DY) {
-      auto P = [&](int row) { return ldr(a.P + (int64_t)row * a.ld, bv); };
-      day = {r.incr, r.dmaxs, r.dnps, r.tth, P(PR_FASP), P(PR_HARSAM)};
-      settle(day.fasp), settle(day.harsam);
-    }
-    fused_ordinary<NH, JV, OUT, DY>(k, a, u, r, steps, fa.nsteps, day);
-    store_states<NH>(a, bv, r);
-  }
-  return ordinary;
-}
-
-// A launch whose forcing may hold weather that the branch-free form does not
-// cover (CellArgs::odd_weather): looks at the cell's steps first, which
-// reads the forcing twice.  Out of line and the only thing such a launch does:
-// a call for the look alone, before the loads, cost every other launch 20 of
-// 1140 us in spilled registers.
-template <int NH, bool JV, bool OUT>
-__device__ __attribute__((noinline)) void fused_odd(ConstArgs *args, uint32_t c, uint32_t bv,
-                                                    uint32_t slot) {
-  ConstArgs *k = uniform(args);
-  const CellArgs a = read_args(k);
-  const __attribute__((address_space(4))) FusedArgs *p =
-      (const __attribute__((address_space(4))) FusedArgs *)(k + 1);
-  const FusedArgs fa{p->t0, p->nsteps, p->step0};
-  const ConstStep *steps = (const ConstStep *)(a.steps + fa.step0);
-  const double incr = ldr(a.P + (int64_t)PR_INCR * a.ld, bv);
-  const double dnp = ldr(a.P + (int64_t)PR_DNPS * a.ld, bv);
-  bool ordinary = true;
-#pragma nounroll
-  for (int32_t s = 0; s < fa.nsteps; ++s) {
-    if (s > 0 && !(steps[s].change & SC_METEO)) continue;
-    double pet, temp, prec;
-    disagg_at<NH>(a, read_step(steps + s), c * 8u, 0.0, pet, temp, prec);
-    ordinary = ordinary & ordinary_weather(incr, dnp, prec, temp);
-  }
-  if (ordinary) ordinary = fused_cell<NH, JV, OUT, false>(k, a, fa, c, bv, slot);
-  if (!ordinary) fused_general<NH, JV, OUT>(k, c, bv, slot);
-}
-
 // ---------------------------------------------------------------------------
 // Fused path: nsteps model steps per launch with parameters and states held
 // in registers.  Forcing and daily PET are read/evaluated once per forcing day
@@ -1194,18 +1099,31 @@ __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(NH > 3 ? 2 : JV || OUT || DY ? 3 : 4)))
 void cell_fused_kernel(CellArgs a, FusedArgs fa) {
   static_assert(sizeof(CellArgs) % alignof(FusedArgs) == 0, "FusedArgs follows CellArgs");
-  const int32_t odd = *(const __attribute__((address_space(4))) int32_t *)a.odd_weather;
   mathtab_fill();  // the chain's powers read it (before any thread returns)
   const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= a.n_cells) return;
   const uint32_t bv = (uint32_t)(blockIdx.y * a.sstride + c) * 8u;
   // this lane's LDS slots (lane_slots doubles, laid out lane by lane)
   const uint32_t slot = threadIdx.x * (uint32_t)lane_slots(NH, JV, OUT ? a.out.n : 0);
-  if (__builtin_expect(odd, 0)) {
-    fused_odd<NH, JV, OUT>(kernel_args(), c, bv, slot);
-    return;
+  const ConstStep *steps = (const ConstStep *)(a.steps + fa.step0);
+  CellRegs<NH> r;
+  load_params<NH, JV>(a, bv, r);
+  load_states<NH>(a, bv, r);
+  const bool ordinary = ordinary_cell<NH, JV>(r, steps->init_sm != 0, a.odd_weather[c]);
+  if (ordinary) {
+    FusedLane u;
+    fused_lane<NH, JV>(a, c, bv, slot, fa.t0, stress_of<NH, JV>(r, true), u);
+    settle(u.scale);
+    settle_all<NH>(r);
+    DayParams day{};
+    if (DY) {
+      auto P = [&](int row) { return ldr(a.P + (int64_t)row * a.ld, bv); };
+      day = {r.incr, r.dmaxs, r.dnps, r.tth, P(PR_FASP), P(PR_HARSAM)};
+      settle(day.fasp), settle(day.harsam);
+    }
+    fused_ordinary<NH, JV, OUT, DY>(a, u, r, steps, fa.nsteps, day);
+    store_states<NH>(a, bv, r);
   }
-  const bool ordinary = fused_cell<NH, JV, OUT, DY>(kernel_args(), a, fa, c, bv, slot);
   // last, where the call finds no other value in use
   if (!ordinary) fused_general<NH, JV, OUT>(kernel_args(), c, bv, slot);
 }
@@ -2213,14 +2131,13 @@ hipError_t launch_row_gather(const double *row, const int32_t *pos, double *out,
   return hipGetLastError();
 }
 
-// Whether n_rows rows of precipitation or temperature (lowest: 0 or -kBig) hold
-// a value outside [lowest, kBig): then *odd becomes 1 (and stays so).  With none
-// the degree-day factor is not below zero in any ordinary cell, and the cell
-// kernels need not look.  60 days of 1024x1024 cells: 0.1 ms beside 9 ms of
-// their upload.
+// Marks the cells whose n_rows rows of precipitation or temperature hold a value
+// outside [lowest, kBig) with bit (CellArgs::odd_weather).  For the others the
+// degree-day factor is not below zero at any step.
 __global__ __launch_bounds__(256) void forcing_scan_kernel(const double *rows, int64_t stride,
                                                            int32_t n_rows, int64_t n_cells,
-                                                           double lowest, int32_t *odd) {
+                                                           double lowest, int32_t bit,
+                                                           uint8_t *odd) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= n_cells) return;
   bool ok = true;
@@ -2228,16 +2145,30 @@ __global__ __launch_bounds__(256) void forcing_scan_kernel(const double *rows, i
     const double v = rows[(int64_t)t * stride + c];
     ok = ok & (v >= lowest) & (v < kBig);
   }
-  if (!ok) *odd = 1;
+  // marks are given from two streams
+  if (!ok) atomicOr(reinterpret_cast<uint32_t *>(odd) + c / 4, (uint32_t)bit << 8 * (c % 4));
+}
+
+// Takes bits out of the marks (n: a multiple of 4).
+__global__ __launch_bounds__(256) void odd_clear_kernel(int64_t n, int32_t bits, uint8_t *odd) {
+  const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (w < n / 4) atomicAnd(reinterpret_cast<uint32_t *>(odd) + w, ~((uint32_t)bits * 0x01010101u));
 }
 
 hipError_t launch_forcing_scan(const double *rows, int64_t stride, int32_t n_rows, int64_t n_cells,
-                               bool temperature, int32_t *odd, hipStream_t s) {
+                               bool temperature, int32_t bit, uint8_t *odd, hipStream_t s) {
   if (n_rows < 1) return hipSuccess;
   if (n_cells < 1 || !rows || !odd) return hipErrorInvalidValue;
   const dim3 grid((unsigned)((n_cells + 255) / 256), (unsigned)(n_rows < 64 ? n_rows : 64));
   hipLaunchKernelGGL(forcing_scan_kernel, grid, dim3(256), 0, s, rows, stride, n_rows, n_cells,
-                     temperature ? -kBig : 0.0, odd);
+                     temperature ? -kBig : 0.0, bit, odd);
+  return hipGetLastError();
+}
+
+hipError_t launch_odd_clear(int64_t n, int32_t bits, uint8_t *odd, hipStream_t s) {
+  if (n < 4 || n % 4 != 0 || !odd) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(odd_clear_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, n,
+                     bits, odd);
   return hipGetLastError();
 }
 

@@ -73,9 +73,9 @@ def estimate_bytes(n_cells, n_sets, n_horizons, n_forcing_days, plan, chunk_step
     sstride = (n_cells + 63) // 64 * 64
     ld = sstride * n_sets
     rows = (19 + 5 * n_horizons + 60) + (5 + n_horizons) + (17 + 2 * n_horizons)
-    # parameter, state and flux rows; forcing columns and a word; MPR-lite's 8
-    # input rows
-    cells = (rows * ld * 8 + FORCING_ROWS[process_pet] * n_forcing_days * sstride * 8 + 8
+    # parameter, state and flux rows; forcing columns and weather marks;
+    # MPR-lite's 8 input rows
+    cells = (rows * ld * 8 + FORCING_ROWS[process_pet] * n_forcing_days * sstride * 8 + sstride
              + 8 * sstride * 8)
     window = 8  # default routing window (mhmhip_run_opts)
     rows_run = min(chunk_steps, n_steps)  # steps of the longest call

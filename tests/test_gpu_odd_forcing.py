@@ -1,6 +1,6 @@
 """Weather for which the branch-free form of the snow (chain.h: snow_meteo) does
 not hold: precipitation so far below zero (errors, nodata of -9999) that the
-degree-day factor is negative.  A cell with such weather in a launch takes the
+degree-day factor is negative.  A cell that has been given such weather takes the
 branches as written, its neighbours in the wave stay as they are.  Every way
 the forcing reaches the device, daily and hourly, fused and plain, single sets
 and the daily launches that share sun terms, against the oracle to the parity
@@ -10,7 +10,7 @@ import sys
 import numpy as np
 import pytest
 
-from mhm_amd import synth
+from mhm_amd import calendar, engine, parameters as PM, synth
 from pairs import START, compare_cells, make_pair
 
 pytestmark = pytest.mark.gpu
@@ -71,3 +71,54 @@ def test_odd_weather_matches_oracle(how, timestep, n_sets):
             bad = compare_cells(model, sim, RTOL, ATOL)
             assert bad == [], bad
         model.close()
+
+
+def _states(model):
+    return {k: model.get(k) for k in ("SNOWPACK", "SOILMOIST", "UNSATSTW", "SATSTW",
+                                      "TOTAL_RUNOFF")}
+
+
+def test_marks_go_with_the_forcing_that_gave_them():
+    """Whole-range forcing without odd days leaves no trace of the odd ones
+    before it: the states are those of a context that never had them, bit for
+    bit (an ordinary cell that took the branches would differ by roundings)."""
+    print("case: odd weather replaced", flush=True)
+    got = []
+    for odd_first in (False, True):
+        dom = _domain(4)
+        model, _, steps, _ = make_pair([dom], n_steps=96, seed=74, route=False)
+        pre = np.abs(dom.forcing["PRE"]) % 40.0
+        if odd_first:
+            model.run(steps[:24], steps_per_launch=12, want_gauges=False)
+            model.set_meteo_weights(*[-v for v in synth.make_meteo_weights(dom.n_cells, 75)])
+            model.set_meteo_weights()
+            model.default_states()
+        model.set_forcing("PRE", pre)
+        model.run(steps, steps_per_launch=12, want_gauges=False)
+        got.append(_states(model))
+        model.close()
+    for k in got[0]:
+        assert np.array_equal(got[0][k], got[1][k]), k
+
+
+def test_marks_follow_the_cells_when_the_network_is_bound():
+    """Binding a network re-lays the cells; the marks go with them."""
+    print("case: odd weather before the network", flush=True)
+    got = []
+    for late in (False, True):
+        dom = _domain(4)
+        steps = calendar.step_table(START, 96, 1)
+        model = engine.Model([dom], n_forcing_days=4)
+        if not late:
+            model.bind_network()
+        model.set_params(synth.cell_params(dom, PM.DEFAULT), 0)
+        model.default_states()
+        model.set_domain_forcing()
+        if late:
+            model.bind_network()
+        model.set_routing_params(PM.routing_gamma(PM.DEFAULT), 0)
+        model.run(steps, steps_per_launch=12)
+        got.append(_states(model))
+        model.close()
+    for k in got[0]:
+        assert np.array_equal(got[0][k], got[1][k]), k
