@@ -582,9 +582,14 @@ __device__ __forceinline__ void ordinary_step(const CellArgs &a, uint32_t bv, Ce
 // The cell's loads are issued before the log / exp tables are filled, so the
 // fill's reads and barrier wait behind them rather than in front.
 //
-// A cell outside the ordinary ranges reloads everything and takes
-// general_step: out of line, so that the registers of the kernel are those of
-// the ordinary step (four waves per SIMD).
+// Bound by the memory it reads and writes (700x900 cells, 3 horizons: 55 us at
+// 5.6 TB/s).  A cell outside the ordinary ranges takes the branches in the
+// same kernel, from the same loads; the end of the step stands in both ways,
+// so that nothing but the step's start is live where they part (four waves
+// per SIMD, no spilled registers at up to 3 horizons).  With the branches in a
+// function of their own, which saves the caller's registers and loads the cell
+// again, 512x512 cells took 91 us a step where all are such cells, 57 with one
+// in 64 and 34 with none; now 31, 34 and 31.
 struct StepArgs {
   StepDev st;
   int64_t t;
@@ -616,31 +621,6 @@ __device__ __forceinline__ void step_start(const CellArgs &a, const StepDev &st,
 }
 
 template <int NH, bool JV, bool OUT>
-__device__ __attribute__((noinline)) void general_step(ConstArgs *args, uint32_t c, uint32_t bv) {
-  ConstArgs *k = uniform(args);
-  const CellArgs a = read_args(k);
-  const __attribute__((address_space(4))) StepArgs *sa =
-      (const __attribute__((address_space(4))) StepArgs *)(k + 1);
-  const StepDev st = read_step(&sa->st);
-  const uint32_t bc = c * 8u;
-  CellRegs<NH> r;
-  FluxRegs<NH> x;
-  load_params<NH, JV>(a, bv, r);
-  load_states<NH>(a, bv, r);
-  const double pre = ldr(frow_ptr(a, MHMHIP_F_PRE, st.day), bc);
-  const double tavg = ldr(frow_ptr(a, MHMHIP_F_TAVG, st.day), bc);
-  const double tmax = a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMAX, st.day), bc) : 0.0;
-  const double tmin = a.pet_case == 1 ? ldr(frow_ptr(a, MHMHIP_F_TMIN, st.day), bc) : 0.0;
-  step_start<NH>(a, st, bc, bv, pre, tavg, tmax, tmin, r, x);
-  const double maxinter = ldr(a.P + (int64_t)(pr_maxinter(NH) + st.month0) * a.ld, bv);
-  chain_step<NH, JV>(r, x, maxinter, 1.0 / maxinter, st.evap, st.revap,
-                     stress_of<NH, JV>(r, false));
-  store_fluxes<NH>(a, bv, x);
-  step_end<NH, JV, OUT>(k, a, c, bv, sa->t, a.ring ? runoff_scale(a, bc) : 0.0,
-                        a.ring && a.lag ? a.lag[c] : 0, r, x);
-}
-
-template <int NH, bool JV, bool OUT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NH > 3 ? 2 : OUT ? 3 : 4)))
 void cell_step_kernel(CellArgs a, StepArgs sa) {
   static_assert(sizeof(CellArgs) % alignof(StepArgs) == 0, "StepArgs follows CellArgs");
@@ -662,22 +642,26 @@ void cell_step_kernel(CellArgs a, StepArgs sa) {
   mathtab_fill();  // the chain's powers read it (every thread, before any returns)
   if (!act) return;
   const bool ordinary = ordinary_cell<NH, JV>(r, st.init_sm != 0, odd);
+  step_start<NH>(a, st, bc, bv, pre, tavg, tmax, tmin, r, x);
+  // after the daily PET's call, which they would have to be kept across
+  double maxinter = ldr(a.P + (int64_t)(pr_maxinter(NH) + st.month0) * a.ld, bv);
+  double scale = a.ring ? runoff_scale(a, bc) : 0.0;
+  int32_t g = a.ring && a.lag ? a.lag[c] : 0;
+  // no load is waited for once the stores start: they share a counter
+  settle(maxinter);
+  settle(scale);
+  asm volatile("" : "+v"(g));
+  settle_all<NH>(r);
   if (ordinary) {
-    double scale = a.ring ? runoff_scale(a, bc) : 0.0;
-    int32_t g = a.ring && a.lag ? a.lag[c] : 0;
-    step_start<NH>(a, st, bc, bv, pre, tavg, tmax, tmin, r, x);
-    double maxinter = ldr(a.P + (int64_t)(pr_maxinter(NH) + st.month0) * a.ld, bv);
-    // no load is waited for once the stores start: they share a counter
-    settle(maxinter);
-    settle(scale);
-    asm volatile("" : "+v"(g));
-    settle_all<NH>(r);
     ordinary_step<NH, JV>(a, bv, r, x, maxinter, maxinter > kEps ? 1.0 / maxinter : 0.0,
                           div_rcp(x.pet, st.evap, st.revap), stress_of<NH, JV>(r, true));
     step_end<NH, JV, OUT>(kernel_args(), a, c, bv, sa.t, scale, g, r, x);
+  } else {
+    chain_step<NH, JV>(r, x, maxinter, 1.0 / maxinter, st.evap, st.revap,
+                       stress_of<NH, JV>(r, false));
+    store_fluxes<NH>(a, bv, x);
+    step_end<NH, JV, OUT>(kernel_args(), a, c, bv, sa.t, scale, g, r, x);
   }
-  // last, where the call finds no other value in use
-  if (!ordinary) general_step<NH, JV, OUT>(kernel_args(), opaque(c), opaque(bv));
 }
 
 // Per-lane LDS slots of the fused kernel (dynamic shared memory,
@@ -1031,8 +1015,12 @@ __device__ __forceinline__ void fused_ordinary(const CellArgs &a, FusedLane &u, 
   if (OUT) store_sums(k, a.ld, u.bv, u.slot + LS_STRESS + stress_slots(NH, JV));
 }
 
-// The time loop of any other cell, out of line and from its own loads (see
-// general_step): the registers of the kernel are those of the ordinary loop.
+// The time loop of any other cell, out of line and from its own loads: the
+// registers of the kernel are those of the ordinary loop (in one kernel the two
+// loops need 156, three waves per SIMD, and 1024x1024 ordinary cells take 1301
+// instead of 1142 us per 144 steps).  A wave with such cells runs both loops:
+// 512x512 cells, 24 steps 85 us without them, 180 with one in 64, 200 where all
+// are.
 struct FusedArgs {
   int64_t t0;
   int32_t nsteps, step0;
