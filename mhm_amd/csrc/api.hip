@@ -1297,7 +1297,6 @@ CellArgs cell_args(mhmhip_ctx *x, bool ring) {
   a.ring = ring ? x->d_ring : nullptr;
   a.area = x->d_area;
   a.tst = kHourSecs * (double)x->cfg.timestep;  // mo_mrm_pre_routing.f90:110
-  a.rtst = 1.0 / a.tst;
   a.steps = x->d_steps;
   a.n_cells = x->n_cells;
   a.sstride = x->sstride;
@@ -1379,14 +1378,6 @@ RouteArgs route_args(mhmhip_ctx *x, int64_t t_lo, int64_t t_hi, int64_t t_base) 
   r.rep = 1;
   r.acc_from = 0;
   return r;
-}
-
-// Largest tree (nodes of one domain) for the workgroup-resident routing.
-int64_t max_domain_nodes(const mhmhip_ctx *x) {
-  int64_t m = 0;
-  for (int d = 0; d < x->n_domains; ++d)
-    m = std::max(m, x->dom_node_start[d + 1] - x->dom_node_start[d]);
-  return m;
 }
 
 // Routing kernel for a route_mode: 1 grid diagonals, 2 workgroup-resident

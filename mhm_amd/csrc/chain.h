@@ -17,12 +17,8 @@ namespace mhmhip {
 
 // src/common/mo_common_constants.f90: eps_dp = epsilon(1.0_dp)
 constexpr double kEps = DBL_EPSILON;
-// FORCES mo_constants: twothird_dp
 // src/mHM/mo_mhm_constants.f90:36-39
 constexpr double kHarSamConst = 17.800;
-constexpr double kDuffieDr = 0.0330;
-constexpr double kDuffieDelta1 = 0.4090;
-constexpr double kDuffieDelta2 = 1.3900;
 // FORCES mo_constants: DaySecs / PI_D / SpecHeatET_dp * SolarConst_dp, folded
 // left to right exactly as the reference expression (mo_pet.f90:353).
 constexpr double kPi = 3.141592653589793238462643383279502884197;
@@ -59,8 +55,6 @@ __host__ __device__ inline double fma_k(double a, double b, double c) {
 // ln 2 split so that k * kLn2Hi is exact for |k| < 2^21 (32 significant bits)
 constexpr double kLn2Hi = 0x1.62e42fee00000p-1;
 constexpr double kLn2Lo = 0x1.a39ef35793c76p-33;
-constexpr double kInvLn2 = 1.4426950408889634;    // RN(1/ln 2)
-constexpr double kSqrtHalf = 0x1.6a09e667f3bcdp-1;  // RN(sqrt(1/2))
 
 // N doubles passed and returned by value (registers across an out-of-line call)
 template <int N>
@@ -90,23 +84,24 @@ __shared__ __attribute__((aligned(16))) double s_mathtab[kPowLogN * 2 + kExpTabN
 
 // Every workgroup of a kernel that evaluates a power or an exp calls this
 // before the first one (all threads, before any of them returns).  The
-// tables (base-2 logarithm rows and 2^(j/256), 6 KB) are copied in 16-byte
-// pieces, a thread's first three loads issued before its stores, so that the
-// copy waits for memory once.
+// tables (2^(j/256) and base-2 logarithm rows, 6 KB) are copied in 16-byte
+// pieces, one a row, a thread's first three loads issued before its stores, so
+// that the copy waits for memory once.  The logarithm's rows come first in LDS.
 __device__ inline void mathtab_fill() {
 #if defined(__HIP_DEVICE_COMPILE__)
-  constexpr int n = (kPowLogN * 2 + kExpTabN * 2) / 2;
-  const double2 *src = reinterpret_cast<const double2 *>(kPowTab);
+  constexpr int n = kPowLogN + kExpTabN;
+  const double2 *src = reinterpret_cast<const double2 *>(kMathTab + kExpTabOff);
   double2 *dst = reinterpret_cast<double2 *>(s_mathtab);
   const int i0 = threadIdx.x, bs = blockDim.x;
+  auto place = [](int i) { return i < kExpTabN ? i + kPowLogN : i - kExpTabN; };
   // pieces past the table copy its last piece again (no branch between the
   // loads: the stores of one value to one place)
   double2 v[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) v[k] = src[min(i0 + k * bs, n - 1)];
 #pragma unroll
-  for (int k = 0; k < 3; ++k) dst[min(i0 + k * bs, n - 1)] = v[k];
-  for (int i = i0 + 3 * bs; i < n; i += bs) dst[i] = src[i];
+  for (int k = 0; k < 3; ++k) dst[place(min(i0 + k * bs, n - 1))] = v[k];
+  for (int i = i0 + 3 * bs; i < n; i += bs) dst[place(i)] = src[i];
   __syncthreads();
 #endif
 }
@@ -119,11 +114,17 @@ __host__ __device__ inline const double *powtab() {
 #if defined(__HIP_DEVICE_COMPILE__)
   return s_mathtab;
 #else
-  return kPowTab;
+  return kMathTab + kExpTabOff + kExpTabN * 2;
 #endif
 }
 
-__host__ __device__ inline const double *exptab() { return powtab() + kPowExpOff; }
+__host__ __device__ inline const double *exptab() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return s_mathtab + kPowLogN * 2;
+#else
+  return kMathTab + kExpTabOff;
+#endif
+}
 
 template <int N>
 __host__ __device__ inline DV<N> log_pos_v(const DV<N> &x) {
@@ -335,10 +336,6 @@ __device__ __forceinline__ double pow_pos_from(double x, double px) {
   return x == 0.0 ? 0.0 : __builtin_nan("");
 }
 
-__device__ __forceinline__ double pow_pos(double x, double y) {
-  return pow_pos_from(x, x > 0.0 ? exp_ylogx(y, x) : 0.0);
-}
-
 // FORCES mo_utils LE: a <= b within eps*|b| (pre-proc/mtCLIM/mo_utils.f90:922-934)
 __device__ __forceinline__ bool le_eps(double a, double b) {
   return !(((DBL_EPSILON * fabs(b) - fabs(a - b)) < 0.0) && (a > b));
@@ -362,11 +359,6 @@ __device__ __forceinline__ bool le_eps(double a, double b) {
 __device__ __forceinline__ double vmin(double a, double b) {
   double d;
   asm("v_min_f64 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
-  return d;
-}
-__device__ __forceinline__ double vmax(double a, double b) {
-  double d;
-  asm("v_max_f64 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
   return d;
 }
 // max(a, 0) and min(a, 1) with the bound an inline constant, and max(a, k) for
@@ -558,15 +550,6 @@ __device__ __forceinline__ void runoff_slow_perc(double k1, double kp, double ka
   const double p = vmin(perc, unsat);  // the whole store when perc exceeds it
   sat = sat + p * karst;
   unsat = unsat - p;
-}
-
-__device__ __forceinline__ void runoff_unsat_zone(double k1, double kp, double k0, double alpha,
-                                                  double karst, double pin, double thr,
-                                                  double &sat, double &unsat, double &slow,
-                                                  double &fast, double &perc) {
-  runoff_fast(k0, pin, thr, unsat, fast);
-  runoff_slow_perc(k1, kp, karst, unsat > 0.0 ? exp_ylogx(1.0 + alpha, unsat) : 0.0, sat, unsat,
-                   slow, perc);
 }
 
 // src/mHM/mo_runoff.f90:191-212

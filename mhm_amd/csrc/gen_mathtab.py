@@ -1,5 +1,5 @@
-"""Writes mathtab.h: the tables of the chain's logarithm and exponential
-(chain.h, log_pos_v and exp_fin_v).
+"""Writes mathtab.h: the tables of the chain's logarithm, exponential and power
+(chain.h, log_pos_v, exp_fin_v and pow_v).
 
 Logarithm, F_j = j / 256 for j = 128..256 (F from 1/2 to 1, the nearest
 point to the frexp mantissa m in [1/2, 1)): RN(1 / F_j) and log(F_j) split as
@@ -21,8 +21,9 @@ elementary functions: a new approach for achieving high accuracy and good
 performance", LNCS 235 (1986) 1-16): one double holds it, and e + L is exact
 for the exponent e of every finite double, also where the two nearly cancel (x
 just above 1).  The first row has R = 2 and the last R = 1, both with exact
-logarithms, so that log2 x is 0 at x = 1.  Then 2^(j/256) as above, and the
-coefficients of log2(1 + u) = u (c0 + ... + c5 u^5) on [-1/256, 1/128] and of
+logarithms, so that log2 x is 0 at x = 1.  These rows stand behind those of
+2^(j/256), which the power uses too: the cell kernels copy both to LDS in one
+piece.  And the coefficients of log2(1 + u) = u (c0 + ... + c5 u^5) on [-1/256, 1/128] and of
 2^(r/256) = 1 + r (d0 + ... + d3 r^3) on [-1/2, 1/2], interpolated at Chebyshev
 nodes; main() checks that log2(1 + u) and 2^(r/256) come out with relative
 errors below 2^-51.8 and 2^-57.5.
@@ -108,8 +109,9 @@ def main():
     print("constexpr int kLogTabJ0 = %d;" % LOG_J0)
     print("constexpr int kLogTabN = %d;" % (LOG_J1 - LOG_J0 + 1))
     print("constexpr int kExpTabN = %d;" % EXP_N)
-    print("constexpr int kExpTabOff = kLogTabN * 4;  // the exp rows' first element")
-    print("alignas(16) constexpr double kMathTab[kLogTabN * 4 + kExpTabN * 2] = {")
+    print("constexpr int kPowLogN = 128;")
+    print("constexpr int kExpTabOff = kLogTabN * 4;  // the exp rows' first element, then the power's")
+    print("alignas(16) constexpr double kMathTab[kLogTabN * 4 + kExpTabN * 2 + kPowLogN * 2] = {")
     print("    // log: {RN(1/F), hi(log F), lo(log F), 0} for F = j/256, j = %d..%d"
           % (LOG_J0, LOG_J1))
     for j in range(LOG_J0, LOG_J1 + 1):
@@ -119,17 +121,9 @@ def main():
     for j in range(EXP_N):
         hi, lo = exp_row(j)
         print("    %s, %s," % (hi.hex(), lo.hex()))
-    print("};")
-    print("constexpr int kPowLogN = 128;")
-    print("constexpr int kPowExpOff = kPowLogN * 2;  // the 2^(j/256) rows' first element")
-    print("alignas(16) constexpr double kPowTab[kPowLogN * 2 + kExpTabN * 2] = {")
-    print("    // {R, L}: log2(m) = L + log2(m R), by interval of m")
+    print("    // power: {R, L}, log2(m) = L + log2(m R), by interval of m")
     for j in range(128):
         print("    %s, %s," % tuple(v.hex() for v in pow_row(j)))
-    print("    // {hi, lo} of 2^(j/%d), j = 0..%d" % (EXP_N, EXP_N - 1))
-    for j in range(EXP_N):
-        hi, lo = exp_row(j)
-        print("    %s, %s," % (hi.hex(), lo.hex()))
     print("};")
     half, u0, u1 = mp.mpf(1) / 2, -mp.mpf(1) / 256, mp.mpf(1) / 128
     c = chebyshev_fit(lambda u: mp.log(1 + u, 2) / u, u0, u1, 6)

@@ -23,8 +23,6 @@
 
 namespace mhmhip {
 
-constexpr int kMaxH = 6;
-
 // parameter rows (device).  Divisions and scalings the reference performs
 // every step on step-invariant operands are done once on the host
 // (bit-identical): DMAXS = degDayMax*c2TSTu, DNPS = degDayNoPre*c2TSTu,
@@ -107,7 +105,6 @@ struct OutAcc {
   uint64_t mask;             // selected bits
   int32_t n;                 // their number
 };
-__host__ __device__ constexpr int out_bits(int nh) { return 16 + 4 * nh; }
 // The bit of output k (horizon h, 0-based, for those per horizon); -1: none.
 __host__ __device__ constexpr int out_bit(int k, int h, int nh) {
   return k == 1 ? 0 : k == 2 ? 1 : k == 9 ? 2 : k == 20 ? 3 : k == 21 ? 4
@@ -127,7 +124,9 @@ struct CellArgs {
   const double *area;      // [n_cells] L1 cell area [km2] (routing input)
   const uint8_t *lag;      // [n_cells] ring lag of the node (tiled routing), null: 0
   double tst;              // HourSecs * timestep [s]
-  double rtst;             // RN(1 / tst)
+  // [n_cells] OddWeather bits: what was given for the cell outside the ranges
+  // that the branch-free form covers (forcing_scan_kernel); 0: nothing
+  const uint8_t *odd_weather;
   const StepDev *steps;    // device step table (fused kernel)
   int64_t n_cells;
   int64_t sstride;
@@ -149,9 +148,6 @@ struct CellArgs {
   const double *sun;
   int32_t sun_step0;       // step of its first pair of rows
   int32_t skip_fluxes;     // 1: a later launch of the call writes the flux rows
-  // [n_cells] OddWeather bits: what was given for the cell outside the ranges
-  // that the branch-free form covers (forcing_scan_kernel); 0: nothing
-  const uint8_t *odd_weather;
   // meteo weights [3][12 * 24][sstride] (pre, temp, pet), null: the day/night
   // factors disaggregate
   const double *W;

@@ -85,7 +85,7 @@ __device__ __forceinline__ ConstArgs *rare(ConstArgs *p) {
 __device__ __forceinline__ CellArgs read_args(ConstArgs *p) {
   CellArgs a;
   a.P = p->P, a.S = p->S, a.X = p->X, a.F = p->F, a.ring = p->ring, a.area = p->area;
-  a.lag = p->lag, a.tst = p->tst, a.rtst = p->rtst, a.steps = p->steps;
+  a.lag = p->lag, a.tst = p->tst, a.steps = p->steps;
   a.n_cells = p->n_cells, a.sstride = p->sstride, a.ld = p->ld;
   a.forcing_days = p->forcing_days, a.ring_len = p->ring_len, a.pet_case = p->pet_case;
   a.jarvis = p->jarvis, a.hourly = p->hourly, a.ring_rep = p->ring_rep;
