@@ -2,8 +2,8 @@
 
   mhm_amd/libmhmhip.so  HIP kernels + C-ABI (include/mhmhip.h), gfx950
   mhm_amd/libmhmsyn.so  host-only synthetic-domain tools (priority-flood D8)
-  tests/native/libmhmcheck.so  host + device evaluation of the chain's log/exp/pow
-                               (test-only, built from tests/native/mathcheck.hip)
+  tests/native/libmhmcheck.so  the chain's log/exp/pow and step by themselves
+                               (test-only, built from tests/native/*.hip)
   mhm_amd/fortran/mhmhip_driver  Fortran host on the iso_c_binding module
 
 Run ``python -m mhm_amd.build`` (or ``__graft_entry__.build()``).
@@ -79,15 +79,21 @@ TEST_NATIVE = os.path.join(ROOT, "tests", "native")
 CHECK_LIB = os.path.join(TEST_NATIVE, "libmhmcheck.so")
 
 
+CHECK_SOURCES = ["mathcheck.hip", "formcheck.hip"]
+
+
 def build_check():
-    """Host + device evaluation of the chain's log/exp/pow (accuracy tests)."""
-    obj = os.path.join(OBJ, "mathcheck.hip.o")
+    """Host + device evaluation of the chain's log/exp/pow and the device
+    evaluation of both forms of its step (accuracy tests)."""
     os.makedirs(OBJ, exist_ok=True)
     hipcc = _hipcc()
-    _run([hipcc] + hip_flags() + ["-c", "-x", "hip", os.path.join(TEST_NATIVE, "mathcheck.hip"),
-                                  "-o", obj])
+    objs = [os.path.join(OBJ, src + ".o") for src in CHECK_SOURCES]
+    jobs = [[hipcc] + hip_flags() + ["-c", "-x", "hip", os.path.join(TEST_NATIVE, src), "-o", o]
+            for src, o in zip(CHECK_SOURCES, objs)]
+    with ThreadPoolExecutor(max_workers=len(jobs)) as ex:
+        list(ex.map(_run, jobs))
     tmp = CHECK_LIB + ".tmp"
-    _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, obj])
+    _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp] + objs)
     os.replace(tmp, CHECK_LIB)
     return CHECK_LIB
 

@@ -585,10 +585,11 @@ constexpr double kBig = 1e15;   // parameters beyond this are not ordinary
 constexpr double kTiny = 1e-15;
 
 // x**(2/3) of a canopy ratio (pow23 without its exponent handling): the seed
-// in single precision straight from x, in range for x >= 2^-32, where its
-// error stays below 2^-18 and the Halley step's below 2^-56.  Smaller
-// ratios go through pow23; 0, negative and NaN ratios give NaN (the caller's
-// maximum with 0 then gives 0, as for the reference's power of them).
+// in single precision straight from x, in range for x >= 2^-32, where the
+// rounding of log2 x leaves its error below 2^-19.7 and the Halley step's below
+// 2^-56 (pow23's 2^-62); within 3 ulp of the exact power like pow23.  Smaller
+// ratios go through pow23; 0, negative and NaN ratios give NaN or -inf (the
+// caller's maximum with 0 then gives 0, as for the reference's power of them).
 __device__ __forceinline__ double pow23_ratio(double x) {
   const float f = (float)x;
   const double y =
