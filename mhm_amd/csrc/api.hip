@@ -86,6 +86,7 @@ struct mhmhip_ctx {
   int32_t frow[MHMHIP_F_COUNT] = {};
   int32_t n_frows = 0;
   uint8_t *d_odd = nullptr;  // [sstride] OddWeather marks of the cells
+  int32_t odd_given = 0;     // bits that forcing given so far may have set in them
   double *W = nullptr;  // meteo weights [3][12 * 24][sstride], null: off
   // MPR-lite inputs (mhmhip_mprlite_inputs): host copies in reference cell
   // order, and the kernel's input rows laid out as the cells are (rebuilt
@@ -157,6 +158,7 @@ struct mhmhip_ctx {
   // work queued before it (which may still read them) is done.
   std::vector<int32_t> col_day;
   std::vector<int64_t> col_seq;
+  std::vector<uint8_t> col_scanned;  // 0: streamed, its weather not looked at yet
   std::vector<hipEvent_t> chunk_ev;
   int64_t waited_seq = -1;
   hipStream_t cstream = nullptr;
@@ -437,6 +439,7 @@ extern "C" int mhmhip_create(const mhmhip_config *cfg, mhmhip_ctx **out) {
   x->col_day.resize(c.n_forcing_days);
   for (int32_t k = 0; k < c.n_forcing_days; ++k) x->col_day[k] = k + 1;
   x->col_seq.assign(c.n_forcing_days, -1);
+  x->col_scanned.assign(c.n_forcing_days, 1);
   int rc = MHMHIP_OK;
   if (hipStreamCreateWithFlags(&x->stream, hipStreamNonBlocking) != hipSuccess) {
     g_create_error = "create: stream creation failed";
@@ -858,30 +861,50 @@ int forcing_columns_direct(mhmhip_ctx *x, int32_t day0, int32_t ndays) {
   return MHMHIP_OK;
 }
 
-// After n columns of a variable from col on were written on stream s: marks the
-// cells with odd weather in them.  whole: the variable has no other column, so
-// that marks of what it held before go.
-int scan_forcing(mhmhip_ctx *x, int32_t var, int32_t col, int32_t n, bool whole, hipStream_t s) {
-  if (var != MHMHIP_F_PRE && var != MHMHIP_F_TAVG) return MHMHIP_OK;
-  const int32_t bit = var == MHMHIP_F_PRE ? OW_PRE : OW_TAVG;
-  if (whole) CHECK_HIP(x, launch_odd_clear(x->sstride, bit, x->d_odd, s), "forcing scan");
-  const double *rows =
-      x->F + ((int64_t)x->frow[var] * x->cfg.n_forcing_days + col) * x->sstride;
-  CHECK_HIP(x, launch_forcing_scan(rows, x->sstride, n, x->n_cells, var == MHMHIP_F_TAVG, bit,
-                                   x->d_odd, s),
+// Marks the cells with odd weather in the columns [col, col + n) of the
+// variables with these bits (OW_PRE, OW_TAVG), on the compute stream: the marks
+// change between its launches, not under them.  whole: the variables have no
+// other columns, so that marks of what they held before go.
+int scan_forcing(mhmhip_ctx *x, int32_t bits, int32_t col, int32_t n, bool whole) {
+  if (whole && (x->odd_given & bits))
+    CHECK_HIP(x, launch_odd_clear(x->sstride, bits, x->d_odd, x->stream), "forcing scan");
+  x->odd_given |= bits;
+  auto rows = [&](int32_t bit, int32_t var) {
+    return bits & bit
+               ? x->F + ((int64_t)x->frow[var] * x->cfg.n_forcing_days + col) * x->sstride
+               : nullptr;
+  };
+  CHECK_HIP(x, launch_forcing_scan(rows(OW_PRE, MHMHIP_F_PRE), rows(OW_TAVG, MHMHIP_F_TAVG),
+                                   x->sstride, n, x->n_cells, OW_PRE, x->d_odd, x->stream),
             "forcing scan");
   return MHMHIP_OK;
 }
 
+int32_t odd_bit(int32_t var) {
+  return var == MHMHIP_F_PRE ? OW_PRE : var == MHMHIP_F_TAVG ? OW_TAVG : 0;
+}
+
 // The compute stream waits for the streamed chunks that wrote the columns
 // the steps read (chunks complete in order on the copy stream: waiting for
-// the newest is enough).
+// the newest is enough) and looks at their weather.
 int forcing_wait(mhmhip_ctx *x, const StepDev *st, int64_t n) {
   int64_t newest = -1;
   for (int64_t k = 0; k < n; ++k) newest = std::max(newest, x->col_seq[st[k].day]);
   if (newest > x->waited_seq) {
     CHECK_HIP(x, hipStreamWaitEvent(x->stream, x->chunk_ev[newest], 0), "forcing wait");
     x->waited_seq = newest;
+  }
+  // streamed columns read for the first time, neighbours together
+  for (int64_t k = 0; k < n; ++k) {
+    const int32_t col = st[k].day;
+    if (x->col_scanned[col]) continue;
+    int64_t e = k;
+    x->col_scanned[col] = 1;
+    while (e + 1 < n && (st[e + 1].day == st[e].day ||
+                         (st[e + 1].day == st[e].day + 1 && !x->col_scanned[st[e + 1].day])))
+      x->col_scanned[st[++e].day] = 1;
+    CHECK_RC(scan_forcing(x, OW_PRE | OW_TAVG, col, st[e].day - col + 1, false));
+    k = e;
   }
   return MHMHIP_OK;
 }
@@ -974,12 +997,6 @@ extern "C" int mhmhip_stream_forcing(mhmhip_ctx *x, int32_t day0, int32_t ndays,
     CHECK_HIP(x, launch_forcing_gather(x->fstage_d[i], map, ndays, x->n_cells, x->d_pos, x->F, nfd,
                                        day0 - 1, x->sstride, x->cstream),
               "stream_forcing gather");
-  const int32_t col0 = (day0 - 1) % nfd, n0 = std::min(ndays, nfd - col0);
-  for (int32_t v : {MHMHIP_F_PRE, MHMHIP_F_TAVG})
-    if (host[v]) {
-      CHECK_RC(scan_forcing(x, v, col0, n0, ndays == nfd, x->cstream));
-      CHECK_RC(scan_forcing(x, v, 0, ndays - n0, false, x->cstream));
-    }
   hipEvent_t done = nullptr;
   CHECK_HIP(x, hipEventCreateWithFlags(&done, hipEventDisableTiming), "stream_forcing event");
   x->chunk_ev.push_back(done);
@@ -989,6 +1006,7 @@ extern "C" int mhmhip_stream_forcing(mhmhip_ctx *x, int32_t day0, int32_t ndays,
     const int32_t col = (day0 - 1 + j) % nfd;
     x->col_day[col] = day0 + j;
     x->col_seq[col] = seq;
+    x->col_scanned[col] = 0;  // forcing_wait
   }
   return MHMHIP_OK;
 }
@@ -1009,7 +1027,8 @@ extern "C" int mhmhip_set_forcing(mhmhip_ctx *x, int32_t var, int32_t day0, int3
         x->F + ((int64_t)x->frow[var] * x->cfg.n_forcing_days + (day0 - 1 + j)) * x->sstride;
     CHECK_RC(put_row(x, dst, host + (int64_t)j * ld, id));
   }
-  CHECK_RC(scan_forcing(x, var, day0 - 1, ndays, ndays == x->cfg.n_forcing_days, x->stream));
+  if (odd_bit(var))
+    CHECK_RC(scan_forcing(x, odd_bit(var), day0 - 1, ndays, ndays == x->cfg.n_forcing_days));
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "set_forcing");
   return MHMHIP_OK;
 }
@@ -1140,8 +1159,9 @@ extern "C" int mhmhip_set_forcing_l2(mhmhip_ctx *x, int32_t var, int32_t domain,
   double *dst = x->F + ((int64_t)x->frow[var] * x->cfg.n_forcing_days + (day0 - 1)) * x->sstride;
   CHECK_HIP(x, launch_meteo_l2(b.data2, b.mask2, nr2, n2, b.cells, ncells, ndays, dst, x->sstride,
                                aggregate, x->stream), "set_forcing_l2 map");
-  CHECK_RC(scan_forcing(x, var, day0 - 1, ndays,
-                        x->n_domains == 1 && ndays == x->cfg.n_forcing_days, x->stream));
+  if (odd_bit(var))
+    CHECK_RC(scan_forcing(x, odd_bit(var), day0 - 1, ndays,
+                          x->n_domains == 1 && ndays == x->cfg.n_forcing_days));
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "set_forcing_l2");
   return MHMHIP_OK;
 }
@@ -1231,11 +1251,9 @@ extern "C" int mhmhip_set_meteo_weights(mhmhip_ctx *x, const double *pre_w,
       for (int h = 0; h < 24; ++h)
         CHECK_RC(put_row(x, x->W + ((int64_t)v * 288 + m * 24 + h) * x->sstride,
                          host[v] + ld * ((int64_t)m + 12 * h), id));
-  for (int v = 0; v < 2; ++v)  // precipitation, temperature
-    CHECK_HIP(x, launch_forcing_scan(x->W + (int64_t)v * 288 * x->sstride, x->sstride, 288,
-                                     x->n_cells, v == 1, v == 0 ? OW_PRE_WEIGHT : OW_TEMP_WEIGHT,
-                                     x->d_odd, x->stream),
-              "set_meteo_weights");
+  CHECK_HIP(x, launch_forcing_scan(x->W, x->W + (int64_t)288 * x->sstride, x->sstride, 288,
+                                   x->n_cells, OW_PRE_WEIGHT, x->d_odd, x->stream),
+            "set_meteo_weights");
   CHECK_HIP(x, hipStreamSynchronize(x->stream), "set_meteo_weights");
   return MHMHIP_OK;
 }

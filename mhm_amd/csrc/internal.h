@@ -69,6 +69,8 @@ enum StepChange {
   SC_INIT = 8,   // the step resets the soil moisture (init_sm)
 };
 
+// What odd weather came from (CellArgs::odd_weather): precipitation and
+// temperature of the forcing, of the meteo weights, the day and night factors.
 enum OddWeather { OW_PRE = 1, OW_TAVG = 2, OW_PRE_WEIGHT = 4, OW_TEMP_WEIGHT = 8, OW_FACTOR = 16 };
 
 // Per-step scalars on the device (host-evaluated from the step clock).

@@ -2119,22 +2119,26 @@ hipError_t launch_row_gather(const double *row, const int32_t *pos, double *out,
   return hipGetLastError();
 }
 
-// Marks the cells whose n_rows rows of precipitation or temperature hold a value
-// outside [lowest, kBig) with bit (CellArgs::odd_weather).  For the others the
-// degree-day factor is not below zero at any step.
-__global__ __launch_bounds__(256) void forcing_scan_kernel(const double *rows, int64_t stride,
-                                                           int32_t n_rows, int64_t n_cells,
-                                                           double lowest, int32_t bit,
+// Marks the cells whose n_rows rows of precipitation (pre) hold a value outside
+// [0, kBig) with bit, those whose rows of temperature (temp) hold one outside
+// (-kBig, kBig) with 2 bit (CellArgs::odd_weather); either may be null.  For the
+// other cells the degree-day factor is not below zero at any step.
+__global__ __launch_bounds__(256) void forcing_scan_kernel(const double *pre, const double *temp,
+                                                           int64_t stride, int32_t n_rows,
+                                                           int64_t n_cells, int32_t bit,
                                                            uint8_t *odd) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= n_cells) return;
-  bool ok = true;
+  bool odd_pre = false, odd_temp = false;
   for (int32_t t = blockIdx.y; t < n_rows; t += gridDim.y) {
-    const double v = rows[(int64_t)t * stride + c];
-    ok = ok & (v >= lowest) & (v < kBig);
+    if (pre) {
+      const double v = pre[(int64_t)t * stride + c];
+      odd_pre = odd_pre | !(v >= 0.0) | !(v < kBig);
+    }
+    if (temp) odd_temp = odd_temp | !(fabs(temp[(int64_t)t * stride + c]) < kBig);
   }
-  // marks are given from two streams
-  if (!ok) atomicOr(reinterpret_cast<uint32_t *>(odd) + c / 4, (uint32_t)bit << 8 * (c % 4));
+  const uint32_t bits = (odd_pre ? bit : 0) | (odd_temp ? 2 * bit : 0);
+  if (bits) atomicOr(reinterpret_cast<uint32_t *>(odd) + c / 4, bits << 8 * (c % 4));
 }
 
 // Takes bits out of the marks (n: a multiple of 4).
@@ -2143,13 +2147,13 @@ __global__ __launch_bounds__(256) void odd_clear_kernel(int64_t n, int32_t bits,
   if (w < n / 4) atomicAnd(reinterpret_cast<uint32_t *>(odd) + w, ~((uint32_t)bits * 0x01010101u));
 }
 
-hipError_t launch_forcing_scan(const double *rows, int64_t stride, int32_t n_rows, int64_t n_cells,
-                               bool temperature, int32_t bit, uint8_t *odd, hipStream_t s) {
-  if (n_rows < 1) return hipSuccess;
-  if (n_cells < 1 || !rows || !odd) return hipErrorInvalidValue;
+hipError_t launch_forcing_scan(const double *pre, const double *temp, int64_t stride,
+                               int32_t n_rows, int64_t n_cells, int32_t bit, uint8_t *odd,
+                               hipStream_t s) {
+  if (n_rows < 1 || n_cells < 1 || (!pre && !temp) || !odd) return hipErrorInvalidValue;
   const dim3 grid((unsigned)((n_cells + 255) / 256), (unsigned)(n_rows < 64 ? n_rows : 64));
-  hipLaunchKernelGGL(forcing_scan_kernel, grid, dim3(256), 0, s, rows, stride, n_rows, n_cells,
-                     temperature ? -kBig : 0.0, bit, odd);
+  hipLaunchKernelGGL(forcing_scan_kernel, grid, dim3(256), 0, s, pre, temp, stride, n_rows,
+                     n_cells, bit, odd);
   return hipGetLastError();
 }
 

@@ -33,8 +33,9 @@ hipError_t launch_state_rows(double *S, const StateValues &v, int32_t n_rows, in
                              int64_t sstride, int64_t ld, int32_t n_sets, hipStream_t s);
 hipError_t launch_row_gather(const double *row, const int32_t *pos, double *out, int64_t lo,
                              int64_t hi, hipStream_t s);
-hipError_t launch_forcing_scan(const double *rows, int64_t stride, int32_t n_rows, int64_t n_cells,
-                               bool temperature, int32_t bit, uint8_t *odd, hipStream_t s);
+hipError_t launch_forcing_scan(const double *pre, const double *temp, int64_t stride,
+                               int32_t n_rows, int64_t n_cells, int32_t bit, uint8_t *odd,
+                               hipStream_t s);
 hipError_t launch_odd_clear(int64_t n, int32_t bits, uint8_t *odd, hipStream_t s);
 hipError_t launch_forcing_gather(const double *raw, const FRowMap &m, int32_t ndays,
                                  int64_t n_cells, const int32_t *pos, double *F, int32_t n_cols,
