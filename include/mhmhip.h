@@ -182,8 +182,9 @@ typedef struct {
 /* Options of mhmhip_run. */
 typedef struct {
   int32_t mode;          /* MHMHIP_RUN_PLAIN or MHMHIP_RUN_FUSED                 */
-  int32_t steps_per_launch; /* fused path: S (0 = 24, or the days that fit the
-                            runoff ring, at most 6, where that is faster)       */
+  int32_t steps_per_launch; /* fused path: S (0 = 24, or as many times 24 steps as
+                            fit the runoff ring, at most 144, where that is
+                            faster)                                             */
   int32_t block;         /* cell-kernel block size 64/128/256 (0 = 256 fused,
                             128 plain)                                          */
   int32_t use_graph;     /* capture the tile sequence in a hipGraph              */

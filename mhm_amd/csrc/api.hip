@@ -1490,7 +1490,8 @@ int flow_check(mhmhip_ctx *x, const char *who) {
 // Measured, workgroups and steps: one launch / windows [us]: 59 x 480 (B 32)
 // 139 / 294, 296 x 720 (8) 579 / 979, 152 x 960 (8) 936 / 1504, 20 x 8760 (64)
 // 2034 / 2636, 1474 x 720 (64) 840 / 955, 2833 x 48 (8) 509 / 781, 4693 x 1440
-// (64) 4912 / 4305, 5120 x 1095 (64) 6365 / 3211.
+// (64) 4912 / 4305, 5120 x 1095 (64) 6365 / 3211.  Not in the model: gauges, the
+// number of boundaries, other contexts on the device.
 bool one_launch_pays(const mhmhip_ctx *x, int32_t B, int64_t nr, int64_t ring_rows) {
   const double groups = (double)x->lay.bins.size() * x->n_sets, H = x->tile_h;
   const double fills = std::ceil((double)nr / (double)std::max<int64_t>(1, ring_rows));
@@ -2735,8 +2736,8 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
   CHECK_RC(forcing_wait(x, hs.data(), nsteps));
   x->s_dirty = x->x_dirty = true;
   int S = o.mode == MHMHIP_RUN_PLAIN ? 1 : (o.steps_per_launch > 0 ? o.steps_per_launch : 24);
-  // default block: 256 for the fused kernel (its per-lane LDS slots fill three
-  // groups per CU), 128 for the one-step kernel (8.2e9 against 7.3e9
+  // default block: 256 for the fused kernel (with its per-lane LDS slots four
+  // groups fill a CU's LDS), 128 for the one-step kernel (8.2e9 against 7.3e9
   // cell-steps/s at 256 on the 1024x1024 basin)
   const int block = o.block > 0 ? o.block : (o.mode == MHMHIP_RUN_PLAIN ? kStepBlock : 256);
   const int kind = route_kind(o.route_mode);
@@ -2749,8 +2750,8 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
   const bool flow = tiled && one_launch_pays(x, B, nr, ring_rows), windows = tiled && !flow;
   // No steps_per_launch given: a launch of 24 steps spends a third of its time
   // before and after them (14 of 39 us with a wave per SIMD), so where the
-  // routing takes what the ring holds anyway, a launch runs as many days as fit
-  // it, at most six: 215x301 cells, 720 steps 2.47 -> 2.36 ms.
+  // routing takes what the ring holds anyway, a launch runs as many times 24 steps
+  // as fit it, at most 144, whatever the step's length: 215x301 cells, 720 steps 2.47 -> 2.36 ms.
   if (o.mode == MHMHIP_RUN_FUSED && o.steps_per_launch <= 0 && (flow || !route) && !x->coarse)
     S = std::max<int>(24, (int)std::min<int64_t>(144, route ? ring_rows / rep : 144) / 24 * 24);
   // the ring's rows in use: whole cell launches, so that no routing launch's

@@ -13,9 +13,11 @@
 // diagonal d-1; a two-slot parity buffer of routed outflow (qTR) keeps step t
 // readable while those nodes already write step t+1.  A whole run of T steps
 // takes T + dmax diagonals instead of T * dmax level sweeps.  The default
-// schedule (route_tile_kernel) runs the same diagonals inside tiles of the
-// tree, one workgroup per bin of tiles and window of steps, with the window
-// handed from tile to tile between launches; route_diag_kernel and
+// schedules run the same diagonals inside tiles of the tree, one workgroup per
+// bin of tiles: route_stream_kernel all steps of the ring in one launch, tiles
+// handing steps on while it runs, route_tile_kernel a window of steps per
+// launch, handed from tile to tile between launches (one_launch_pays in api.hip
+// chooses), route_step_kernel a single step; route_diag_kernel and
 // route_wg_kernel run them over the whole grid or inside one workgroup.
 #include <hip/hip_runtime.h>
 
@@ -1485,6 +1487,9 @@ __global__ __launch_bounds__(kTileSlots) void route_tile_kernel(RouteArgs r, Til
 // last, which holds the lowest lags, first) at 85 ns a level: an LDS write and
 // read and six to eight dependent FP64 operations.  A step of 1024x1024 nodes
 // in tiles of 32 levels, 53 deep: 473 -> 183 us; of 24x30 nodes: 27 -> 11 us.
+// Many bins do not change that (a ticket each, one counter per set), with eight
+// coupled steps in place of a launch per depth: 600 basins of 400 nodes 749 ->
+// 490 us, 2000 of 42 nodes 480 -> 255, 256 sets of 2000 nodes 1199 -> 690.
 // Levels with only their own slots unmasked took 220 us.
 //
 // Order: a workgroup's bin is its ticket, not its block index, and tickets
