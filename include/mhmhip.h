@@ -227,7 +227,10 @@ int mhmhip_default_states(mhmhip_ctx *ctx, const double *horizon_depth);
 
 /* Forcing columns day0..day0+ndays-1 (1-based) of one variable, host X(ld, ndays).
  * Replaces the meteo handler's L1_* arrays and the set_meteo seam
- * (src/meteo/mo_meteo_handler.f90:1462-1605). */
+ * (src/meteo/mo_meteo_handler.f90:1462-1605).  Any value is taken; a cell given
+ * precipitation below 0 (nodata) or not finite goes the reference's branches one
+ * by one from then on, which is slower, until the variable is given anew for all
+ * n_forcing_days columns. */
 int mhmhip_set_forcing(mhmhip_ctx *ctx, int32_t var, int32_t day0, int32_t ndays,
                        const double *host, int64_t ld);
 /* Streamed forcing: days day0..day0+ndays-1 (1-based iMeteoTS, any day of the

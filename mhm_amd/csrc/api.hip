@@ -2751,7 +2751,8 @@ int run_impl(mhmhip_ctx *x, const mhmhip_step *steps, int32_t nsteps,
   // No steps_per_launch given: a launch of 24 steps spends a third of its time
   // before and after them (14 of 39 us with a wave per SIMD), so where the
   // routing takes what the ring holds anyway, a launch runs as many times 24 steps
-  // as fit it, at most 144, whatever the step's length: 215x301 cells, 720 steps 2.47 -> 2.36 ms.
+  // as fit it, at most 144, whatever the step's length: 215x301 cells, 720 steps
+  // 2.47 -> 2.36 ms.
   if (o.mode == MHMHIP_RUN_FUSED && o.steps_per_launch <= 0 && (flow || !route) && !x->coarse)
     S = std::max<int>(24, (int)std::min<int64_t>(144, route ? ring_rows / rep : 144) / 24 * 24);
   // the ring's rows in use: whole cell launches, so that no routing launch's
