@@ -85,7 +85,7 @@ struct mhmhip_ctx {
   // not read it), n_frows rows in all
   int32_t frow[MHMHIP_F_COUNT] = {};
   int32_t n_frows = 0;
-  uint8_t *d_odd = nullptr;  // [sstride] OddWeather marks of the cells
+  uint8_t *d_odd = nullptr;  // [sstride] OddWeather marks of the cells, after F's rows
   int32_t odd_given = 0;     // bits that forcing given so far may have set in them
   double *W = nullptr;  // meteo weights [3][12 * 24][sstride], null: off
   // MPR-lite inputs (mhmhip_mprlite_inputs): host copies in reference cell
@@ -453,16 +453,16 @@ extern "C" int mhmhip_create(const mhmhip_config *cfg, mhmhip_ctx **out) {
   x->n_frows = forcing_rows(c.process_pet);
   x->n_srows = sr_count(x->nh);
   x->n_xrows = xr_count(x->nh);
+  const int64_t n_forcing = (int64_t)x->n_frows * c.n_forcing_days * x->sstride;
   if ((rc = x->dalloc(&x->P, x->n_prows * x->ld, "alloc params")) ||
       (rc = x->dalloc(&x->S, x->n_srows * x->ld, "alloc states")) ||
       (rc = x->dalloc(&x->X, x->n_xrows * x->ld, "alloc fluxes")) ||
-      (rc = x->dalloc(&x->F, (int64_t)x->n_frows * c.n_forcing_days * x->sstride,
-                      "alloc forcing")) ||
-      (rc = x->dalloc(&x->d_odd, x->sstride, "alloc weather marks"))) {
+      (rc = x->dalloc(&x->F, n_forcing + x->sstride / 8, "alloc forcing"))) {
     g_create_error = x->err;
     mhmhip_destroy(x);
     return rc;
   }
+  x->d_odd = reinterpret_cast<uint8_t *>(x->F + n_forcing);
   bool usual = true;  // the day's and night's shares of the precipitation, temperature shifts
   for (int m = 0; m < 12; ++m)
     usual = usual && c.fnight_prec[m] >= 0.0 && c.fnight_prec[m] <= 1.0 &&
@@ -504,7 +504,6 @@ extern "C" int mhmhip_destroy(mhmhip_ctx *x) {
   (void)hipFree(x->S);
   (void)hipFree(x->X);
   (void)hipFree(x->F);
-  (void)hipFree(x->d_odd);
   (void)hipFree(x->W);
   (void)hipFree(x->d_agg_start);
   (void)hipFree(x->d_cring);

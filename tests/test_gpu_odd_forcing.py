@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 from mhm_amd import calendar, engine, parameters as PM, synth
+from oracle_sim import OracleSim
 from pairs import START, compare_cells, make_pair
 
 pytestmark = pytest.mark.gpu
@@ -148,3 +149,26 @@ def test_streamed_marks_change_between_launches():
     for other in got[1:]:
         for k in got[0]:
             assert np.array_equal(got[0][k], other[k]), k
+
+
+def test_a_night_share_above_one_matches_oracle():
+    """The day's share is then negative: every cell takes the branches."""
+    print("case: odd day and night shares", flush=True)
+    share = [1.6] * 12
+    dom = _domain(4)
+    dom.forcing["PRE"] = 30.0 * np.abs(dom.forcing["PRE"]) % 60.0
+    steps, recs = calendar.step_table(START, 96, 1), calendar.step_records(START, 96, 1)
+    params = synth.cell_params(dom, PM.DEFAULT)
+    for mode in (1, 0):
+        model = engine.Model([dom], route=False, n_forcing_days=4, fnight_prec=share)
+        sim = OracleSim([dom], n_forcing_days=4, route=False, fnight_prec=share)
+        for m in (model, sim):
+            m.set_params(params, 0)
+            m.default_states()
+            m.set_domain_forcing()
+        model.run(steps, mode=mode, steps_per_launch=12, want_gauges=False)
+        for r in recs:
+            sim.step(r)
+        bad = compare_cells(model, sim, RTOL, ATOL)
+        assert bad == [], bad
+        model.close()
